@@ -66,7 +66,7 @@ __device__ __forceinline__ void coords(const Geo& g, long c, int& i, int& j, int
     else { j = (int)rest; k = 0; }
 }
 
-__global__ void k_ctrl_init(Ctrl* ctrl, const double* count, int max_iter, double tol, int tol_mode, int project,
+static __global__ void k_ctrl_init(Ctrl* ctrl, const double* count, int max_iter, double tol, int tol_mode, int project,
                             int flexible, double* hist) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         Ctrl c = {};
@@ -98,7 +98,7 @@ __device__ __forceinline__ void d_init_sum(const double* __restrict__ rhs, const
     }
     block_store<1>(v, partials);
 }
-__global__ void k_init_sum(const double* __restrict__ rhs, const uint8_t* __restrict__ nbr, long N4,
+static __global__ void k_init_sum(const double* __restrict__ rhs, const uint8_t* __restrict__ nbr, long N4,
                            double* partials, Ctrl* ctrl) {
     d_init_sum(rhs, nbr, N4, partials, ctrl, blockIdx.x, gridDim.x);
 }
@@ -107,7 +107,7 @@ __device__ __forceinline__ void d_fin_init_sum(const double* partials, int nbt, 
     reduce_partials_at<1>(partials, nbt, base, nb, tot);
     if (threadIdx.x == 0) ctrl->m1 = (ctrl->project && ctrl->count > 0) ? tot[0] / ctrl->count : 0.0;
 }
-__global__ void k_fin_init_sum(const double* partials, int nb, Ctrl* ctrl) {
+static __global__ void k_fin_init_sum(const double* partials, int nb, Ctrl* ctrl) {
     d_fin_init_sum(partials, nb, 0, nb, ctrl);
 }
 
@@ -143,7 +143,7 @@ __device__ __forceinline__ void d_fin_init_r(const double* partials, int nbt, in
     reduce_partials_at<1>(partials, nbt, base, nb, tot);
     if (threadIdx.x == 0) ctrl->m2 = (ctrl->project && ctrl->count > 0) ? tot[0] / ctrl->count : 0.0;
 }
-__global__ void k_fin_init_r(const double* partials, int nb, Ctrl* ctrl) {
+static __global__ void k_fin_init_r(const double* partials, int nb, Ctrl* ctrl) {
     d_fin_init_r(partials, nb, 0, nb, ctrl);
 }
 
@@ -182,7 +182,7 @@ __device__ __forceinline__ void d_fin_init_sub(const double* partials, int nbt, 
         ctrl->tolsq = (tot[0] > 0) ? tot[0] * ctrl->tol * ctrl->tol : ctrl->tol * ctrl->tol;
     }
 }
-__global__ void k_fin_init_sub(const double* partials, int nb, Ctrl* ctrl) {
+static __global__ void k_fin_init_sub(const double* partials, int nb, Ctrl* ctrl) {
     d_fin_init_sub(partials, nb, 0, nb, ctrl);
 }
 
@@ -310,7 +310,7 @@ __device__ __forceinline__ void d_fin_matvec(const double* partials, int nbt, in
         ctrl->xalpha = ctrl->alpha;
     }
 }
-__global__ void k_fin_matvec(const double* partials, int nb, Ctrl* ctrl) {
+static __global__ void k_fin_matvec(const double* partials, int nb, Ctrl* ctrl) {
     d_fin_matvec(partials, nb, 0, nb, ctrl);
 }
 
@@ -354,7 +354,7 @@ __device__ __forceinline__ void d_fin_init_warm(const double* partials, int nbt,
         if (ctrl->tol_mode == 1 && tot[0] < ctrl->tolsq) { ctrl->done = 1; ctrl->status = ST_CONVERGED; }
     }
 }
-__global__ void k_fin_init_warm(const double* partials, int nb, Ctrl* ctrl) {
+static __global__ void k_fin_init_warm(const double* partials, int nb, Ctrl* ctrl) {
     d_fin_init_warm(partials, nb, 0, nb, ctrl);
 }
 
@@ -470,7 +470,7 @@ __device__ __forceinline__ void d_fin_zsums(const double* partials, int nbt, int
     reduce_partials_at<3>(partials, nbt, base, nb, tot);
     if (threadIdx.x == 0) finish_zsums(ctrl, tot[0], tot[1], tot[2]);
 }
-__global__ void k_fin_zsums(const double* partials, int nb, Ctrl* ctrl) {
+static __global__ void k_fin_zsums(const double* partials, int nb, Ctrl* ctrl) {
     d_fin_zsums(partials, nb, 0, nb, ctrl);
 }
 

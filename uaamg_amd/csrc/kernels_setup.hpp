@@ -64,7 +64,7 @@ __global__ void k_nbr0(const uint8_t* __restrict__ solid, uint8_t* __restrict__ 
 }
 
 // fluid-cell count from the k_nbr0 partials (one workgroup)
-__global__ void k_fin_count(const double* partials, int nb, double* count_out) {
+static __global__ void k_fin_count(const double* partials, int nb, double* count_out) {
     double tot[1];
     reduce_partials<1>(partials, nb, tot);
     if (threadIdx.x == 0) *count_out = tot[0];

@@ -13,149 +13,10 @@
 #include <string>
 #include "../../include/uaamg.h"
 #include "kernels_proj.hpp"
-#include "batch.hpp"
-#include "engine.hpp"
+#include "engines.hpp"
 #include "amgpcg.hpp"
 
 using namespace uaamg;
-
-namespace uaamg {
-
-template <typename A, typename B>
-__global__ void k_cast_all(const A* __restrict__ src, B* __restrict__ dst, long n) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x, s = (long)gridDim.x * blockDim.x;
-    for (; t < n; t += s) dst[t] = (B)src[t];
-}
-
-template <int D, typename T, typename S, typename R>
-void Engine<D, T, S, R>::cast_in_all(const double* src, T* dst) {
-    long n = g0_.N;
-    k_cast_all<double, T><<<(unsigned)std::min<long>((n + 255) / 256, 4096), 256, 0, stream_>>>(src, dst, n);
-    HIPCHK(hipGetLastError());
-}
-template <int D, typename T, typename S, typename R>
-void Engine<D, T, S, R>::cast_out_all(const T* src, double* dst) {
-    long n = g0_.N;
-    k_cast_all<T, double><<<(unsigned)std::min<long>((n + 255) / 256, 4096), 256, 0, stream_>>>(src, dst, n);
-    HIPCHK(hipGetLastError());
-}
-
-template <int D, typename T, typename S, typename R>
-void Engine<D, T, S, R>::allocate() {
-    const int nl = nlevels();
-    lv_.resize(nl);
-    lv_[0].g = g0_;
-    lv_[0].lc = lc0_;
-    solid0_ = dalloc<uint8_t>(g0_.N);
-    // kRowSlack: the row kernels load CPL consecutive cells per lane from a
-    // clamped row start, up to CPL - 1 cells past the last ghost cell
-    nbr0_ = dalloc<uint8_t>(N4_ + kRowSlack);
-    count_ = dalloc<double>(1);
-    ctrl_ = dalloc<Ctrl>(1);
-    HIPCHK(hipHostMalloc((void**)&ctrl_host_, sizeof(Ctrl), hipHostMallocDefault));
-    r_ = dalloc_margin<T>(N4_); z_ = dalloc_margin<T>(N4_); p_ = dalloc_margin<T>(N4_); Ap_ = dalloc_margin<T>(N4_);
-    if (!x_is_p()) x_ = dalloc_margin<T>(N4_);
-    if (pmv_on_) { p2_ = dalloc_margin<T>(N4_); r2_ = dalloc_margin<T>(N4_); partials_m_ = dalloc<double>(pmv_blocks_ + 64); }
-    long maxb = std::max<long>(lc0_.nblocks(), 2048);
-    for (int l = 1; l < nl; l++) {
-        Level& L = lv_[l];
-        L.g = shape_[l];
-        L.lc = cells_launch(L.g, D);
-        L.b = dalloc<S>(L.g.N + kRowSlack); L.x = dalloc<S>(L.g.N + kRowSlack);
-        L.mask = dalloc<uint8_t>(L.g.N);
-        L.coef = dalloc<C4>(L.g.N + kRowSlack);
-        L.ex = dalloc<S>(L.g.N);
-        maxb = std::max(maxb, L.lc.nblocks());
-    }
-    maxb = std::max(maxb, fused_max_blocks());
-    maxb = std::max(maxb, (long)rows_blocks_);
-    partials_ = dalloc<double>(3 * maxb + 64);
-    fused_ok_ = fused_supported();
-    HIPCHK(hipStreamSynchronize(stream_));
-}
-
-template <int D, typename T, typename S, typename R>
-void Engine<D, T, S, R>::release() {
-    (void)hipStreamSynchronize(stream_);
-    for (void* p : allocs_) (void)hipFree(p);
-    allocs_.clear();
-    if (ctrl_host_) (void)hipHostFree(ctrl_host_);
-    ctrl_host_ = nullptr;
-    if (hist_) (void)hipFree(hist_);
-    hist_ = nullptr;
-}
-
-template <int D, typename T, typename S, typename R>
-void Engine<D, T, S, R>::level_data(int level, uint8_t* solid, double* diag, double* cx, double* cy, double* cz, double* ex) {
-    const Geo g = shape_[level];
-    const long N = g.N;
-    std::vector<uint8_t> m(N);
-    std::vector<double> vx(N, 0.0), vy(N, 0.0), vz(N, 0.0), ve(N, 0.0), vd(N, 0.0);
-    auto IX = [&](int i, int j, int k) { return (long)i + (long)j * g.sx + (long)k * g.sy; };
-    const int klo = (D == 3) ? 1 : 0, khi = (D == 3) ? g.nz : 0;
-    if (level == 0) {
-        std::vector<uint8_t> nb(N);
-        HIPCHK(hipMemcpyAsync(m.data(), solid0_, N, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipMemcpyAsync(nb.data(), nbr0_, N, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-        const Consts<double>& c = c0d_;
-        for (int i = 1; i <= g.nx; i++)
-            for (int j = 1; j <= g.ny; j++)
-                for (int k = klo; k <= khi; k++) {
-                    long id = IX(i, j, k);
-                    if (!(nb[id] & NB_FLUID)) continue;
-                    vx[id] = (nb[id] & NB_XP) ? c.idx2 : 0.0;
-                    vy[id] = (nb[id] & NB_YP) ? c.idy2 : 0.0;
-                    if (D == 3) vz[id] = (nb[id] & NB_ZP) ? c.idz2 : 0.0;
-                    double e = 0.0;
-                    if (c.wall[0] && i == 1) e += c.ex2[0];
-                    if (c.wall[1] && i == g.nx) e += c.ex2[1];
-                    if (c.wall[2] && j == 1) e += c.ex2[2];
-                    if (c.wall[3] && j == g.ny) e += c.ex2[3];
-                    if (D == 3) {
-                        if (c.wall[4] && k == 1) e += c.ex2[4];
-                        if (c.wall[5] && k == g.nz) e += c.ex2[5];
-                    }
-                    ve[id] = e;
-                }
-        for (int i = 1; i <= g.nx; i++)
-            for (int j = 1; j <= g.ny; j++)
-                for (int k = klo; k <= khi; k++) {
-                    long id = IX(i, j, k);
-                    if (!(nb[id] & NB_FLUID)) continue;
-                    double d = (D == 3) ? vx[id] + vx[id - 1] + vy[id] + vy[id - g.sx] + vz[id] + vz[id - g.sy]
-                                        : vx[id] + vx[id - 1] + vy[id] + vy[id - g.sx];
-                    if (ve[id] != 0.0) d += ve[id];
-                    vd[id] = d;
-                }
-    } else {
-        const Level& L = lv_[level];
-        std::vector<C4> cf(N);
-        std::vector<S> exv(N);
-        HIPCHK(hipMemcpyAsync(m.data(), L.mask, N, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipMemcpyAsync(cf.data(), L.coef, N * sizeof(C4), hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipMemcpyAsync(exv.data(), L.ex, N * sizeof(S), hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-        for (int i = 1; i <= g.nx; i++)
-            for (int j = 1; j <= g.ny; j++)
-                for (int k = klo; k <= khi; k++) {
-                    long id = IX(i, j, k);
-                    vx[id] = (double)cf[id].x; vy[id] = (double)cf[id].y;
-                    if (D == 3) vz[id] = (double)cf[id].z;
-                    ve[id] = (double)exv[id];
-                    // the record's diagonal as stored (solid cells carry -1, reported as 0)
-                    vd[id] = m[id] ? 0.0 : (double)cf[id].w;
-                }
-    }
-    if (solid) std::memcpy(solid, m.data(), N);
-    if (diag) std::memcpy(diag, vd.data(), N * sizeof(double));
-    if (cx) std::memcpy(cx, vx.data(), N * sizeof(double));
-    if (cy) std::memcpy(cy, vy.data(), N * sizeof(double));
-    if (cz && D == 3) std::memcpy(cz, vz.data(), N * sizeof(double));
-    if (ex) std::memcpy(ex, ve.data(), N * sizeof(double));
-}
-
-}  // namespace uaamg
 
 // ------------------------------------------------------------------ C-ABI
 
@@ -313,25 +174,15 @@ static long padded_n(const uaamg_ctx* c) {
 static std::unique_ptr<EngineBase> make_engine(const uaamg_opts& o, const uaamg_grid& g, hipStream_t s) {
     int n[3] = {g.n[0], g.n[1], g.dim == 3 ? g.n[2] : 1};
     double h[3] = {g.h[0], g.h[1], g.dim == 3 ? g.h[2] : 1.0};
-    if (g.dim == 2) {
-        switch (o.precision) {
-            case UAAMG_FP64: return std::make_unique<Engine<2, double, double>>(o, n, h, g.wall, s);
-            case UAAMG_FP32: return std::make_unique<Engine<2, float, float>>(o, n, h, g.wall, s);
-            // 2D hierarchies keep FP32 levels under MIXED_BF16: with 8-bit mantissas in
-            // the level state, 2D solves with solids take 2-3x the iterations or
-            // stagnate (measured on the batched mixed-size stream); 3D loses ~10 %
-            case UAAMG_MIXED_BF16: return std::make_unique<Engine<2, float, float>>(o, n, h, g.wall, s);
-            case UAAMG_MIXED_BF16R: return std::make_unique<Engine<2, float, float>>(o, n, h, g.wall, s);
-            case UAAMG_MIXED_F64: return std::make_unique<Engine<2, double, float>>(o, n, h, g.wall, s);
-            default: throw HipError{hipErrorInvalidValue, "precision not built"};   // opts_valid rejects it first
-        }
-    }
     switch (o.precision) {
-        case UAAMG_FP64: return std::make_unique<Engine<3, double, double>>(o, n, h, g.wall, s);
-        case UAAMG_FP32: return std::make_unique<Engine<3, float, float>>(o, n, h, g.wall, s);
-        case UAAMG_MIXED_BF16: return std::make_unique<Engine<3, float, __bf16>>(o, n, h, g.wall, s);
-        case UAAMG_MIXED_BF16R: return std::make_unique<Engine<3, float, float, __bf16>>(o, n, h, g.wall, s);
-        case UAAMG_MIXED_F64: return std::make_unique<Engine<3, double, float>>(o, n, h, g.wall, s);
+        case UAAMG_FP64: return make_engine_f64(g.dim, o, n, h, g.wall, s);
+        case UAAMG_FP32: return make_engine_f32(g.dim, o, n, h, g.wall, s);
+        // 2D hierarchies keep FP32 levels under MIXED_BF16: with 8-bit mantissas in
+        // the level state, 2D solves with solids take 2-3x the iterations or
+        // stagnate (measured on the batched mixed-size stream); 3D loses ~10 %
+        case UAAMG_MIXED_BF16: return g.dim == 2 ? make_engine_f32(2, o, n, h, g.wall, s) : make_engine_bf16(false, o, n, h, g.wall, s);
+        case UAAMG_MIXED_BF16R: return g.dim == 2 ? make_engine_f32(2, o, n, h, g.wall, s) : make_engine_bf16(true, o, n, h, g.wall, s);
+        case UAAMG_MIXED_F64: return make_engine_mixed_f64(g.dim, o, n, h, g.wall, s);
         default: throw HipError{hipErrorInvalidValue, "precision not built"};   // opts_valid rejects it first
     }
 }
@@ -751,9 +602,8 @@ static int bfail(uaamg_batch* b, int code, const std::string& msg) {
     catch (const std::bad_alloc&) { return bfail(b, UAAMG_ERR_OOM, "host allocation failed"); }
 
 static std::unique_ptr<uaamg::BatchBase> make_batch_part(int dim, const uaamg_opts& o, hipStream_t s) {
-    if (dim == 2) return std::make_unique<uaamg::BatchEngine<2, float>>(o, s);   // FP32 levels in 2D (see make_engine)
-    if (o.precision == UAAMG_FP32) return std::make_unique<uaamg::BatchEngine<3, float>>(o, s);
-    return std::make_unique<uaamg::BatchEngine<3, __bf16>>(o, s);
+    if (dim == 2 || o.precision == UAAMG_FP32) return uaamg::make_batch_f32(dim, o, s);   // FP32 levels in 2D (see make_engine)
+    return uaamg::make_batch_bf16(o, s);
 }
 
 extern "C" int uaamg_batch_create(uaamg_batch** out, const uaamg_opts* o) {
