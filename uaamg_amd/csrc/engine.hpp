@@ -471,7 +471,7 @@ public:
     double alg_bytes_of(int iters) const { return alg_bytes(iters); }
     long padded_cells() const { return g0_.N; }
     long n4() const { return N4_; }
-    int rows_cpl() const { return rows_cpl_; }
+    int rows_cpl() const { return rows_win_ ? 0 : rows_cpl_; }   // of the batched row kernels (whole rows only)
     int tail_first() const { return tail_first_; }
     // fill the batch descriptor (ctrl: the batch's scalar slot for this grid)
     void fill_batch(BGrid<S>& d, Ctrl* ctrl) const {
@@ -490,7 +490,7 @@ public:
                 d.lb[l] = lv_[l].b; d.lx[l] = lv_[l].x; d.lcoef[l] = lv_[l].coef;
                 d.lKC[l] = 8;
             }
-            d.cpl = rows_cpl_;
+            d.cpl = rows_cpl();
             d.rtab = rtab_;
             d.rgeo = rgeo_;
             d.tail = targs_;
@@ -565,28 +565,47 @@ public:
         k_tail<D, S, C4, TAIL_NLMAX><<<1, TAIL_THREADS, 0, stream_>>>(targs_);
     }
 
-    // ---- level-0 row kernels (3D, FP32 vectors, nx <= 256) ----
-    static constexpr int ROWS_NW = 10, ROWS_RW = 2;
+    // ---- level-0 row kernels (3D) ----
+    // A wave takes whole x-rows while 64 lanes of CPL cells cover them (FP32:
+    // nx <= 128 with 2 cells a lane, <= 256 with 4; FP64: 2 cells, nx <= 128,
+    // which is the same bytes and registers per lane as FP32 with 4), wider
+    // rows in windows.  Against the march kernels and flat CG passes that ran
+    // here before: 128 x 64 x 64 FP64 projection 3.02 -> 2.22 ms, 256 x 128 x
+    // 128 FP64 solve (3 windows) 4.98 -> 4.02, 512 x 256 x 256 FP32 solve (3
+    // windows) 57.7 -> 37.5; down / up kernel at 256 x 128 x 128 FP64 66 -> 49
+    // / 75 -> 39 us.
+    static constexpr int ROWS_NW = 10, ROWS_RW = 2, ROWS_CPL = sizeof(T) == 8 ? 2 : 4;   // ROWS_CPL: of wide rows
     int rows_cpl_ = 0;          // cells per lane (0: row kernels not used)
-    RowTab rtab_{};
+    bool rows_win_ = false;     // rows are cut into windows
+    RowTabOf<T> rtab_{};
     RowGeo rgeo_{};
     unsigned rows_blocks_ = 0;
+    // cells per lane and windows of rows of nx cells (0: no row kernels)
+    static int row_lanes(int nx, int& nwx, int& wl) {
+        const int cpl = sizeof(T) == 8 || nx <= 128 ? 2 : 4;
+        const int lanes = (nx + cpl - 1) / cpl;
+        nwx = lanes <= 64 ? 1 : (lanes <= 126 ? 2 : (lanes + 61) / 62);
+        wl = nwx == 1 ? 64 : (lanes + nwx - 1) / nwx;
+        return cpl;
+    }
+    // the row kernels address a level by 32-bit element offsets
+    static bool rows_addressable(const Geo& g) { return g.N < (1L << 31) - 1024; }
     void rows_setup(const double h[3], const int wall[6]) {
         rows_cpl_ = 0;
-        if constexpr (D == 3 && std::is_same<T, float>::value) {
+        if constexpr (D == 3) {
             if (!(o_.forms & UAAMG_FORM_ROWS)) return;
-            if (nlevels() < 2) return;
-            const int nx = n_[0];
-            rows_cpl_ = nx <= 128 ? 2 : (nx <= 256 ? 4 : 0);
-            if (!rows_cpl_) return;
+            if (nlevels() < 2 || !rows_addressable(g0_)) return;
+            int nwx, wl;
+            rows_cpl_ = row_lanes(n_[0], nwx, wl);
+            rows_win_ = nwx > 1;
             const double ix = 1.0 / (h[0] * h[0]), iy = 1.0 / (h[1] * h[1]), iz = 1.0 / (h[2] * h[2]);
             for (int m = 0; m < 64; m++) {
                 double d = ix * (((m >> 0) & 1) + ((m >> 1) & 1)) + iy * (((m >> 2) & 1) + ((m >> 3) & 1))
                          + iz * (((m >> 4) & 1) + ((m >> 5) & 1));
-                rtab_.d[m] = (float)d;
-                rtab_.rinv[m] = d >= 1e-30 ? (float)(1.0 / d) : 0.0f;
+                rtab_.d[m] = (T)d;
+                rtab_.rinv[m] = d >= 1e-30 ? (T)(1.0 / d) : T(0);
             }
-            rtab_.idx2 = (float)ix; rtab_.idy2 = (float)iy; rtab_.idz2 = (float)iz;
+            rtab_.idx2 = (T)ix; rtab_.idy2 = (T)iy; rtab_.idz2 = (T)iz;
             for (int m = 0; m < 64; m++)
                 ptab_.d[m] = ix * (((m >> 0) & 1) + ((m >> 1) & 1)) + iy * (((m >> 2) & 1) + ((m >> 3) & 1))
                            + iz * (((m >> 4) & 1) + ((m >> 5) & 1));
@@ -595,15 +614,15 @@ public:
             rtab_.any_dirichlet = 0;
             for (int f = 0; f < 6; f++) {
                 const bool on = wall[f] == UAAMG_WALL_DIRICHLET;
-                rtab_.ex[f] = on ? (float)e[f] : 0.0f;
+                rtab_.ex[f] = on ? (T)e[f] : T(0);
                 ptab_.ex[f] = on ? e[f] : 0.0;
                 rtab_.any_dirichlet |= on;
             }
             ptab_.any_dirichlet = rtab_.any_dirichlet;
-            rgeo_ = make_rowgeo(n_[1], n_[2], ROWS_NW * ROWS_RW - 4, o_.rows_kc);
+            rgeo_ = make_rowgeo(n_[1], n_[2], ROWS_NW * ROWS_RW - 4, o_.rows_kc, nwx, wl);
             rows_blocks_ = 8u * (unsigned)rgeo_.per_xcd;
             pmv_on_ = (o_.forms & UAAMG_FORM_PMV) != 0;
-            pgeo_ = make_rowgeo(n_[1], n_[2], PMV_NW * PMV_RW - 2, o_.rows_kc);
+            pgeo_ = make_rowgeo(n_[1], n_[2], PMV_NW * PMV_RW - 2, o_.rows_kc, nwx, wl);
             pmv_blocks_ = 8u * (unsigned)pgeo_.per_xcd;
         }
     }
@@ -611,14 +630,16 @@ public:
     // so that about 256 tiles (one per CU) cover the level (KC <= 16; more
     // planes per tile amortise the 4 halo plane steps, more tiles fill the chip)
     // unless kc_force > 0 sets it
-    static RowGeo make_rowgeo(int ny, int nz, int TY = ROWS_NW * ROWS_RW - 4, int kc_force = 0) {
+    static RowGeo make_rowgeo(int ny, int nz, int TY = ROWS_NW * ROWS_RW - 4, int kc_force = 0, int nwx = 1, int wl = 64) {
         RowGeo rg{};
+        rg.nwx = nwx;
+        rg.wl = wl;
         rg.nty = (ny + TY - 1) / TY;
-        int KC = (int)std::min<long>(16, std::max<long>(4, (long)nz * rg.nty / 256 / 4 * 4));
+        int KC = (int)std::min<long>(16, std::max<long>(4, (long)nz * rg.nty * nwx / 256 / 4 * 4));
         if (kc_force > 0) KC = std::max(4, kc_force / 4 * 4);
         rg.KC = KC;
         rg.nkc = (nz + KC - 1) / KC;
-        rg.ntiles = rg.nty * rg.nkc;
+        rg.ntiles = nwx * rg.nty * rg.nkc;
         rg.per_xcd = (rg.ntiles + 7) / 8;
         return rg;
     }
@@ -672,40 +693,53 @@ public:
     }
     // every lane's cells lie inside the row (nx == 64 cells-per-lane): the
     // row kernels' instantiations without lane masks
-    bool rows_full() const { return rows_cpl_ > 0 && g0_.nx == 64 * rows_cpl_; }
+    bool rows_full() const { return rows_cpl_ > 0 && !rows_win_ && g0_.nx == 64 * rows_cpl_; }
+    // nontemporal loads of a level-0 kernel's last-use inputs where the form
+    // is allowed: rows of more than 128 cells
+    bool rows_nt(int form) const { return (o_.forms & form) && (rows_cpl_ == 4 || rows_win_); }
     void rows_down0(const T* r, Level& C, const int* skip) {
-        if constexpr (D == 3 && std::is_same<T, float>::value) {
+        if constexpr (D == 3) {
             if (fr_old_) {   // alpha from the operator's partials; r = r_old - alpha Ap written to r; r.r -> convergence
                 // nontemporal loads of r_old and Ap (last use of both; without
                 // UAAMG_FORM_NT_D plain): 34.5 vs 33.5 solves/s at 256^3 in three paired runs
-                const bool dnt = (o_.forms & UAAMG_FORM_NT_D) && rows_cpl_ == 4;
+                const bool dnt = rows_nt(UAAMG_FORM_NT_D);
                 forms_used_ |= dnt ? UAAMG_FORM_NT_D : 0;
-                tlaunch(timer_, UAAMG_K_DOWN0, rows_cpl_ == 4 ? (dnt ? (rows_full() ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, true>
-                                                                                    : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true>)
-                                                                     : k_rows_down0r<4, ROWS_NW, ROWS_RW, S>)
-                                                              : k_rows_down0r<2, ROWS_NW, ROWS_RW, S>,
-                        dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, (const float*)fr_old_, (const uint8_t*)nbr0_, g0_, rtab_,
-                        rgeo_, C.b, C.g, skip, (const float*)Ap_, (float*)r, partials_, (const double*)partials_m_,
-                        (int)pmv_blocks_, ctrl_, xslot_);
+                auto kern = rows_win_ ? (dnt ? k_rows_down0r<ROWS_CPL, ROWS_NW, ROWS_RW, S, true, false, true, T>
+                                             : k_rows_down0r<ROWS_CPL, ROWS_NW, ROWS_RW, S, false, false, true, T>)
+                                      : k_rows_down0r<2, ROWS_NW, ROWS_RW, S, false, false, false, T>;
+                if constexpr (ROWS_CPL == 4)
+                    if (!rows_win_ && rows_cpl_ == 4)
+                        kern = dnt ? (rows_full() ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true>)
+                                   : k_rows_down0r<4, ROWS_NW, ROWS_RW, S>;
+                tlaunch(timer_, UAAMG_K_DOWN0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, (const T*)fr_old_,
+                        (const uint8_t*)nbr0_, g0_, rtab_, rgeo_, C.b, C.g, skip, (const T*)Ap_, (T*)r, partials_,
+                        (const double*)partials_m_, (int)pmv_blocks_, ctrl_, xslot_);
                 fin_fold_ = fin_foldable();
                 if (!fin_fold_) k_fin_update<false><<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)rows_blocks_, ctrl_);
                 return;
             }
-            tlaunch(timer_, UAAMG_K_DOWN0, rows_cpl_ == 4 ? k_rows_down0<4, ROWS_NW, ROWS_RW, S> : k_rows_down0<2, ROWS_NW, ROWS_RW, S>,
-                    dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, nbr0_, g0_, rtab_, rgeo_, C.b, C.g, skip);
+            auto kern = rows_win_ ? k_rows_down0<ROWS_CPL, ROWS_NW, ROWS_RW, S, true, T> : k_rows_down0<2, ROWS_NW, ROWS_RW, S, false, T>;
+            if constexpr (ROWS_CPL == 4)
+                if (!rows_win_ && rows_cpl_ == 4) kern = k_rows_down0<4, ROWS_NW, ROWS_RW, S>;
+            tlaunch(timer_, UAAMG_K_DOWN0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, (const uint8_t*)nbr0_, g0_, rtab_,
+                    rgeo_, C.b, C.g, skip);
         }
     }
     void rows_up0(const T* r, Level& C, T* z, const int* skip) {
-        if constexpr (D == 3 && std::is_same<T, float>::value) {
+        if constexpr (D == 3) {
             // nontemporal loads of r (without UAAMG_FORM_NT_U plain): 34.6 vs
             // 33.9 solves/s at 256^3 in three paired runs
-            const bool unt = (o_.forms & UAAMG_FORM_NT_U) && rows_cpl_ == 4;
+            const bool unt = rows_nt(UAAMG_FORM_NT_U);
             forms_used_ |= unt ? UAAMG_FORM_NT_U : 0;
-            tlaunch(timer_, UAAMG_K_UP0, rows_cpl_ == 4 ? (unt ? (rows_full() ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, true>
-                                                                              : k_rows_up0<4, ROWS_NW, ROWS_RW, S, true>)
-                                                               : k_rows_up0<4, ROWS_NW, ROWS_RW, S>)
-                                                        : k_rows_up0<2, ROWS_NW, ROWS_RW, S>,
-                    dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, nbr0_, g0_, rtab_, rgeo_, C.x, C.g, z, skip, partials_);
+            auto kern = rows_win_ ? (unt ? k_rows_up0<ROWS_CPL, ROWS_NW, ROWS_RW, S, true, false, true, T>
+                                         : k_rows_up0<ROWS_CPL, ROWS_NW, ROWS_RW, S, false, false, true, T>)
+                                  : k_rows_up0<2, ROWS_NW, ROWS_RW, S, false, false, false, T>;
+            if constexpr (ROWS_CPL == 4)
+                if (!rows_win_ && rows_cpl_ == 4)
+                    kern = unt ? (rows_full() ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_up0<4, ROWS_NW, ROWS_RW, S, true>)
+                               : k_rows_up0<4, ROWS_NW, ROWS_RW, S>;
+            tlaunch(timer_, UAAMG_K_UP0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, (const uint8_t*)nbr0_, g0_, rtab_, rgeo_,
+                    (const S*)C.x, C.g, z, skip, partials_);
             // with the split update the next operator pass does this finish
             if (!fr_) k_fin_zsums<<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)rows_blocks_, ctrl_);
         }
@@ -1023,18 +1057,23 @@ public:
             // p.Ap partials in their own buffer: the down kernel that sums
             // them writes its r.r partials while other workgroups still read
             // (with the split update it also finishes the level-0 up kernel's z sums)
-            if constexpr (D == 3 && std::is_same<T, float>::value) {
+            if constexpr (D == 3) {
                 // nontemporal loads of z and p_old (last use of both; without
                 // UAAMG_FORM_NT_P plain): 33.6 vs 33.0 solves/s at 256^3 in three paired runs
-                const bool pnt = (o_.forms & UAAMG_FORM_NT_P) && fr_ && rows_cpl_ == 4;
+                const bool pnt = rows_nt(UAAMG_FORM_NT_P) && fr_;
                 forms_used_ |= pnt ? UAAMG_FORM_NT_P : 0;
-                auto kern = fr_ ? (rows_cpl_ == 4 ? (pnt ? (rows_full() ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, true>
-                                                                        : k_rows_pmv<4, PMV_NW, PMV_RW, true, true>)
-                                                         : k_rows_pmv<4, PMV_NW, PMV_RW, true>)
-                                                  : k_rows_pmv<2, PMV_NW, PMV_RW, true>)
-                                : (rows_cpl_ == 4 ? k_rows_pmv<4, PMV_NW, PMV_RW, false> : k_rows_pmv<2, PMV_NW, PMV_RW, false>);
-                tlaunch(timer_, UAAMG_K_MATVEC, kern, dim3(pmv_blocks_), dim3(PMV_NW * 64), stream_, (const float*)z_,
-                        (const float*)pold, (float*)pnew, (float*)Ap_, (const uint8_t*)nbr0_, g0_, ptab_, pgeo_,
+                auto kern = rows_win_ ? (fr_ ? (pnt ? k_rows_pmv<ROWS_CPL, PMV_NW, PMV_RW, true, true, false, true, T>
+                                                    : k_rows_pmv<ROWS_CPL, PMV_NW, PMV_RW, true, false, false, true, T>)
+                                             : k_rows_pmv<ROWS_CPL, PMV_NW, PMV_RW, false, false, false, true, T>)
+                                      : (fr_ ? k_rows_pmv<2, PMV_NW, PMV_RW, true, false, false, false, T>
+                                             : k_rows_pmv<2, PMV_NW, PMV_RW, false, false, false, false, T>);
+                if constexpr (ROWS_CPL == 4)
+                    if (!rows_win_ && rows_cpl_ == 4)
+                        kern = fr_ ? (pnt ? (rows_full() ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, true> : k_rows_pmv<4, PMV_NW, PMV_RW, true, true>)
+                                          : k_rows_pmv<4, PMV_NW, PMV_RW, true>)
+                                   : k_rows_pmv<4, PMV_NW, PMV_RW, false>;
+                tlaunch(timer_, UAAMG_K_MATVEC, kern, dim3(pmv_blocks_), dim3(PMV_NW * 64), stream_, (const T*)z_,
+                        (const T*)pold, (T*)pnew, (T*)Ap_, (const uint8_t*)nbr0_, g0_, ptab_, pgeo_,
                         partials_m_, ctrl_, (const double*)partials_, (int)rows_blocks_);
             }
             pv = pnew;

@@ -1,16 +1,16 @@
-// kernels_pmv.hpp -- level-0 search direction and operator in one pass
-// (FP32 vectors, 3D).
+// kernels_pmv.hpp -- level-0 search direction and operator in one pass (3D;
+// vectors of type F: float, or double).
 //
 // One pass replaces the p update of iteration k-1 and the operator of
 // iteration k (pcg_3d.cpp:116-122 and 94-96):
 //   p_new = (z - mean_z) + beta p_old      on fluid cells (0 elsewhere)
-//   Ap    = d p_new - sum_nb c p_new_nb     (FP64 arithmetic on the FP32
+//   Ap    = d p_new - sum_nb c p_new_nb     (FP64 arithmetic on the
 //                                            values, rounded once; d from the
 //                                            neighbour byte + Dirichlet excess)
 //   partial sums of p_new . Ap             (deterministic, per workgroup)
 // p_old and p_new are separate buffers: a workgroup recomputes p_new on its
 // halo row and planes from z and p_old, so no workgroup reads what another
-// one writes.  p_new is k_pupdate's formula (in FP32); the operator is k_matvec_dot's
+// one writes.  p_new is k_pupdate's formula (in F); the operator is k_matvec_dot's
 // (apply_A) in the stencil form of the row kernels: p_new is 0 on every
 // non-fluid cell, so a face to a solid cell or a Neumann wall drops out of
 // both d and the sum, and a Dirichlet wall face adds 2/h^2 to d (apply_A's
@@ -40,9 +40,9 @@ struct PmvTab {
     int any_dirichlet;
 };
 
-template <int CPL, int NW>
+template <int CPL, int NW, typename F>
 struct PmvLDS {
-    float ex[2][NW][2][CPL][64];   // [step parity][wave][first / last row][cell][lane]
+    F ex[2][NW][2][CPL][64];   // [step parity][wave][first / last row][cell][lane]
 };
 
 // With FZ the pass also does the finish of the z sums (finish_zsums,
@@ -51,40 +51,40 @@ struct PmvLDS {
 // and beta; workgroup 0 stores them.  rsold and the first-iteration flag are
 // read here and only written by the next kernel (the level-0 down kernel),
 // so no workgroup can see a value of this launch.
-template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false>
-__device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const float* __restrict__ pold,
-                                           float* __restrict__ pnew, float* __restrict__ Ap,
+template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false, bool WIN = false, typename F>
+__device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __restrict__ pold,
+                                           F* __restrict__ pnew, F* __restrict__ Ap,
                                            const uint8_t* __restrict__ nbr, const Geo& g, const PmvTab& K,
                                            const RowGeo& rg, double* partials, Ctrl* ctrl, int tile,
                                            const double* zp = nullptr, int nzp = 0) {
+    using RV = typename RowVec<CPL, F>::V;
     if (ctrl->done) return;
-    __shared__ PmvLDS<CPL, NW> L;
+    __shared__ PmvLDS<CPL, NW, F> L;
     __shared__ double sd[64];
     __shared__ double s_zs[3];
     double acc[1] = {0.0};
     const bool active = tile < rg.ntiles;   // idle workgroups still store a zero partial
-    const int ty = tile % rg.nty, kc = tile / rg.nty;
+    RowThread<CPL, NW, RW, 1, FULL, WIN> th;
+    th.init(g, rg, active ? tile : 0);
     // odd z-chunks march downwards, so the two tiles on either side of a
     // chunk boundary read the planes they share at about the same time (both
     // first or both last), and the second read can hit the L2: at 256^3 the
     // pass fetches 195.9 instead of 199.3 MB (28.44 vs 28.54 ms per solve)
-    const int dir = (kc & 1) ? -1 : 1;
-    RowThread<CPL, NW, RW, 1, FULL> th;
-    th.init(g, rg, active ? ty : 0, active ? kc : 0);
+    const int dir = (th.kc & 1) ? -1 : 1;
     const int lane = th.lane, w = th.w;
 
-    float PN[4][RW][CPL];        // p_new of planes (slot = plane & 3)
+    F PN[4][RW][CPL];        // p_new of planes (slot = plane & 3)
     uint8_t NB[4][RW][CPL];
-    float pfz[2][RW][CPL], pfp[2][RW][CPL];
+    F pfz[2][RW][CPL], pfp[2][RW][CPL];
     uint8_t pfn[2][RW][CPL];
     auto issue = [&](int slot, int P) {
         const int po = th.plane(g, P);
 #pragma unroll
         for (int t = 0; t < RW; t++) {
             row_load<CPL, NT>(z, nbr, th.roff[t] + po, th.okx, pfz[slot][t], pfn[slot][t]);
-            typename RowVec<CPL>::V v;
-            if constexpr (NT) v = __builtin_nontemporal_load((const typename RowVec<CPL>::V*)(pold + th.roff[t] + po));
-            else v = *(const typename RowVec<CPL>::V*)(pold + th.roff[t] + po);
+            RV v;
+            if constexpr (NT) v = __builtin_nontemporal_load((const RV*)(pold + th.roff[t] + po));
+            else v = *(const RV*)(pold + th.roff[t] + po);
 #pragma unroll
             for (int q = 0; q < CPL; q++) pfp[slot][t][q] = v[q];
         }
@@ -109,10 +109,10 @@ __device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const fl
         if (threadIdx.x == 0) { s_zs[0] = zs[0]; s_zs[1] = zs[1]; s_zs[2] = zs[2]; }
     }
     __syncthreads();
-    // the p update runs in FP32 (one FMA) with the FP64 scalars rounded once:
-    // it differs from k_pupdate's FP64 form by the rounding of the scalars,
-    // far below the FP32 storage of the vectors
-    float mean, beta;
+    // FP32 vectors: the p update runs in FP32 (one FMA) with the FP64 scalars
+    // rounded once: it differs from k_pupdate's FP64 form by the rounding of
+    // the scalars, far below the FP32 storage of the vectors
+    F mean, beta;
     if constexpr (FZ) {
         const double sz = s_zs[0], srz = s_zs[1], sr = s_zs[2];
         const double m = (ctrl->project && ctrl->count > 0) ? sz / ctrl->count : 0.0;
@@ -124,9 +124,9 @@ __device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const fl
             if (!isfinite(rz)) { ctrl->done = 1; ctrl->status = ST_NONFINITE; }
         }
         if (!isfinite(rz)) return;   // the whole solve stops; the down kernel sees done
-        mean = (float)m; beta = (float)b;
+        mean = (F)m; beta = (F)b;
     } else {
-        mean = (float)ctrl->mean_z; beta = (float)ctrl->beta;
+        mean = (F)ctrl->mean_z; beta = (F)ctrl->beta;
     }
 
     if (active) {
@@ -135,7 +135,7 @@ __device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const fl
 #pragma unroll
             for (int t = 0; t < RW; t++)
 #pragma unroll
-                for (int q = 0; q < CPL; q++) { PN[s][t][q] = 0.0f; NB[s][t][q] = 0; }
+                for (int q = 0; q < CPL; q++) { PN[s][t][q] = F(0); NB[s][t][q] = 0; }
 
         // step: plane P enters (slot S); the operator on plane P-1
         auto step = [&](auto Sc, int P) {
@@ -150,7 +150,7 @@ __device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const fl
                     const uint8_t nb = pin ? pfn[PB][t][q] : (uint8_t)0;
                     NB[S][t][q] = nb;
                     PN[S][t][q] = (nb & NB_FLUID)
-                        ? fmaf(beta, pfp[PB][t][q], pfz[PB][t][q] - mean) : 0.0f;
+                        ? rfma(beta, pfp[PB][t][q], pfz[PB][t][q] - mean) : F(0);
                 }
             // the last plane to enter is last + 1 (upwards) or m0 - 1 (downwards);
             // beyond it the loads repeat that cached plane (no memory traffic), so
@@ -189,16 +189,16 @@ __device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const fl
                 }
                 sfor<RW>([&](auto tc) {
                     constexpr int t = decltype(tc)::value;
-                    const float el = lane_from_left(PN[S1][t][CPL - 1]);
-                    const float er = lane_from_right(PN[S1][t][0]);
-                    float out[CPL];
-                    float pap = 0.0f;   // the row's p.Ap in FP32, accumulated in FP64
+                    const F el = lane_from_left(PN[S1][t][CPL - 1]);
+                    const F er = lane_from_right(PN[S1][t][0]);
+                    F out[CPL];
+                    F pap = F(0);   // the row's p.Ap in F, accumulated in FP64
                     sfor<CPL>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
-                        const float vc = PN[S1][t][q];
-                        const float vl = (q > 0) ? PN[S1][t][q > 0 ? q - 1 : 0] : el;
-                        const float vr = (q < CPL - 1) ? PN[S1][t][q < CPL - 1 ? q + 1 : 0] : er;
-                        float vb, vt;
+                        const F vc = PN[S1][t][q];
+                        const F vl = (q > 0) ? PN[S1][t][q > 0 ? q - 1 : 0] : el;
+                        const F vr = (q < CPL - 1) ? PN[S1][t][q < CPL - 1 ? q + 1 : 0] : er;
+                        F vb, vt;
                         if constexpr (t > 0) vb = PN[S1][t - 1][q]; else vb = L.ex[RB][w > 0 ? w - 1 : 0][1][q][lane];
                         if constexpr (t < RW - 1) vt = PN[S1][t + 1][q]; else vt = L.ex[RB][w < NW - 1 ? w + 1 : NW - 1][0][q][lane];
                         const uint8_t nb = NB[S1][t][q];
@@ -206,23 +206,23 @@ __device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const fl
                         const double sum = K.idx2 * ((double)vl + (double)vr) + K.idy2 * ((double)vb + (double)vt)
                                          + K.idz2 * ((double)PN[S2][t][q] + (double)PN[S][t][q]);
                         const bool fl = nb & NB_FLUID;
-                        const float o = fl ? (float)(d * (double)vc - sum) : 0.0f;
-                        pap = fmaf(th.okx[q] ? vc : 0.0f, o, pap);
+                        const F o = fl ? (F)(d * (double)vc - sum) : F(0);
+                        pap = rfma(th.okw[q] ? vc : F(0), o, pap);
                         out[q] = o;
                     });
                     if (th.tile_row[t]) acc[0] += (double)pap;
                     if (th.tile_row[t]) {
                         const int id = th.roff[t] + R * (int)g.sy;
-                        if (th.full || th.okx[CPL - 1]) {
-                            typename RowVec<CPL>::V vp, va;
+                        if (th.full || th.okw[CPL - 1]) {
+                            RV vp, va;
 #pragma unroll
                             for (int q = 0; q < CPL; q++) { vp[q] = PN[S1][t][q]; va[q] = out[q]; }
-                            *(typename RowVec<CPL>::V*)(pnew + id) = vp;
-                            *(typename RowVec<CPL>::V*)(Ap + id) = va;
+                            *(RV*)(pnew + id) = vp;
+                            *(RV*)(Ap + id) = va;
                         } else {
 #pragma unroll
                             for (int q = 0; q < CPL; q++)
-                                if (th.okx[q]) { pnew[id + q] = PN[S1][t][q]; Ap[id + q] = out[q]; }
+                                if (th.okw[q]) { pnew[id + q] = PN[S1][t][q]; Ap[id + q] = out[q]; }
                         }
                     }
                 });
@@ -242,13 +242,13 @@ __device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const fl
     block_store<1>(acc, partials);
 }
 
-template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false>
-__global__ __launch_bounds__(NW * 64) void k_rows_pmv(const float* __restrict__ z, const float* __restrict__ pold,
-                                                      float* __restrict__ pnew, float* __restrict__ Ap,
+template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false, bool WIN = false, typename F = float>
+__global__ __launch_bounds__(NW * 64) void k_rows_pmv(const F* __restrict__ z, const F* __restrict__ pold,
+                                                      F* __restrict__ pnew, F* __restrict__ Ap,
                                                       const uint8_t* __restrict__ nbr, Geo g, PmvTab K,
                                                       RowGeo rg, double* partials, Ctrl* ctrl,
                                                       const double* zp, int nzp) {
-    d_rows_pmv<CPL, NW, RW, FZ, NT, FULL>(z, pold, pnew, Ap, nbr, g, K, rg, partials, ctrl, row_tile_of_block(rg, blockIdx.x),
+    d_rows_pmv<CPL, NW, RW, FZ, NT, FULL, WIN, F>(z, pold, pnew, Ap, nbr, g, K, rg, partials, ctrl, row_tile_of_block(rg, blockIdx.x),
                                 zp, nzp);
 }
 

@@ -1,4 +1,5 @@
-// kernels_rows.hpp -- level-0 V(1,1) kernels of the FP32 path (3D).
+// kernels_rows.hpp -- level-0 V(1,1) kernels in 3D, in the vectors' type F
+// (float, or double for the forms with FP64 vectors).
 //
 // The same preconditioner as the reference's level-0 smooth /
 // restrictResidual / prolongateAdd (uaamg_preconditioner_3d.cpp:123-181).
@@ -12,14 +13,15 @@
 //   even cells: z = (r + sum_nb c x'_nb) / d    (reverse sweep, even colour)
 //   odd  cells: z = (r + sum_nb c z_nb) / d     (reverse sweep, odd colour)
 //   isolated cells keep x'.
-// These are identities in exact arithmetic; the FP32 path rounds them
-// differently from the FP64 parity kernels (which keep the reference order).
+// These are identities in exact arithmetic; they round differently from the
+// per-pass and march kernels (which keep the reference's order), in FP64 by a
+// few units of its last place (the parity bar of a V-cycle is 1e-12).
 // Level-0 couplings are 1/h^2 on every face between two fluid interior cells
 // and 0 otherwise, and x is 0 on every non-fluid cell, so the neighbour sums
 // use the per-axis constants.
 //
 // Mapping (wave64): a wave owns whole x-rows, CPL consecutive cells per lane
-// (nx <= 64*CPL, no x halo); RW rows per wave, NW waves stacked in y (2 halo
+// (nx <= 64*CPL, no x halo; wider grids: WIN, below); RW rows per wave, NW waves stacked in y (2 halo
 // rows on each side of the tile); the workgroup marches along z over a chunk
 // of KC planes (+2 halo planes each side).  Colours are compile-time per
 // (cell, row, plane slot), so no lane idles on the other colour.  x-neighbours
@@ -28,6 +30,13 @@
 // queue.  The 2x2x2 restriction children all live in one thread.  Workgroups
 // are numbered XCD-first (consecutive ids go to different XCDs), so the tiles
 // one XCD runs are neighbours in y and share their halo rows in its L2.
+//
+// WIN: rows wider than 64 CPL cells are cut into windows of 64 lanes; each
+// window owns up to 62 lanes (63 at a wall) and recomputes one lane of halo on
+// its inner sides, which covers the two cells that the sweeps reach.  At
+// 512 x 256 x 256 FP32 the three level-0 kernels read and write what they do
+// at 256^3 per cell; the 64 x 16 march tiles they replace, whose planes cost
+// four barriers, took FILLME.
 #pragma once
 #include <type_traits>
 #include "common.hpp"
@@ -37,21 +46,30 @@ namespace uaamg {
 // Level-0 stencil constants of the FP32 path: 1/d and d per neighbour pattern
 // (nb >> 1 = +x,-x,+y,-y,+z,-z present; 1/d = 0 where d < 1e-30).  Dirichlet
 // walls add their excess per cell.
-struct RowTab {
-    float rinv[64];
-    float d[64];
-    float idx2, idy2, idz2;
-    float ex[6];
+template <typename F>
+struct RowTabOf {
+    F rinv[64];
+    F d[64];
+    F idx2, idy2, idz2;
+    F ex[6];
     int any_dirichlet;
 };
+using RowTab = RowTabOf<float>;
 
 struct RowGeo {
     int nty;       // tiles in y
     int nkc;       // chunks in z
     int KC;        // planes per chunk (multiple of 4)
-    int ntiles;    // nty * nkc
+    int ntiles;    // nwx * nty * nkc
     int per_xcd;   // ceil(ntiles / 8)
+    int nwx;       // windows in x (1: a wave owns whole rows)
+    int wl;        // lanes a window owns (the last one: the rest)
 };
+
+// a b + c: one FMA on FP32 vectors; FP64 vectors keep the separate roundings
+// of the flat kernels
+__device__ __forceinline__ float rfma(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double rfma(double a, double b, double c) { return a * b + c; }
 
 // Whole-wave shifts by one lane with DPP (wave_shr:1 = 0x138, wave_shl:1 =
 // 0x130; all rows and banks enabled, lanes with no source keep old = 0):
@@ -61,6 +79,15 @@ __device__ __forceinline__ float lane_from_left(float v) {   // lane l gets lane
 }
 __device__ __forceinline__ float lane_from_right(float v) {  // lane l gets lane l+1; lane 63 gets 0
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xF, 0xF, false));
+}
+struct F2 { float a, b; };
+__device__ __forceinline__ double lane_from_left(double v) {
+    const F2 f = __builtin_bit_cast(F2, v);
+    return __builtin_bit_cast(double, F2{lane_from_left(f.a), lane_from_left(f.b)});
+}
+__device__ __forceinline__ double lane_from_right(double v) {
+    const F2 f = __builtin_bit_cast(F2, v);
+    return __builtin_bit_cast(double, F2{lane_from_right(f.a), lane_from_right(f.b)});
 }
 
 // tile of block b of a single-grid launch: consecutive block ids go
@@ -72,14 +99,14 @@ __device__ __forceinline__ int row_tile_of_block(const RowGeo& rg, int b) {
 
 // 1/d of the RW x CPL cells of a lane's plane (0 on non-fluid cells and
 // where d < 1e-30): without Dirichlet walls the table value; with them d =
-// the table's d plus each touching wall's excess, divided in FP32.  Every
+// the table's d plus each touching wall's excess, divided in F.  Every
 // table read is issued before the first is used (one LDS round trip per
 // plane, not one per cell) and the Dirichlet test is one uniform branch.
-template <int RW, int CPL>
-__device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], float (&ri)[RW][CPL], const float* srinv,
-                                                const float* sd, const RowTab& T, const Geo& g, int i0,
+template <int RW, int CPL, typename F>
+__device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], F (&ri)[RW][CPL], const F* srinv,
+                                                const F* sd, const RowTabOf<F>& T, const Geo& g, int i0,
                                                 const int (&jrow)[RW], int k) {
-    float v[RW][CPL];
+    F v[RW][CPL];
     if (!T.any_dirichlet) {
 #pragma unroll
         for (int t = 0; t < RW; t++)
@@ -88,7 +115,7 @@ __device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], fl
 #pragma unroll
         for (int t = 0; t < RW; t++)
 #pragma unroll
-            for (int q = 0; q < CPL; q++) ri[t][q] = (nb[t][q] & NB_FLUID) ? v[t][q] : 0.0f;
+            for (int q = 0; q < CPL; q++) ri[t][q] = (nb[t][q] & NB_FLUID) ? v[t][q] : F(0);
     } else {
 #pragma unroll
         for (int t = 0; t < RW; t++)
@@ -98,7 +125,7 @@ __device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], fl
         for (int t = 0; t < RW; t++)
 #pragma unroll
             for (int q = 0; q < CPL; q++) {
-                float d = v[t][q];
+                F d = v[t][q];
                 const int i = i0 + q, j = jrow[t];
                 if (i == 1) d += T.ex[0];
                 if (i == g.nx) d += T.ex[1];
@@ -106,7 +133,7 @@ __device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], fl
                 if (j == g.ny) d += T.ex[3];
                 if (k == 1) d += T.ex[4];
                 if (k == g.nz) d += T.ex[5];
-                ri[t][q] = (nb[t][q] & NB_FLUID) ? (d >= 1e-30f ? 1.0f / d : 0.0f) : 0.0f;
+                ri[t][q] = (nb[t][q] & NB_FLUID) ? (d >= F(1e-30) ? F(1) / d : F(0)) : F(0);
             }
     }
 }
@@ -116,35 +143,40 @@ __device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], fl
 // types carry 4-byte (values) and 1-byte (bytes) alignment; gfx950 global
 // loads take unaligned addresses.  Lanes past nx read the ghost cell and what
 // follows it (inside the array and its margin) and are masked with okx.
-template <int CPL> struct RowVec;
-template <> struct RowVec<4> {
+template <int CPL, typename F = float> struct RowVec;
+template <> struct RowVec<4, float> {
     typedef float V __attribute__((ext_vector_type(4), aligned(4)));
     typedef uint32_t B __attribute__((aligned(1)));
 };
-template <> struct RowVec<2> {
+template <> struct RowVec<2, float> {
     typedef float V __attribute__((ext_vector_type(2), aligned(4)));
     typedef uint16_t B __attribute__((aligned(1)));
 };
-template <int CPL, bool NT = false>
-__device__ __forceinline__ void row_load(const float* __restrict__ r, const uint8_t* __restrict__ nbr, int id,
-                                         const bool (&okx)[CPL], float (&vr)[CPL], uint8_t (&vn)[CPL]) {
-    typename RowVec<CPL>::V v;
-    if constexpr (NT) v = __builtin_nontemporal_load((const typename RowVec<CPL>::V*)(r + id));
-    else v = *(const typename RowVec<CPL>::V*)(r + id);
-    const uint32_t b = *(const typename RowVec<CPL>::B*)(nbr + id);
+template <> struct RowVec<2, double> {
+    typedef double V __attribute__((ext_vector_type(2), aligned(8)));
+    typedef uint16_t B __attribute__((aligned(1)));
+};
+template <int CPL, bool NT = false, typename F>
+__device__ __forceinline__ void row_load(const F* __restrict__ r, const uint8_t* __restrict__ nbr, int id,
+                                         const bool (&okx)[CPL], F (&vr)[CPL], uint8_t (&vn)[CPL]) {
+    using V = typename RowVec<CPL, F>::V;
+    V v;
+    if constexpr (NT) v = __builtin_nontemporal_load((const V*)(r + id));
+    else v = *(const V*)(r + id);
+    const uint32_t b = *(const typename RowVec<CPL, F>::B*)(nbr + id);
 #pragma unroll
     for (int q = 0; q < CPL; q++) {
-        vr[q] = okx[q] ? v[q] : 0.0f;
+        vr[q] = okx[q] ? v[q] : F(0);
         vn[q] = okx[q] ? (uint8_t)(b >> (8 * q)) : (uint8_t)0;
     }
 }
 
-template <int CPL, int NW, int RW>
+template <int CPL, int NW, int RW, typename F = float>
 struct RowLDS {
-    float tab[2][64];
+    F tab[2][64];
     // rows shared between waves: [buffer][kind 0: S1 output, 1: S2 output]
     // [wave][0: first row, 1: last row][colour cell q/2][lane]
-    float ex[2][2][NW][2][CPL / 2][64];
+    F ex[2][2][NW][2][CPL / 2][64];
 };
 
 template <int V> using IC = std::integral_constant<int, V>;
@@ -152,10 +184,10 @@ template <int V> using IC = std::integral_constant<int, V>;
 // Sum over the 6 neighbours of cell (T, Q) of plane slot s: in-plane values
 // from X[s] (other waves' rows from the LDS exchange eb/kind), z-neighbours
 // from slots sp and sm; edge = the neighbour across the lane boundary.
-template <int CPL, int NW, int RW, int T, int Q, int s, int sp, int sm>
-__device__ __forceinline__ float row_nsum(const float (&X)[4][RW][CPL], float edge, const RowLDS<CPL, NW, RW>& L,
-                                          int eb, int kind, int w, int lane, const RowTab& K) {
-    float xl, xr, xu, xd;
+template <int CPL, int NW, int RW, int T, int Q, int s, int sp, int sm, typename F>
+__device__ __forceinline__ F row_nsum(const F (&X)[4][RW][CPL], F edge, const RowLDS<CPL, NW, RW, F>& L,
+                                      int eb, int kind, int w, int lane, const RowTabOf<F>& K) {
+    F xl, xr, xu, xd;
     if constexpr (Q > 0) xl = X[s][T][Q - 1]; else xl = edge;
     if constexpr (Q < CPL - 1) xr = X[s][T][Q + 1]; else xr = edge;
     if constexpr (T > 0) xu = X[s][T - 1][Q]; else xu = L.ex[eb][kind][w > 0 ? w - 1 : 0][1][Q / 2][lane];
@@ -178,27 +210,40 @@ __device__ __forceinline__ void sfor(F&& f) {
 // launch guarantees nx == 64 CPL, so okx and full are compile-time true and
 // every lane mask folds away (the masks cost about a tenth of the level-0
 // kernels' VALU instructions).
-template <int CPL, int NW, int RW, int H = 2, bool FULL = false>
+// WIN: window tx of the row; okw masks what the window owns (its stores,
+// sums and coarse cells), okx what lies in the row.
+template <int CPL, int NW, int RW, int H = 2, bool FULL = false, bool WIN = false>
 struct RowThread {
     static constexpr int TY = NW * RW - 2 * H;
     int lane, w, i0, b0, m0, last;
     int jrow[RW];
     int roff[RW];
     bool okx[CPL];
+    bool okw[CPL];
     bool tile_row[RW];
-    bool full;        // every lane of every row is inside the grid (nx == 64 CPL)
-    __device__ void init(const Geo& g, const RowGeo& rg, int ty, int kc) {
+    bool full;        // every lane of every row is inside the grid and owned (nx == 64 CPL)
+    int kc;           // z-chunk
+    __device__ void init(const Geo& g, const RowGeo& rg, int tile) {
+        int t2 = tile, tx = 0;
+        if constexpr (WIN) { tx = tile % rg.nwx; t2 = tile / rg.nwx; }
+        init(g, rg, t2 % rg.nty, t2 / rg.nty, tx);
+    }
+    __device__ void init(const Geo& g, const RowGeo& rg, int ty, int kc_, int tx = 0) {
+        static_assert(!(FULL && WIN), "a full row is one window");
+        kc = kc_;
         lane = threadIdx.x & 63;
         // the wave index is uniform: in a scalar register, the row tests
         // below (jrow, tile_row) are scalar branches, not exec-mask ones
         w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        full = FULL || g.nx == 64 * CPL;
-        i0 = 1 + CPL * lane;
+        full = !WIN && (FULL || g.nx == 64 * CPL);
+        const int l0 = WIN && tx > 0 ? tx * rg.wl - 1 : 0;   // the row's lane that lane 0 of this window is
+        i0 = 1 + CPL * (l0 + lane);
         b0 = 1 + ty * TY;
         m0 = 1 + kc * rg.KC;
         last = min(m0 + rg.KC - 1, g.nz);
+        const bool own = !WIN || (l0 + lane >= tx * rg.wl && l0 + lane < (tx + 1) * rg.wl);
 #pragma unroll
-        for (int q = 0; q < CPL; q++) okx[q] = FULL || i0 + q <= g.nx;
+        for (int q = 0; q < CPL; q++) { okx[q] = FULL || i0 + q <= g.nx; okw[q] = own && okx[q]; }
 #pragma unroll
         for (int t = 0; t < RW; t++) {
             jrow[t] = b0 - H + w * RW + t;
@@ -235,9 +280,10 @@ struct FinUpd {
     Ctrl* ctrl = nullptr;
 };
 
-struct RUpd {
-    const float* Ap = nullptr;
-    float* rnew = nullptr;
+template <typename F>
+struct RUpdOf {
+    const F* Ap = nullptr;
+    F* rnew = nullptr;
     double* partials = nullptr;      // r.r partials (this kernel's)
     const double* pap = nullptr;     // p.Ap partials of the operator pass
     int npap = 0;
@@ -245,18 +291,19 @@ struct RUpd {
     int xslot = 0;                   // ctrl->xa slot of this iteration's x pass (its p buffer)
 };
 
-template <int CPL, int NW, int RW, typename VC, bool FR = false, bool NT = false, bool FULL = false>
-__device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
-                                             const RowTab& K, const RowGeo& rg, VC* __restrict__ bc, const Geo& cg,
-                                             const int* skip, int tile, const RUpd& u = RUpd{}) {
+template <int CPL, int NW, int RW, typename VC, bool FR = false, bool NT = false, bool FULL = false, bool WIN = false, typename F>
+__device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
+                                             const RowTabOf<F>& K, const RowGeo& rg, VC* __restrict__ bc, const Geo& cg,
+                                             const int* skip, int tile, const RUpdOf<F>& u = RUpdOf<F>{}) {
+    using RV = typename RowVec<CPL, F>::V;
     static_assert(CPL % 2 == 0 && RW % 2 == 0, "pairs of cells and rows");
     if (skip && *skip) {
         // a stopped solve: no x update for this iteration
         if constexpr (FR) { if (blockIdx.x == 0 && threadIdx.x == 0) u.ctrl->xa[u.xslot] = 0.0; }
         return;
     }
-    __shared__ RowLDS<CPL, NW, RW> L;
-    float alpha = 0.0f;   // r update in FP32 (one FMA), as in k_rows_pmv
+    __shared__ RowLDS<CPL, NW, RW, F> L;
+    F alpha = F(0);   // FP32: r update in FP32 (one FMA), as in k_rows_pmv
     if constexpr (FR) {
         __shared__ double s_pap;
         double tot[1];
@@ -278,36 +325,35 @@ __device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const 
             c->first = 0;
         }
         if (!ok) return;   // the whole solve stops; the finish after this kernel sees done
-        alpha = (float)(u.ctrl->rz / pAp);
+        alpha = (F)(u.ctrl->rz / pAp);
     }
     if (tile >= rg.ntiles) {   // the whole workgroup leaves together
         if constexpr (FR) { double z0[1] = {0.0}; block_store<1>(z0, u.partials); }
         return;
     }
-    const int ty = tile % rg.nty, kc = tile / rg.nty;
     double rr[1] = {0.0};
-    RowThread<CPL, NW, RW, 2, FULL> th;
-    th.init(g, rg, ty, kc);
+    RowThread<CPL, NW, RW, 2, FULL, WIN> th;
+    th.init(g, rg, tile);
     const int lane = th.lane, w = th.w;
     for (int e = threadIdx.x; e < 64; e += NW * 64) { L.tab[0][e] = K.rinv[e]; L.tab[1][e] = K.d[e]; }
-    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = 0.0f;
+    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = F(0);
     __syncthreads();
 
-    float X[4][RW][CPL], Rq[2][RW][CPL], Iq[4][RW][CPL];
-    float pfr[2][RW][CPL];
-    float pfa[FR ? 2 : 1][RW][CPL];
+    F X[4][RW][CPL], Rq[2][RW][CPL], Iq[4][RW][CPL];
+    F pfr[2][RW][CPL];
+    F pfa[FR ? 2 : 1][RW][CPL];
     uint8_t pfn[2][RW][CPL];
-    float acc[RW / 2][CPL / 2];
+    F acc[RW / 2][CPL / 2];
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
         for (int t = 0; t < RW; t++)
 #pragma unroll
-            for (int q = 0; q < CPL; q++) { X[s][t][q] = 0.0f; Rq[s & 1][t][q] = 0.0f; Iq[s][t][q] = 0.0f; }
+            for (int q = 0; q < CPL; q++) { X[s][t][q] = F(0); Rq[s & 1][t][q] = F(0); Iq[s][t][q] = F(0); }
 #pragma unroll
     for (int a = 0; a < RW / 2; a++)
 #pragma unroll
-        for (int c = 0; c < CPL / 2; c++) acc[a][c] = 0.0f;
+        for (int c = 0; c < CPL / 2; c++) acc[a][c] = F(0);
 
     auto issue = [&](int slot, int P) {
         // unconditional loads from clamped addresses: straight-line code lets
@@ -317,9 +363,9 @@ __device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const 
         for (int t = 0; t < RW; t++) {
             row_load<CPL, NT>(r, nbr, th.roff[t] + po, th.okx, pfr[slot][t], pfn[slot][t]);
             if constexpr (FR) {
-                typename RowVec<CPL>::V v;
-                if constexpr (NT) v = __builtin_nontemporal_load((const typename RowVec<CPL>::V*)(u.Ap + th.roff[t] + po));
-                else v = *(const typename RowVec<CPL>::V*)(u.Ap + th.roff[t] + po);
+                RV v;
+                if constexpr (NT) v = __builtin_nontemporal_load((const RV*)(u.Ap + th.roff[t] + po));
+                else v = *(const RV*)(u.Ap + th.roff[t] + po);
 #pragma unroll
                 for (int q = 0; q < CPL; q++) pfa[slot][t][q] = v[q];
             }
@@ -341,45 +387,45 @@ __device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const 
             const bool pin = P >= th.m0 && P <= th.last;
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
-                float rs = 0.0f;   // the row's r.r in FP32, accumulated in FP64
+                F rs = F(0);   // the row's r.r in F, accumulated in FP64
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     const bool fl = pfn[PB][t][q] & NB_FLUID;
-                    const float rn = fl ? fmaf(-alpha, pfa[PB][t][q], pfr[PB][t][q]) : 0.0f;
+                    const F rn = fl ? rfma(-alpha, pfa[PB][t][q], pfr[PB][t][q]) : F(0);
                     pfr[PB][t][q] = rn;
-                    rs = fmaf(th.okx[q] ? rn : 0.0f, rn, rs);
+                    rs = rfma(th.okw[q] ? rn : F(0), rn, rs);
                 });
                 if (pin && th.tile_row[t]) rr[0] += (double)rs;
                 if (pin && th.tile_row[t]) {
                     const int id = th.roff[t] + P * (int)g.sy;
-                    if (th.full || th.okx[CPL - 1]) {
-                        typename RowVec<CPL>::V v;
+                    if (th.full || th.okw[CPL - 1]) {
+                        RV v;
 #pragma unroll
                         for (int q = 0; q < CPL; q++) v[q] = pfr[PB][t][q];
-                        *(typename RowVec<CPL>::V*)(u.rnew + id) = v;
+                        *(RV*)(u.rnew + id) = v;
                     } else {
 #pragma unroll
                         for (int q = 0; q < CPL; q++)
-                            if (th.okx[q]) u.rnew[id + q] = pfr[PB][t][q];
+                            if (th.okw[q]) u.rnew[id + q] = pfr[PB][t][q];
                     }
                 }
             });
         }
-        float riP[RW][CPL];
-        rows_rinv_plane<RW, CPL>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
+        F riP[RW][CPL];
+        rows_rinv_plane<RW, CPL, F>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
         sfor<RW>([&](auto tc) {
             constexpr int t = decltype(tc)::value;
             sfor<CPL>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
                 const uint8_t nb = pfn[PB][t][q];
-                const float rv = (nb & NB_FLUID) ? pfr[PB][t][q] : 0.0f;
-                const float ri = riP[t][q];
+                const F rv = (nb & NB_FLUID) ? pfr[PB][t][q] : F(0);
+                const F ri = riP[t][q];
                 Rq[S & 1][t][q] = rv;
                 Iq[S][t][q] = ri;
                 // isolated fluid cells (ri == 0, no fluid neighbour: their x is
                 // never read) carry r, their residual; non-fluid cells carry 0
-                if constexpr (((q + t + S) & 1) == 1) X[S][t][q] = (ri != 0.0f) ? rv * ri : rv;
-                else X[S][t][q] = (ri != 0.0f) ? 0.0f : rv;
+                if constexpr (((q + t + S) & 1) == 1) X[S][t][q] = (ri != F(0)) ? rv * ri : rv;
+                else X[S][t][q] = (ri != F(0)) ? F(0) : rv;
             });
         });
         issue(PB, min(P + 2, th.last + 2));   // past last + 2 (never used): the cached plane last + 2 again, no memory traffic
@@ -393,15 +439,15 @@ __device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const 
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
                 constexpr bool q0 = ((t + S1) & 1) == 0;   // cell 0 of this row is even
-                const float edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
+                const F edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     if constexpr (((q + t + S1) & 1) == 0) {
-                        const float s = row_nsum<CPL, NW, RW, t, q, S1, S, S2>(X, edge, L, ER, 0, w, lane, K);
+                        const F s = row_nsum<CPL, NW, RW, t, q, S1, S, S2, F>(X, edge, L, ER, 0, w, lane, K);
                         // (r + s) / d on cells with 1/d != 0; isolated and non-fluid
                         // cells keep X.  Written as a blend so it stays branch-free.
-                        const float ri = Iq[S1][t][q];
-                        X[S1][t][q] = (Rq[S1 & 1][t][q] + s) * ri + ((ri != 0.0f) ? 0.0f : X[S1][t][q]);
+                        const F ri = Iq[S1][t][q];
+                        X[S1][t][q] = (Rq[S1 & 1][t][q] + s) * ri + ((ri != F(0)) ? F(0) : X[S1][t][q]);
                     }
                 });
             });
@@ -419,21 +465,21 @@ __device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const 
 #pragma unroll
                 for (int a = 0; a < RW / 2; a++)
 #pragma unroll
-                    for (int c = 0; c < CPL / 2; c++) acc[a][c] = 0.0f;
+                    for (int c = 0; c < CPL / 2; c++) acc[a][c] = F(0);
             }
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
                 constexpr bool q0 = ((t + S2) & 1) == 1;   // cell 0 of this row is odd
-                const float edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
+                const F edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     if constexpr (((q + t + S2) & 1) == 1) {
-                        const float s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3>(X, edge, L, ER, 1, w, lane, K);
-                        const bool iso = Iq[S2][t][q] == 0.0f;
-                        acc[t / 2][q / 2] += (iso ? 0.0f : s) + (iso ? X[S2][t][q] : 0.0f);
+                        const F s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3, F>(X, edge, L, ER, 1, w, lane, K);
+                        const bool iso = Iq[S2][t][q] == F(0);
+                        acc[t / 2][q / 2] += (iso ? F(0) : s) + (iso ? X[S2][t][q] : F(0));
                     } else {
                         // even cells: residual 0 after the even update, r on isolated cells
-                        acc[t / 2][q / 2] += (Iq[S2][t][q] != 0.0f) ? 0.0f : X[S2][t][q];
+                        acc[t / 2][q / 2] += (Iq[S2][t][q] != F(0)) ? F(0) : X[S2][t][q];
                     }
                 });
             });
@@ -446,7 +492,7 @@ __device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const 
 #pragma unroll
                     for (int c = 0; c < CPL / 2; c++) {
                         const int ic = (th.i0 + 2 * c + 1) >> 1;
-                        if (ic <= cg.nx && jc <= cg.ny && kcc <= cg.nz)
+                        if ((!WIN || th.okw[2 * c]) && ic <= cg.nx && jc <= cg.ny && kcc <= cg.nz)
                             bc[ic + jc * (int)cg.sx + kcc * (int)cg.sy] = (VC)acc[a][c];
                     }
                 }
@@ -466,51 +512,51 @@ __device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const 
     if constexpr (FR) block_store<1>(rr, u.partials);
 }
 
-template <int CPL, int NW, int RW, typename VC>
-__global__ __launch_bounds__(NW * 64) void k_rows_down0(const float* __restrict__ r, const uint8_t* __restrict__ nbr,
-                                                        Geo g, RowTab K, RowGeo rg, VC* __restrict__ bc, Geo cg,
+template <int CPL, int NW, int RW, typename VC, bool WIN = false, typename F = float>
+__global__ __launch_bounds__(NW * 64) void k_rows_down0(const F* __restrict__ r, const uint8_t* __restrict__ nbr,
+                                                        Geo g, RowTabOf<F> K, RowGeo rg, VC* __restrict__ bc, Geo cg,
                                                         const int* skip) {
-    d_rows_down0<CPL, NW, RW, VC>(r, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x));
+    d_rows_down0<CPL, NW, RW, VC, false, false, false, WIN, F>(r, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x));
 }
 
 // down0 with the fused residual update (r_old -> r_new, r.r partials) and
 // the operator's finish (alpha from the p.Ap partials)
-template <int CPL, int NW, int RW, typename VC, bool NT = false, bool FULL = false>
-__global__ __launch_bounds__(NW * 64) void k_rows_down0r(const float* __restrict__ rold, const uint8_t* __restrict__ nbr,
-                                                         Geo g, RowTab K, RowGeo rg, VC* __restrict__ bc, Geo cg,
-                                                         const int* skip, const float* __restrict__ Ap,
-                                                         float* __restrict__ rnew, double* partials,
+template <int CPL, int NW, int RW, typename VC, bool NT = false, bool FULL = false, bool WIN = false, typename F = float>
+__global__ __launch_bounds__(NW * 64) void k_rows_down0r(const F* __restrict__ rold, const uint8_t* __restrict__ nbr,
+                                                         Geo g, RowTabOf<F> K, RowGeo rg, VC* __restrict__ bc, Geo cg,
+                                                         const int* skip, const F* __restrict__ Ap,
+                                                         F* __restrict__ rnew, double* partials,
                                                          const double* pap, int npap, Ctrl* ctrl, int xslot) {
-    RUpd u;
+    RUpdOf<F> u;
     u.Ap = Ap; u.rnew = rnew; u.partials = partials; u.pap = pap; u.npap = npap; u.ctrl = ctrl; u.xslot = xslot;
-    d_rows_down0<CPL, NW, RW, VC, true, NT, FULL>(rold, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x), u);
+    d_rows_down0<CPL, NW, RW, VC, true, NT, FULL, WIN, F>(rold, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x), u);
 }
 
 // ------------------------------------------------------------------ up
 // r, coarse x -> z (prolongation + reverse sweep), with sum z, sum r z, sum r
 // over fluid cells reduced per workgroup into partials.
-template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false>
-__device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
-                                           const RowTab& K, const RowGeo& rg, const VCX* __restrict__ xc, const Geo& cg,
-                                           float* __restrict__ z, const int* skip, double* partials, int tile) {
+template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false, bool WIN = false, typename F>
+__device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
+                                           const RowTabOf<F>& K, const RowGeo& rg, const VCX* __restrict__ xc, const Geo& cg,
+                                           F* __restrict__ z, const int* skip, double* partials, int tile) {
     static_assert(CPL % 2 == 0 && RW % 2 == 0, "pairs of cells and rows");
+    using RV = typename RowVec<CPL, F>::V;
     if (skip && *skip) return;
-    __shared__ RowLDS<CPL, NW, RW> L;
+    __shared__ RowLDS<CPL, NW, RW, F> L;
     const bool active = tile < rg.ntiles;   // idle workgroups still store zero partials
-    const int ty = tile % rg.nty, kc = tile / rg.nty;
-    RowThread<CPL, NW, RW, 2, FULL> th;
-    th.init(g, rg, active ? ty : 0, active ? kc : 0);
+    RowThread<CPL, NW, RW, 2, FULL, WIN> th;
+    th.init(g, rg, active ? tile : 0);
     const int lane = th.lane, w = th.w;
     for (int e = threadIdx.x; e < 64; e += NW * 64) { L.tab[0][e] = K.rinv[e]; L.tab[1][e] = K.d[e]; }
-    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = 0.0f;
+    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = F(0);
     __syncthreads();
     double red[3] = {0.0, 0.0, 0.0};
 
     if (active) {
-        float X[4][RW][CPL], Rq[4][RW][CPL], Iq[4][RW][CPL];
-        float pfr[2][RW][CPL];
+        F X[4][RW][CPL], Rq[4][RW][CPL], Iq[4][RW][CPL];
+        F pfr[2][RW][CPL];
         uint8_t pfn[2][RW][CPL];
-        float pfx[2][RW / 2][CPL / 2];
+        F pfx[2][RW / 2][CPL / 2];
         bool pcin[2];
         int coff[RW / 2][CPL / 2];
         bool cok[RW / 2][CPL / 2];
@@ -527,7 +573,7 @@ __device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const ui
 #pragma unroll
             for (int t = 0; t < RW; t++)
 #pragma unroll
-                for (int q = 0; q < CPL; q++) { X[s][t][q] = 0.0f; Rq[s][t][q] = 0.0f; Iq[s][t][q] = 0.0f; }
+                for (int q = 0; q < CPL; q++) { X[s][t][q] = F(0); Rq[s][t][q] = F(0); Iq[s][t][q] = F(0); }
 
         auto issue = [&](int slot, int P) {
             const int po = th.plane(g, P);
@@ -541,7 +587,7 @@ __device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const ui
 #pragma unroll
             for (int a = 0; a < RW / 2; a++)
 #pragma unroll
-                for (int c = 0; c < CPL / 2; c++) pfx[slot][a][c] = (float)xc[coff[a][c] + cpo];
+                for (int c = 0; c < CPL / 2; c++) pfx[slot][a][c] = (F)xc[coff[a][c] + cpo];
         };
         issue(1, th.m0 - 2);
         issue(0, th.m0 - 1);
@@ -553,17 +599,17 @@ __device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const ui
             // S1: plane P: x' = x0 + 2 x_coarse (x0 = r/d on odd cells; the
             // even x0 is replaced by the reverse sweep, except on isolated cells
             // where it is 0)
-            float riP[RW][CPL];
-            rows_rinv_plane<RW, CPL>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
+            F riP[RW][CPL];
+            rows_rinv_plane<RW, CPL, F>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     const uint8_t nb = pfn[PB][t][q];
                     const bool fl = nb & NB_FLUID;
-                    const float rv = fl ? pfr[PB][t][q] : 0.0f;
-                    const float ri = riP[t][q];
-                    const float w2 = (fl && pcin[PB] && cok[t / 2][q / 2]) ? 2.0f * pfx[PB][t / 2][q / 2] : 0.0f;
+                    const F rv = fl ? pfr[PB][t][q] : F(0);
+                    const F ri = riP[t][q];
+                    const F w2 = (fl && pcin[PB] && cok[t / 2][q / 2]) ? F(2) * pfx[PB][t / 2][q / 2] : F(0);
                     Rq[S][t][q] = rv;
                     Iq[S][t][q] = ri;
                     if constexpr (((q + t + S) & 1) == 1) X[S][t][q] = rv * ri + w2;
@@ -581,13 +627,13 @@ __device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const ui
                 sfor<RW>([&](auto tc) {
                     constexpr int t = decltype(tc)::value;
                     constexpr bool q0 = ((t + S1) & 1) == 0;
-                    const float edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
+                    const F edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
                     sfor<CPL>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
                         if constexpr (((q + t + S1) & 1) == 0) {
-                            const float s = row_nsum<CPL, NW, RW, t, q, S1, S, S2>(X, edge, L, ER, 0, w, lane, K);
-                            const float ri = Iq[S1][t][q];
-                            X[S1][t][q] = (Rq[S1][t][q] + s) * ri + ((ri != 0.0f) ? 0.0f : X[S1][t][q]);
+                            const F s = row_nsum<CPL, NW, RW, t, q, S1, S, S2, F>(X, edge, L, ER, 0, w, lane, K);
+                            const F ri = Iq[S1][t][q];
+                            X[S1][t][q] = (Rq[S1][t][q] + s) * ri + ((ri != F(0)) ? F(0) : X[S1][t][q]);
                         }
                     });
                 });
@@ -603,39 +649,39 @@ __device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const ui
                 sfor<RW>([&](auto tc) {
                     constexpr int t = decltype(tc)::value;
                     constexpr bool q0 = ((t + S2) & 1) == 1;
-                    const float edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
+                    const F edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
                     sfor<CPL>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
                         if constexpr (((q + t + S2) & 1) == 1) {
-                            const float s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3>(X, edge, L, ER, 1, w, lane, K);
-                            const float ri = Iq[S2][t][q];
-                            X[S2][t][q] = (Rq[S2][t][q] + s) * ri + ((ri != 0.0f) ? 0.0f : X[S2][t][q]);
+                            const F s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3, F>(X, edge, L, ER, 1, w, lane, K);
+                            const F ri = Iq[S2][t][q];
+                            X[S2][t][q] = (Rq[S2][t][q] + s) * ri + ((ri != F(0)) ? F(0) : X[S2][t][q]);
                         }
                     });
                     if (th.tile_row[t]) {
-                        // the row's CPL cells summed in FP32 (one FMA each), the
-                        // row sums accumulated in FP64
-                        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
+                        // the row's CPL cells summed in F (FP32: one FMA each),
+                        // the row sums accumulated in FP64
+                        F s0 = F(0), s1 = F(0), s2 = F(0);
                         sfor<CPL>([&](auto qc) {
                             constexpr int q = decltype(qc)::value;
-                            const float zv = th.okx[q] ? X[S2][t][q] : 0.0f, rv = th.okx[q] ? Rq[S2][t][q] : 0.0f;
+                            const F zv = th.okw[q] ? X[S2][t][q] : F(0), rv = th.okw[q] ? Rq[S2][t][q] : F(0);
                             s0 += zv;
-                            s1 = fmaf(rv, zv, s1);
+                            s1 = rfma(rv, zv, s1);
                             s2 += rv;
                         });
                         red[0] += (double)s0;
                         red[1] += (double)s1;
                         red[2] += (double)s2;
                         const int id = th.roff[t] + R * (int)g.sy;
-                        if (th.full || th.okx[CPL - 1]) {
-                            typename RowVec<CPL>::V v;
+                        if (th.full || th.okw[CPL - 1]) {
+                            RV v;
 #pragma unroll
                             for (int q = 0; q < CPL; q++) v[q] = X[S2][t][q];
-                            *(typename RowVec<CPL>::V*)(z + id) = v;
+                            *(RV*)(z + id) = v;
                         } else {
 #pragma unroll
                             for (int q = 0; q < CPL; q++)
-                                if (th.okx[q]) z[id + q] = X[S2][t][q];
+                                if (th.okw[q]) z[id + q] = X[S2][t][q];
                         }
                     }
                 });
@@ -655,11 +701,11 @@ __device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const ui
     block_store<3>(red, partials);
 }
 
-template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false>
-__global__ __launch_bounds__(NW * 64) void k_rows_up0(const float* __restrict__ r, const uint8_t* __restrict__ nbr,
-                                                      Geo g, RowTab K, RowGeo rg, const VCX* __restrict__ xc, Geo cg,
-                                                      float* __restrict__ z, const int* skip, double* partials) {
-    d_rows_up0<CPL, NW, RW, VCX, NT, FULL>(r, nbr, g, K, rg, xc, cg, z, skip, partials, row_tile_of_block(rg, blockIdx.x));
+template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false, bool WIN = false, typename F = float>
+__global__ __launch_bounds__(NW * 64) void k_rows_up0(const F* __restrict__ r, const uint8_t* __restrict__ nbr,
+                                                      Geo g, RowTabOf<F> K, RowGeo rg, const VCX* __restrict__ xc, Geo cg,
+                                                      F* __restrict__ z, const int* skip, double* partials) {
+    d_rows_up0<CPL, NW, RW, VCX, NT, FULL, WIN, F>(r, nbr, g, K, rg, xc, cg, z, skip, partials, row_tile_of_block(rg, blockIdx.x));
 }
 
 // ================================================================== record levels

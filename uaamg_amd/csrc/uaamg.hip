@@ -460,11 +460,14 @@ extern "C" size_t uaamg_bytes_required(const uaamg_grid* g, const uaamg_opts* o)
     const size_t N0 = (size_t)g0.N, N4 = (N0 + 3) / 4 * 4;
     const size_t margin = (size_t)((g0.sx + 8 + 63) / 64) * 64;
     // level-0 vectors r, z, p, Ap, x and the second p and r buffers of the
-    // fused CG kernels (3D FP32 forms with rows of at most 256 cells)
-    const bool pmv = g->dim == 3 && !v64 && g0.nx <= 256 && shape.size() >= 2 &&
+    // fused CG kernels (3D, on the level-0 row kernels)
+    int nwx = 1, wl = 64;
+    if (v64) Engine<3, double, double>::row_lanes(g0.nx, nwx, wl);
+    else Engine<3, float, float>::row_lanes(g0.nx, nwx, wl);
+    const bool pmv = g->dim == 3 && shape.size() >= 2 && Engine<3, float, float>::rows_addressable(g0) &&
                      (o->forms & UAAMG_FORM_ROWS) && (o->forms & UAAMG_FORM_PMV);
     size_t bytes = N0 + N4 + kRowSlack + 8 + sizeof(uaamg::Ctrl) + (pmv ? 7 : 5) * (N4 + 2 * margin) * sv;
-    if (pmv) bytes += (size_t)(8 * ((((g0.ny + 15) / 16) * ((g0.nz + 3) / 4) + 7) / 8) + 64) * 8;   // p.Ap partials
+    if (pmv) bytes += (size_t)(8 * (((long)nwx * ((g0.ny + 15) / 16) * ((g0.nz + 3) / 4) + 7) / 8) + 64) * 8;   // p.Ap partials
     long maxb = std::max<long>(cells_launch(g0, g->dim).nblocks(), 2048);
     for (size_t l = 1; l < shape.size(); l++) {
         bytes += (size_t)shape[l].N * (3 * sl + 4 * sr + 1) + (size_t)kRowSlack * 6 * std::max(sl, sr);
@@ -478,7 +481,7 @@ extern "C" size_t uaamg_bytes_required(const uaamg_grid* g, const uaamg_opts* o)
                                       : E2::march_launch(g0, E2::RX0, E2::RY0, o->march_target, o->march_kc_min).grid;
         maxb = std::max(maxb, (long)mg.x * mg.y * mg.z);
         if (g->dim == 3) {
-            const long tiles = (long)((g0.ny + 15) / 16) * ((g0.nz + 3) / 4);
+            const long tiles = (long)nwx * ((g0.ny + 15) / 16) * ((g0.nz + 3) / 4);
             maxb = std::max(maxb, 8 * ((tiles + 7) / 8));
         }
     }
