@@ -626,16 +626,24 @@ public:
             pmv_blocks_ = 8u * (unsigned)pgeo_.per_xcd;
         }
     }
-    // Tiles of the row kernels: TY rows by KC planes, KC a multiple of 4 chosen
-    // so that about 256 tiles (one per CU) cover the level (KC <= 16; more
-    // planes per tile amortise the 4 halo plane steps, more tiles fill the chip)
-    // unless kc_force > 0 sets it
+    // Tiles of the row kernels: TY rows by KC planes, KC a multiple of 4, unless
+    // kc_force > 0 sets it
     static RowGeo make_rowgeo(int ny, int nz, int TY = ROWS_NW * ROWS_RW - 4, int kc_force = 0, int nwx = 1, int wl = 64) {
         RowGeo rg{};
         rg.nwx = nwx;
         rg.wl = wl;
         rg.nty = (ny + TY - 1) / TY;
-        int KC = (int)std::min<long>(16, std::max<long>(4, (long)nz * rg.nty * nwx / 256 / 4 * 4));
+        // fewest plane steps in sequence on a CU: rounds of 256 workgroups
+        // (one per CU: ten waves of about 145 VGPRs) times the planes of a
+        // chunk, its 4 halo planes and about 2 steps' time to start
+        int KC = 4;
+        long best = 0;
+        for (int k = 4; k <= 64; k += 4) {
+            const long tiles = (long)rg.nty * nwx * ((nz + k - 1) / k);
+            const long cost = (tiles + 255) / 256 * (k + 6);
+            if (k == 4 || cost < best) { best = cost; KC = k; }
+            if (tiles <= (long)rg.nty * nwx) break;
+        }
         if (kc_force > 0) KC = std::max(4, kc_force / 4 * 4);
         rg.KC = KC;
         rg.nkc = (nz + KC - 1) / KC;
