@@ -113,7 +113,8 @@ enum {
     UAAMG_FORM_TAIL = 1 << 2,        /* small coarse levels in one LDS-resident workgroup */
     UAAMG_FORM_PMV = 1 << 3,         /* p update fused into the operator pass; with the fused
                                         V-cycle also r update in the level-0 down kernel and
-                                        x update on a second stream */
+                                        x update on a second stream (2D: the finishes of the
+                                        dot products in the launches that use them) */
     UAAMG_FORM_XMASK = 1 << 4,       /* x update reads the mask (default: it does not need to) */
     UAAMG_FORM_NT_X = 1 << 5,        /* nontemporal loads/stores in the x update */
     UAAMG_FORM_NT_P = 1 << 6,        /* nontemporal loads of z, p_old in the operator pass */
@@ -137,7 +138,8 @@ typedef struct {
     double alg_bytes;          /* canonical algorithmic HBM bytes of this solve */
     int    kernel_set;         /* level-0 CG kernels used: 0 separate passes; 1 p update fused into the
                                   operator; 2 in addition r update in the level-0 down kernel and the
-                                  x update on a second stream, beside the coarse levels */
+                                  x update on a second stream, beside the coarse levels (2D: both in
+                                  one launch that also forms alpha) */
     int    forms_used;         /* UAAMG_FORM_* bits of the kernel forms that ran */
 } uaamg_stats;
 

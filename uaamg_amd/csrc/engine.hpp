@@ -19,6 +19,7 @@
 #include "kernels_rows.hpp"
 #include "kernels_tail.hpp"
 #include "kernels_pmv.hpp"
+#include "kernels_tile.hpp"
 #include "kernels_batch.hpp"
 #include "kernels_gmg.hpp"
 
@@ -195,8 +196,12 @@ public:
             throw HipError{hipErrorInvalidValue, "GMG / AMG preconditioners: 2D grids, FP64 or FP32 levels"};
         if (gmg_) { gmg_setup(); gmg_tail_setup(); }
         if (!ident_ && !gmg_) rows_setup(h, wall);   // the identity and GMG / AMG forms run the flat kernels only
+        if (D == 2) {
+            pmv_on_ = t2_pmv(o, shape_);
+            pmv_blocks_ = flat_blocks(2048);
+        }
         timer_.s = stream_;
-        if (pmv_on_) {   // the x update's stream, created before any capture
+        if (D == 3 && pmv_on_) {   // the x update's stream, created before any capture
             HIPCHK(hipStreamCreateWithFlags(&xs_, hipStreamNonBlocking));
             HIPCHK(hipEventCreateWithFlags(&xfork_, hipEventDisableTiming));
             HIPCHK(hipEventCreateWithFlags(&xjoin_, hipEventDisableTiming));
@@ -559,10 +564,91 @@ public:
         k_tail_records<D, SC, C4><<<TAIL_MAXP + targs_.nl - 1, TAIL_THREADS, 0, stream_>>>(targs_, reinterpret_cast<SC*>(tail_rec_));
         HIPCHK(hipGetLastError());
     }
-    void tail_launch(const int* skip) {
+    // nrr > 0: with the convergence test of the nrr r.r partials in partials_
+    void tail_launch(const int* skip, int nrr = 0) {
         targs_.npass = (o_.coarsest_sweeps > 0) ? 2 * o_.coarsest_sweeps + 1 : 0;
         targs_.skip = skip;
+        targs_.rr = nrr ? partials_ : nullptr;
+        targs_.nrr = nrr;
+        targs_.ctrl = ctrl_;
         k_tail<D, S, C4, TAIL_NLMAX><<<1, TAIL_THREADS, 0, stream_>>>(targs_);
+    }
+
+    // ---- 2D tile kernels (kernels_tile.hpp) ----
+    // The CG passes of 2D grids: p update, operator and the finish of the z
+    // sums in one launch, alpha and the CG update in the next, the
+    // convergence test in the tail (kernel_set 2).
+    static bool t2_pmv(const uaamg_opts& o, const std::vector<Geo>& shape) {
+        return (o.forms & UAAMG_FORM_PMV) && o.preconditioner != UAAMG_PRECOND_NONE && shape.size() >= 2;
+    }
+    // the level-0 up launch's workgroups are the march kernel's (252 columns
+    // by KC rows), and so are the partials of the z sums
+    MLaunch up0_launch() const { return mlaunch(g0_, RX0, RY0); }
+    // partials of the z sums (GMG / AMG: of the flat pass)
+    int nzp() const {
+        const MLaunch m = up0_launch();
+        return gmg_ ? (int)flat_blocks(2048) : (int)(m.grid.x * m.grid.z);
+    }
+    int nrr_ = 0;                // r.r partials that the tail finishes (0: none pending)
+    void vcycle_t2(const T* r, T* z, const int* skip) {
+        if constexpr (D == 2) {
+            const int lt = tail_first_ ? tail_first_ : nlevels() - 1;
+            FusedArgs<2, true, CT, C4> A0{g0_, nbr0_, nullptr, c0_};
+            auto coarse = [&](int l) { return FusedArgs<2, false, SC, C4>{lv_[l].g, nullptr, lv_[l].coef, Consts<SC>{}}; };
+            for (int l = 0; l < lt; l++) {
+                Level& C = lv_[l + 1];
+                const unsigned nb = tile_blocks(t2_tiles(lv_[l].g));
+                if (l == 0) {
+                    tlaunch(timer_, UAAMG_K_DOWN0, k_t2_down<true, T, C4, S>, dim3(nb), dim3(T2_THREADS), stream_, r, A0, C.b, C.g, skip);
+                } else {
+                    TScope ts(timer_, UAAMG_K_COARSE);
+                    k_t2_down<false, S, C4, S><<<nb, T2_THREADS, 0, stream_>>>(lv_[l].b, coarse(l), C.b, C.g, skip);
+                }
+                HIPCHK(hipGetLastError());
+            }
+            coarse_solve(skip, nrr_);
+            nrr_ = 0;
+            for (int l = lt - 1; l >= 1; l--) {
+                TScope ts(timer_, UAAMG_K_COARSE);
+                Level& C = lv_[l + 1];
+                k_t2_up<S, C4><<<tile_blocks(t2_tiles(lv_[l].g)), T2_THREADS, 0, stream_>>>(lv_[l].b, coarse(l), C.x, C.g, lv_[l].x, skip);
+                HIPCHK(hipGetLastError());
+            }
+            Level& C = lv_[1];
+            const MLaunch m = up0_launch();
+            const int U = (m.KC + 4 + 3) / 4;
+            if (U <= T2U_MAXU) {
+                auto kern = U <= 2 ? k_t2_up0<2, T, S> : (U == 3 ? k_t2_up0<3, T, S> : k_t2_up0<4, T, S>);
+                const int np = (int)(m.grid.x * m.grid.z);
+                tlaunch(timer_, UAAMG_K_UP0, kern, dim3(tile_blocks(np)), dim3(512), stream_, r, (const uint8_t*)nbr0_, g0_, c0_,
+                        (const S*)C.x, C.g, z, m.KC, (int)m.grid.x, np, skip, partials_);
+            } else {   // longer chunks: the march kernel
+                tlaunch(timer_, UAAMG_K_UP0, k_up_m<2, true, RX0, RY0, PPT0, true, T, C4, T, S>, m.grid, dim3(256), stream_,
+                        r, A0, (const S*)C.x, C.g, z, m.KC, skip, partials_);
+            }
+            // with the fused CG passes the next operator launch does this finish
+            if (!fr_) k_fin_zsums<<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)(m.grid.x * m.grid.z), ctrl_);
+            HIPCHK(hipGetLastError());
+        }
+    }
+    // one CG iteration of the fused 2D form
+    void iteration_t2(T* x, const int* skip) {
+        if constexpr (D == 2) {
+            const T* pold = pbuf(pcur_);
+            T* pnew = pbuf(pcur_ ^ 1);
+            tlaunch(timer_, UAAMG_K_MATVEC, vlap_.d ? k_t2_pmv<T, true> : k_t2_pmv<T, false>, dim3(pmv_blocks_), dim3(FIN_THREADS),
+                    stream_, (const T*)z_, pold, pnew, Ap_, (const uint8_t*)nbr0_, g0_, c0d_, N4_, ctrl_, (const double*)partials_,
+                    nzp(), partials_m_, vlap_);
+            pcur_ ^= 1;
+            const unsigned fb = flat_blocks(2048);
+            tlaunch(timer_, UAAMG_K_UPDATE, k_t2_update<T>, dim3(tile_blocks(fb)), dim3(FIN_THREADS), stream_, x, r_, (const T*)pnew, (const T*)Ap_,
+                    (const uint8_t*)nbr0_, N4_, (int)fb, partials_, (const double*)partials_m_, (int)pmv_blocks_, ctrl_);
+            HIPCHK(hipGetLastError());
+            if (tail_first_ && !gmg_) nrr_ = (int)fb;
+            else k_fin_update<false><<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)fb, ctrl_);
+            vcycle(r_, z_, skip);
+            zsums(skip);
+        }
     }
 
     // ---- level-0 row kernels (3D) ----
@@ -759,7 +845,28 @@ public:
     }
     bool fused_supported() const { return nlevels() >= 2; }
 
+    // the levels below the launched ones: the tail, or the coarsest solve alone
+    // (nrr > 0: the tail runs the convergence test first)
+    void coarse_solve(const int* skip, int nrr) {
+        if (tail_first_) {
+            TScope ts(timer_, UAAMG_K_COARSE);
+            tail_launch(skip, nrr);
+        } else {
+            TScope ts(timer_, UAAMG_K_COARSE);
+            Level& C = lv_[nlevels() - 1];
+            int npass = (o_.coarsest_sweeps > 0) ? 2 * o_.coarsest_sweeps + 1 : 0;
+            if (C.g.N <= CMAX) {
+                k_coarsest<D, CMAX, S, C4><<<1, 256, 0, stream_>>>(C.x, C.b, C.coef, C.g, npass, skip);
+            } else {
+                fill_async(C.x, C.g.N, skip);
+                LevelArgs<S, C4> LC{C.g, C.b, C.x, C.mask, C.coef};
+                coarsest_pass<false>(LC, skip);
+            }
+            HIPCHK(hipGetLastError());
+        }
+    }
     void vcycle_fused(const T* r, T* z, const int* skip) {
+        if constexpr (D == 2) { vcycle_t2(r, z, skip); return; }
         const int nl = nlevels();
         FusedArgs<D, true, CT, C4> A0{g0_, nbr0_, nullptr, c0_};
         const int lt = tail_first_ ? tail_first_ : nl - 1;   // levels >= lt: tail kernel / coarsest solve
@@ -795,22 +902,7 @@ public:
             if (fr_old_ && l > 0 && xfork_level() == l) fork_x();
         }
         if (fr_old_ && !xforked_ && xfork_level() >= lt) fork_x();   // before the tail / coarsest solve
-        if (tail_first_) {
-            TScope ts(timer_, UAAMG_K_COARSE);
-            tail_launch(skip);
-        } else {
-            TScope ts(timer_, UAAMG_K_COARSE);
-            Level& C = lv_[nl - 1];
-            int npass = (o_.coarsest_sweeps > 0) ? 2 * o_.coarsest_sweeps + 1 : 0;
-            if (C.g.N <= CMAX) {
-                k_coarsest<D, CMAX, S, C4><<<1, 256, 0, stream_>>>(C.x, C.b, C.coef, C.g, npass, skip);
-            } else {
-                fill_async(C.x, C.g.N, skip);
-                LevelArgs<S, C4> LC{C.g, C.b, C.x, C.mask, C.coef};
-                coarsest_pass<false>(LC, skip);
-            }
-            HIPCHK(hipGetLastError());
-        }
+        coarse_solve(skip, 0);
         for (int l = lt - 1; l >= 0; l--) {
             Level& C = lv_[l + 1];
             if (l == 0 && rows_cpl_) {
@@ -901,8 +993,9 @@ public:
         T* x = x_is_p() ? reinterpret_cast<T*>(p_dev) : x_;
         forms_used_ = 0;
         // the split update needs the fused V-cycle (its level-0 row kernels)
-        fr_ = pmv_on_ && !o_.flexible && o_.fused && o_.nu_pre == 1 && o_.nu_post == 1 && fused_ok_;
-        start(rhs_dev, p_dev, warm, max_iter, tol, pmv_on_);
+        fr_ = pmv_on_ && !o_.flexible && (gmg_ || (o_.fused && o_.nu_pre == 1 && o_.nu_post == 1 && fused_ok_));
+        pmv_now_ = pmv_on_ && (D == 3 || fr_);   // 2D: with the split update only
+        start(rhs_dev, p_dev, warm, max_iter, tol, pmv_now_);
         const int* skip = &ctrl_->done;
         int it_cap = max_iter;
         int every = std::max(1, o_.check_every);
@@ -950,7 +1043,7 @@ public:
             st->ms_total = std::chrono::duration<double, std::milli>(t1 - t0).count();
             timer_.collect(st);
             st->alg_bytes = alg_bytes(hc.iter);
-            st->kernel_set = fr_ ? 2 : (pmv_on_ ? 1 : 0);
+            st->kernel_set = fr_ ? 2 : (pmv_now_ ? 1 : 0);
             st->forms_used = forms_used();
         }
         return st ? st->status : 0;
@@ -980,7 +1073,8 @@ public:
 
     // UAAMG_FORM_* bits of the forms the last solve ran
     int forms_used() const {
-        int f = forms_used_ | (pmv_on_ ? UAAMG_FORM_PMV : 0) | (fr_ ? UAAMG_FORM_SPLIT : 0);
+        int f = forms_used_;
+        if (!gmg_) f |= (pmv_now_ ? UAAMG_FORM_PMV : 0) | (fr_ ? UAAMG_FORM_SPLIT : 0);
         if (zsums_fused_) {
             f |= (rows_cpl_ ? UAAMG_FORM_ROWS : 0) | (tail_first_ ? UAAMG_FORM_TAIL : 0);
             const int lt = tail_first_ ? tail_first_ : nlevels() - 1;
@@ -1040,13 +1134,14 @@ public:
             }
             HIPCHK(hipGraphLaunch(gexec_[k], stream_));
             forms_used_ |= graph_forms_[k];
-            if (pmv_on_ && (chunk & 1)) pcur_ ^= 1;
+            if (pmv_now_ && (chunk & 1)) pcur_ ^= 1;
             return;
         }
         for (int c = 0; c < chunk; c++) iteration(x, skip);
     }
 
     void iteration(T* x, const int* skip) {
+        if (D == 2 && fr_) { iteration_t2(x, skip); return; }
         const unsigned fb = flat_blocks(2048);
         const T* pv = p_;        // the p of this iteration's operator and update
         unsigned mb = fb;        // workgroups of the operator launch (its partials)
@@ -1059,7 +1154,7 @@ public:
         // at 256^3).  Other forms join every iteration.
         xforked_ = false;
         if (!fr_ || pcur_ == 1) join_x();
-        if (pmv_on_) {
+        if (pmv_now_) {
             const T* pold = pbuf(pcur_);
             T* pnew = pbuf(pcur_ ^ 1);
             // p.Ap partials in their own buffer: the down kernel that sums
@@ -1104,7 +1199,7 @@ public:
             zsums(skip);
             return;
         }
-        if (pmv_on_) pcur_ ^= 1;
+        if (pmv_now_) pcur_ ^= 1;
         if (o_.flexible) {
             tlaunch(timer_, UAAMG_K_UPDATE, k_update<T, true>, dim3(fb), dim3(256), stream_,
                     x, r_, pv, (const T*)Ap_, (const T*)z_, (const uint8_t*)nbr0_, N4_, partials_, ctrl_);
@@ -1116,7 +1211,7 @@ public:
         }
         vcycle(r_, z_, skip);
         zsums(skip);
-        if (!pmv_on_) pupdate();
+        if (!pmv_now_) pupdate();
     }
 
     void zsums(const int*) {
@@ -1124,7 +1219,7 @@ public:
         TScope ts(timer_, UAAMG_K_PUPDATE);
         const unsigned fb = flat_blocks(2048);
         k_zsums<T><<<fb, 256, 0, stream_>>>(z_, r_, nbr0_, N4_, partials_, ctrl_);
-        k_fin_zsums<<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)fb, ctrl_);
+        if (!fr_) k_fin_zsums<<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)fb, ctrl_);
     }
     void pupdate() {
         tlaunch(timer_, UAAMG_K_PUPDATE, k_pupdate<T>, dim3(flat_blocks(2048)), dim3(256), stream_,
@@ -1257,6 +1352,7 @@ private:
     T* r2_ = nullptr;
     double* partials_m_ = nullptr;       // p.Ap partials of k_rows_pmv
     bool pmv_on_ = false;
+    bool pmv_now_ = false;               // this solve uses them
     bool fr_ = false;                    // this solve uses the split update
     const T* fr_old_ = nullptr;          // r_old of the fused down kernel (nullptr: plain)
     // The x update (x += alpha p, k_xupdate) runs on a second stream, forked

@@ -42,7 +42,7 @@ void Engine<D, T, S, R>::allocate() {
     HIPCHK(hipHostMalloc((void**)&ctrl_host_, sizeof(Ctrl), hipHostMallocDefault));
     r_ = dalloc_margin<T>(N4_); z_ = dalloc_margin<T>(N4_); p_ = dalloc_margin<T>(N4_); Ap_ = dalloc_margin<T>(N4_);
     if (!x_is_p()) x_ = dalloc_margin<T>(N4_);
-    if (pmv_on_) { p2_ = dalloc_margin<T>(N4_); r2_ = dalloc_margin<T>(N4_); partials_m_ = dalloc<double>(pmv_blocks_ + 64); }
+    if (pmv_on_) { p2_ = dalloc_margin<T>(N4_); if (D == 3) r2_ = dalloc_margin<T>(N4_); partials_m_ = dalloc<double>(pmv_blocks_ + 64); }
     long maxb = std::max<long>(lc0_.nblocks(), 2048);
     for (int l = 1; l < nl; l++) {
         Level& L = lv_[l];

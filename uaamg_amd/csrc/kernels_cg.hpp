@@ -396,22 +396,34 @@ __global__ void k_update(T* __restrict__ x, T* __restrict__ r, const T* __restri
                          Ctrl* ctrl) {
     d_update<T, FLEX>(x, r, p, Ap, z, nbr, N4, partials, ctrl, blockIdx.x, gridDim.x);
 }
+// What the convergence test reads of the scalars.  Read before anything is
+// stored, they are one memory round trip.
+struct FinState { int done, tol_mode, iter, max_iter; double tol, tolsq; double* hist; };
+__device__ __forceinline__ FinState fin_state(const Ctrl* c) {
+    return FinState{c->done, c->tol_mode, c->iter, c->max_iter, c->tol, c->tolsq, c->hist};
+}
+// r.r of this iteration: history, convergence, iteration cap; whether the solve stops
+__device__ __forceinline__ int fin_update_scalars(Ctrl* ctrl, const FinState& f, double rs) {
+    if (f.done) return 1;
+    const bool conv = (f.tol_mode == 1) ? (rs < f.tolsq) : (sqrt(rs) < f.tol);
+    const int iter = f.iter + 1;
+    const int status = conv ? ST_CONVERGED : (!isfinite(rs) ? ST_NONFINITE : (iter >= f.max_iter ? ST_MAXITER : ST_RUNNING));
+    ctrl->rsnew = rs;
+    if (f.hist) f.hist[f.iter] = rs;
+    ctrl->iter = iter;
+    if (status != ST_RUNNING) { ctrl->done = 1; ctrl->status = status; }
+    return status != ST_RUNNING;
+}
 template <bool FLEX>
 __device__ __forceinline__ void d_fin_update(const double* partials, int nbt, int base, int nb, Ctrl* ctrl) {
-    if (ctrl->done) return;
+    const FinState f = fin_state(ctrl);
+    if (f.done) return;
     double tot[3] = {0.0, 0.0, 0.0};
     if (FLEX) reduce_partials_at<3>(partials, nbt, base, nb, tot);
     else { double t1[1]; reduce_partials_at<1>(partials, nbt, base, nb, t1); tot[0] = t1[0]; }
     if (threadIdx.x == 0) {
-        double rs = tot[0];
-        ctrl->rsnew = rs;
         if (FLEX) ctrl->rz_cross = tot[1] - ctrl->mean_z * tot[2];
-        if (ctrl->hist) ctrl->hist[ctrl->iter] = rs;
-        ctrl->iter += 1;
-        bool conv = (ctrl->tol_mode == 1) ? (rs < ctrl->tolsq) : (sqrt(rs) < ctrl->tol);
-        if (conv) { ctrl->done = 1; ctrl->status = ST_CONVERGED; }
-        else if (!isfinite(rs)) { ctrl->done = 1; ctrl->status = ST_NONFINITE; }
-        else if (ctrl->iter >= ctrl->max_iter) { ctrl->done = 1; ctrl->status = ST_MAXITER; }
+        fin_update_scalars(ctrl, f, tot[0]);
     }
 }
 template <bool FLEX>

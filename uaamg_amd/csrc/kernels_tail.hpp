@@ -16,7 +16,7 @@
 // A thread owns pairs of x-adjacent cells (i odd, i+1): one cell of each
 // colour, so every RBGS pass keeps all lanes busy.
 #pragma once
-#include "kernels_vcycle.hpp"
+#include "kernels_cg.hpp"
 
 namespace uaamg {
 
@@ -50,6 +50,11 @@ struct TailArgs {
     void* x;                       // x of the first tail level (written at the end)
     const int* skip;               // stop flag (nullptr: never skip)
     const void* rec;               // pair records (compute type), TAIL_NSLOT slots at most
+    // the convergence test of this iteration (k_fin_update), run before the
+    // levels: r.r partials (nullptr: no test here) and the scalars
+    const double* rr;
+    int nrr;
+    Ctrl* ctrl;
 };
 
 // Stencils of one owned pair of cells, in the reference channel order.
@@ -341,6 +346,11 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag) {
         asm volatile("" : "+v"(z));
         skipped = gload(A.skip + z);
     }
+    double rs[1] = {0.0};
+    FinState fs{};
+    if (A.rr && tid == 0) fs = fin_state(A.ctrl);
+    if (A.rr && tid < FIN_THREADS)   // the finish kernel's order
+        for (int e = tid; e < A.nrr; e += FIN_THREADS) rs[0] += gload(A.rr + e);
 
     // x = 0 on every level (ghosts included) while the loads are in flight
     for (int l = 0; l < nl; l++) {
@@ -363,6 +373,13 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag) {
         }
     }
     __syncthreads();
+    if (A.rr) {   // one launch less per iteration than a finish kernel of its own (2.7 us)
+        __shared__ int s_stop;
+        block_sum<1>(rs);
+        if (tid == 0) s_stop = fin_update_scalars(A.ctrl, fs, rs[0]);
+        __syncthreads();
+        skipped |= s_stop;
+    }
     if (skipped) return;   // uniform: every thread read the same flag
 
     auto level_down = [&](auto& P, int l) {
