@@ -61,3 +61,27 @@ def test_tile_levels_and_solve(gpu, prec, n, wall):
         a, b = a - a.mean(), b - b.mean()
     bar = (1e-7 if prec == U.FP64 else 2e-5) * np.abs(b).max()
     assert np.abs(a - b).max() <= bar
+
+
+GMG_SIZES = [(111, 47), (112, 48), (113, 49), (57, 97), (168, 72), (169, 73), (224, 25), (300, 200), (80, 40), (40, 24)]
+
+
+@pytest.mark.parametrize("n", GMG_SIZES, ids=lambda n: f"{n[0]}x{n[1]}")
+@pytest.mark.parametrize("kind", [(U.PRECOND_GMG, ob.PRECOND_GMG), (U.PRECOND_AMG, ob.PRECOND_AMG)], ids=["gmg", "amg"])
+def test_gmg_tiles(gpu, kind, n):
+    """The GMG / AMG tile kernels (56 x 24 cells) and their one-workgroup levels
+    at the sizes where tiles end and where levels move into the one workgroup:
+    the FP64 cycle equals the oracle's bit for bit, FP32 to 1e-4."""
+    pb = _problem(n, None)
+    print(f"[gmg tiles] n={n}", flush=True)
+    m = pb.fluid_interior_mask()
+    r = cases.random_rhs(pb, np.random.default_rng(7)) * m
+    zo = ob.precond_apply(pb, r, kind[1])
+    for prec in (U.FP64, U.FP32, U.MIXED_F64):
+        c = U.Context(precision=prec, preconditioner=kind[0])
+        c.set_grid(pb.n, pb.h, pb.solid, pb.wall)
+        z = c.apply(r)
+        c.close()
+        if prec == U.FP64:
+            assert np.array_equal(z[m], zo[m])
+        assert np.abs(z[m] - zo[m]).max() <= 1e-4 * np.abs(zo[m]).max()

@@ -55,6 +55,9 @@ inline Launch cells_launch(const Geo& g, int D) {
     return L;
 }
 
+// elements from one level-0 vector of an engine to the next (256-byte steps)
+inline size_t vec_stride(long N4, long margin) { return ((size_t)N4 + 63) / 64 * 64 + 2 * (size_t)margin; }
+
 // elements allocated past the end of level buffers read by the row kernels
 constexpr long kRowSlack = 64;
 
@@ -363,21 +366,24 @@ public:
     // above it with one tiled launch down and one up per level
     int gmg_lt_ = 0;
     GmgTailArgs gmg_targs_{};
-    size_t gmg_tail_lds_ = 0;
     void gmg_tail_setup() {
         const int nl = nlevels();
         const size_t cb = (sizeof(T) == 8 || sizeof(S) == 8) ? 8 : 4;   // LDS element size, the larger form
         size_t bytes = 0;
         int lt = nl;
         while (lt > 0 && nl - (lt - 1) <= GMG_TAIL_MAXL) {
-            const size_t add = (size_t)shape_[lt - 1].N * (2 * cb + 1);
-            if (bytes + add > (size_t)GMG_TAIL_LDS) break;
+            const Geo& g = shape_[lt - 1];
+            const size_t add = (size_t)g.N * (3 * cb + 1);
+            if (bytes + add > (size_t)GMG_TAIL_LDS || (long)((g.nx + 1) / 2) * g.ny > (long)GMG_TAIL_PAIRS * GMG_TAIL_THREADS) break;
             bytes += add;
             lt--;
         }
         if (lt == nl)   // a coarsest level of side <= coarsest_side in one dimension only, long in the other
             throw HipError{hipErrorInvalidValue, "GMG / AMG: coarsest level too large for the one-workgroup solve"};
         gmg_lt_ = lt;
+        size_t xd = 0;
+        for (int l = 1; l < lt; l++) xd += (size_t)shape_[l].N;
+        if (xd > (size_t)g0_.N) throw HipError{hipErrorInvalidValue, "GMG / AMG: coarse levels larger than the grid"};
     }
     void gmg_tail_args(int csweeps) {
         const int nl = nlevels();
@@ -394,29 +400,40 @@ public:
         }
         A.total = off;
         A.csweeps = csweeps;
-        const size_t cb = gmg_lt_ == 0 ? sizeof(typename CTOf<T>::type) : sizeof(typename CTOf<S>::type);
-        gmg_tail_lds_ = (size_t)off * (2 * cb + 1);
+        A.rr = nrr_ ? partials_ : nullptr;
+        A.nrr = nrr_;
+        A.ctrl = ctrl_;
+        nrr_ = 0;
     }
-    static dim3 gmg_tiles(const Geo& g) { return dim3((unsigned)((g.nx + GT_X - 1) / GT_X), (unsigned)((g.ny + GT_Y - 1) / GT_Y)); }
+    static unsigned gmg_tiles(const Geo& g) { return tile_blocks((long)((g.nx + GT_X - 1) / GT_X) * ((g.ny + GT_Y - 1) / GT_Y)); }
+    // x of the way down of a launched level: level 0 in Ap (free between the
+    // CG update and the next operator pass), the others one after the other in
+    // the p buffer that does not hold p (each level has about a quarter of the
+    // cells of the one above it; nothing reads that buffer's non-fluid cells)
+    S* gmg_xd(int l) const {
+        size_t off = 0;
+        for (int k = 1; k < l; k++) off += (size_t)shape_[k].N;
+        return reinterpret_cast<S*>(pbuf(pcur_ ^ 1)) + off;
+    }
     template <typename VX>
-    void gmg_down(VX* x, const VX* b, const uint8_t* m, int l, const int* skip) {
+    void gmg_down(VX* xd, const VX* b, const uint8_t* m, int l, const int* skip) {
         Level& C = lv_[l + 1];
         auto kern = gmg_ == 2 ? k_gmg_down<true, VX, S> : k_gmg_down<false, VX, S>;
-        kern<<<gmg_tiles(shape_[l]), GT_THREADS, 0, stream_>>>(x, b, m, shape_[l], gmg_c<VX>(l), C.b, C.mask, C.g, skip);
+        kern<<<gmg_tiles(shape_[l]), GT_THREADS, 0, stream_>>>(xd, b, m, shape_[l], gmg_c<VX>(l), C.b, C.mask, C.g, skip);
         HIPCHK(hipGetLastError());
     }
     template <typename VX>
-    void gmg_up(VX* x, const VX* b, const uint8_t* m, int l, const int* skip) {
+    void gmg_up(const VX* xd, VX* x, const VX* b, const uint8_t* m, int l, const int* skip) {
         Level& C = lv_[l + 1];
         auto kern = gmg_ == 2 ? k_gmg_up<true, VX, S> : k_gmg_up<false, VX, S>;
-        kern<<<gmg_tiles(shape_[l]), GT_THREADS, 0, stream_>>>(x, b, m, shape_[l], gmg_c<VX>(l), C.x, C.mask, C.g, skip);
+        kern<<<gmg_tiles(shape_[l]), GT_THREADS, 0, stream_>>>(xd, x, b, m, shape_[l], gmg_c<VX>(l), C.x, C.mask, C.g, skip);
         HIPCHK(hipGetLastError());
     }
     template <typename VF>
     void gmg_tail(VF* x, const VF* b, const int* skip) {
         gmg_tail_args(std::max(0, o_.coarsest_sweeps));
         auto kern = gmg_ == 2 ? k_gmg_tail<true, VF> : k_gmg_tail<false, VF>;
-        kern<<<1, GMG_TAIL_THREADS, gmg_tail_lds_, stream_>>>(gmg_targs_, x, b, skip);
+        kern<<<1, GMG_TAIL_THREADS, 0, stream_>>>(gmg_targs_, x, b, skip);
         HIPCHK(hipGetLastError());
     }
     // z = M r: levels 0 .. lt-1 down (x of each level and b of the next
@@ -428,14 +445,14 @@ public:
             TScope ts(timer_, UAAMG_K_DOWN0);
             const int lt = gmg_lt_;
             for (int l = 0; l < lt; l++) {
-                if (l == 0) gmg_down<T>(z, r, solid0_, 0, skip);
-                else gmg_down<S>(lv_[l].x, lv_[l].b, lv_[l].mask, l, skip);
+                if (l == 0) gmg_down<T>(Ap_, r, solid0_, 0, skip);
+                else gmg_down<S>(gmg_xd(l), lv_[l].b, lv_[l].mask, l, skip);
             }
             if (lt == 0) gmg_tail<T>(z, r, skip);
             else gmg_tail<S>(lv_[lt].x, lv_[lt].b, skip);
             for (int l = lt - 1; l >= 0; l--) {
-                if (l == 0) gmg_up<T>(z, r, solid0_, 0, skip);
-                else gmg_up<S>(lv_[l].x, lv_[l].b, lv_[l].mask, l, skip);
+                if (l == 0) gmg_up<T>(Ap_, z, r, solid0_, 0, skip);
+                else gmg_up<S>(gmg_xd(l), lv_[l].x, lv_[l].b, lv_[l].mask, l, skip);
             }
         }
     }
@@ -644,7 +661,7 @@ public:
             tlaunch(timer_, UAAMG_K_UPDATE, k_t2_update<T>, dim3(tile_blocks(fb)), dim3(FIN_THREADS), stream_, x, r_, (const T*)pnew, (const T*)Ap_,
                     (const uint8_t*)nbr0_, N4_, (int)fb, partials_, (const double*)partials_m_, (int)pmv_blocks_, ctrl_);
             HIPCHK(hipGetLastError());
-            if (tail_first_ && !gmg_) nrr_ = (int)fb;
+            if (tail_first_ || gmg_) nrr_ = (int)fb;   // the tail does the convergence test
             else k_fin_update<false><<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)fb, ctrl_);
             vcycle(r_, z_, skip);
             zsums(skip);
@@ -1434,10 +1451,6 @@ private:
     // stencil loads of k_matvec_dot / k_init_warm touch up to sx+4 cells past
     // the first/last interior cell (2D first/last rows)
     long margin_ = 0;
-    template <typename P> P* dalloc_margin(size_t n) {
-        P* base = dalloc<P>(n + 2 * (size_t)margin_);
-        return base + margin_;
-    }
     template <typename P> P* dalloc(size_t n) {
         void* p = nullptr;
         size_t bytes = n * sizeof(P);

@@ -40,9 +40,15 @@ void Engine<D, T, S, R>::allocate() {
     count_ = dalloc<double>(1);
     ctrl_ = dalloc<Ctrl>(1);
     HIPCHK(hipHostMalloc((void**)&ctrl_host_, sizeof(Ctrl), hipHostMallocDefault));
-    r_ = dalloc_margin<T>(N4_); z_ = dalloc_margin<T>(N4_); p_ = dalloc_margin<T>(N4_); Ap_ = dalloc_margin<T>(N4_);
-    if (!x_is_p()) x_ = dalloc_margin<T>(N4_);
-    if (pmv_on_) { p2_ = dalloc_margin<T>(N4_); if (D == 3) r2_ = dalloc_margin<T>(N4_); partials_m_ = dalloc<double>(pmv_blocks_ + 64); }
+    // the level-0 vectors in one allocation: r, z, p, Ap, x and, where the CG
+    // passes are fused, the second p (GMG / AMG have it in any case, for x of
+    // the coarse levels' way down) and in 3D the second r
+    T** vec[] = {&r_, &z_, &p_, &Ap_, &x_, &p2_, &r2_};
+    const int nv = pmv_on_ ? (D == 3 ? 7 : 6) : (gmg_ ? 6 : 5);
+    const size_t stride = vec_stride(N4_, margin_);
+    T* base = dalloc<T>(nv * stride);
+    for (int q = 0; q < nv; q++) *vec[q] = base + q * stride + margin_;
+    if (pmv_on_) partials_m_ = dalloc<double>(pmv_blocks_ + 64);
     long maxb = std::max<long>(lc0_.nblocks(), 2048);
     for (int l = 1; l < nl; l++) {
         Level& L = lv_[l];

@@ -492,7 +492,7 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z,
                 po[q] = pc[q + 1];
                 v[0] += pm * (double)oq;
             }
-            *(vec4<T>*)(pnew + c0) = po;   // vectors without a fluid cell stay 0
+            *(vec4<T>*)(pnew + c0) = po;   // nothing reads the p of the other cells
         }
         *(vec4<T>*)(Ap + c0) = out;
     }
