@@ -20,6 +20,7 @@
 #include "kernels_tail.hpp"
 #include "kernels_pmv.hpp"
 #include "kernels_tile.hpp"
+#include "kernels_tile3.hpp"
 #include "kernels_batch.hpp"
 #include "kernels_gmg.hpp"
 
@@ -591,6 +592,14 @@ public:
         k_tail<D, S, C4, TAIL_NLMAX><<<1, TAIL_THREADS, 0, stream_>>>(targs_);
     }
 
+    // Record levels on tile kernels (kernels_tile3.hpp): FP32 arithmetic and at
+    // most 512 tiles, which the chip holds at once (two workgroups per CU).
+    // Larger levels read less on the march kernels (tiles: 4.3 x the level;
+    // 256 x 128 x 128, 5120 tiles: 60 / 83 us down / up); in FP64 (one
+    // workgroup per CU, the divisions) both take the same time (64 x 32 x 32:
+    // 7.6 / 6.3 us on tiles, 7.4 / 5.7 marching).
+    bool t3_level(int l) const { return D == 3 && sizeof(SC) == 4 && t3_tiles(lv_[l].g) <= 512; }
+
     // ---- 2D tile kernels (kernels_tile.hpp) ----
     // The CG passes of 2D grids: p update, operator and the finish of the z
     // sums in one launch, alpha and the CG update in the next, the
@@ -826,7 +835,8 @@ public:
                         (const uint8_t*)nbr0_, g0_, rtab_, rgeo_, C.b, C.g, skip, (const T*)Ap_, (T*)r, partials_,
                         (const double*)partials_m_, (int)pmv_blocks_, ctrl_, xslot_);
                 fin_fold_ = fin_foldable();
-                if (!fin_fold_) k_fin_update<false><<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)rows_blocks_, ctrl_);
+                if (!fin_fold_ && tail_first_) nrr_ = (int)rows_blocks_;   // the tail does the convergence test
+                else if (!fin_fold_) k_fin_update<false><<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)rows_blocks_, ctrl_);
                 return;
             }
             auto kern = rows_win_ ? k_rows_down0<ROWS_CPL, ROWS_NW, ROWS_RW, S, true, T> : k_rows_down0<2, ROWS_NW, ROWS_RW, S, false, T>;
@@ -904,22 +914,25 @@ public:
                 Level& F = lv_[l];
                 FusedArgs<D, false, SC, C4> A{F.g, nullptr, F.coef, Consts<SC>{}};
                 MLaunch m = mlaunch(F.g, RXC, RYC);
-                auto kern = k_down_m<D, false, RXC, RYC, PPTC, S, C4, S, C4>;
-                if (fr_old_ && xfork_level() == l && !timer_.on && !capturing_) {
-                    // the fork event rides on this dispatch's completion: no
-                    // marker packet between it and the next kernel on stream_
-                    hipExtLaunchKernelGGL(kern, m.grid, dim3(256), 0, stream_, nullptr, xfork_, 0,
-                                          F.b, A, C.b, C.coef, C.g, m.KC, skip);
-                    fork_recorded_ = true;
-                } else {
-                    kern<<<m.grid, 256, 0, stream_>>>(F.b, A, C.b, C.coef, C.g, m.KC, skip);
-                }
+                auto launch = [&](auto kern, dim3 grid, int threads, auto... args) {
+                    if (fr_old_ && xfork_level() == l && !timer_.on && !capturing_) {
+                        // the fork event rides on this dispatch's completion: no
+                        // marker packet between it and the next kernel on stream_
+                        hipExtLaunchKernelGGL(kern, grid, dim3(threads), 0, stream_, nullptr, xfork_, 0, args...);
+                        fork_recorded_ = true;
+                    } else {
+                        kern<<<grid, threads, 0, stream_>>>(args...);
+                    }
+                };
+                if (t3_level(l)) launch(k_t3_down<S, C4>, dim3(tile_blocks(t3_tiles(F.g))), T3_THREADS, (const S*)F.b, (const C4*)F.coef, F.g, C.b, C.g, skip);
+                else launch(k_down_m<D, false, RXC, RYC, PPTC, S, C4, S, C4>, m.grid, 256, (const S*)F.b, A, C.b, (const C4*)C.coef, C.g, m.KC, skip);
             }
             HIPCHK(hipGetLastError());
             if (fr_old_ && l > 0 && xfork_level() == l) fork_x();
         }
         if (fr_old_ && !xforked_ && xfork_level() >= lt) fork_x();   // before the tail / coarsest solve
-        coarse_solve(skip, 0);
+        coarse_solve(skip, nrr_);
+        nrr_ = 0;
         for (int l = lt - 1; l >= 0; l--) {
             Level& C = lv_[l + 1];
             if (l == 0 && rows_cpl_) {
@@ -935,10 +948,14 @@ public:
             } else {
                 TScope ts(timer_, UAAMG_K_COARSE);
                 Level& F = lv_[l];
-                FusedArgs<D, false, SC, C4> A{F.g, nullptr, F.coef, Consts<SC>{}};
-                MLaunch m = mlaunch(F.g, RXC, RYC);
-                k_up_m<D, false, RXC, RYC, PPTC, false, S, C4, S, S><<<m.grid, 256, 0, stream_>>>(
-                    F.b, A, C.x, C.g, F.x, m.KC, skip, nullptr);
+                if (t3_level(l)) {
+                    k_t3_up<S, C4><<<tile_blocks(t3_tiles(F.g)), T3_THREADS, 0, stream_>>>(F.b, F.coef, F.g, C.x, C.g, F.x, skip);
+                } else {
+                    FusedArgs<D, false, SC, C4> A{F.g, nullptr, F.coef, Consts<SC>{}};
+                    MLaunch m = mlaunch(F.g, RXC, RYC);
+                    k_up_m<D, false, RXC, RYC, PPTC, false, S, C4, S, S><<<m.grid, 256, 0, stream_>>>(
+                        F.b, A, C.x, C.g, F.x, m.KC, skip, nullptr);
+                }
             }
             HIPCHK(hipGetLastError());
         }
