@@ -2,7 +2,8 @@
 whole, longer ones in windows of 60; 4 x 4 rows a tile) at the level-1 sizes
 where tiles and windows begin and end, with every level but the coarsest on
 them (no one-workgroup tail, no row kernels above level 0), Dirichlet walls,
-solids at tile borders.  Bars are the repository's: V-cycle 2e-5 (FP32
+solids at tile borders.  16-bit records, which stay on the march kernels,
+run through the same sizes.  Bars are the repository's: V-cycle 2e-5 (FP32
 levels), 5e-2 (BF16 levels) of the oracle's, pressures 2e-5."""
 import numpy as np
 import pytest

@@ -130,8 +130,8 @@ public:
             kb_init_warm<D, S><<<nflat_, 256, 0, s_>>>(dd_, flat_, pflat_);
             kb_fin_init_warm<S><<<G, FIN_THREADS, 0, s_>>>(dd_, pflat_, nflat_);
         }
-        vcycle();
-        kb_pupdate<S><<<nflat_, 256, 0, s_>>>(dd_, flat_);
+        vcycle(false);
+        pupdate();
         HIPCHK(hipGetLastError());
     }
     bool done() const override { return done_ || eng_.empty(); }
@@ -229,36 +229,60 @@ private:
     // ---- one PCG iteration of every member ----
     void iteration() {
         const int G = size();
-        kb_matvec<D, S><<<nflat_, 256, 0, s_>>>(dd_, flat_, pflat_);
-        kb_fin_matvec<S><<<G, FIN_THREADS, 0, s_>>>(dd_, pflat_, nflat_);
+        kb_matvec<D, S><<<nflat_, 256, 0, s_>>>(dd_, flat_, pap_);
         if (o_.flexible) {
+            kb_fin_matvec<S><<<G, FIN_THREADS, 0, s_>>>(dd_, pap_, nflat_);
             kb_update<S, true><<<nflat_, 256, 0, s_>>>(dd_, flat_, pflat_);
             kb_fin_update<S, true><<<G, FIN_THREADS, 0, s_>>>(dd_, pflat_, nflat_);
+            vcycle(false);
         } else {
-            kb_update<S, false><<<nflat_, 256, 0, s_>>>(dd_, flat_, pflat_);
-            kb_fin_update<S, false><<<G, FIN_THREADS, 0, s_>>>(dd_, pflat_, nflat_);
+            kb_update_f<S><<<nflat_, FIN_THREADS, 0, s_>>>(dd_, flat_, pflat_);
+            vcycle(true);
         }
-        vcycle();
-        kb_pupdate<S><<<nflat_, 256, 0, s_>>>(dd_, flat_);
+        pupdate();
     }
-    void vcycle() {
+    void pupdate() {
+        if (o_.flexible) {
+            kb_fin_zsums<S><<<size(), FIN_THREADS, 0, s_>>>(dd_);
+            kb_pupdate<S><<<nflat_, 256, 0, s_>>>(dd_, flat_);
+        } else {
+            kb_pupdate_f<S><<<nflat_, FIN_THREADS, 0, s_>>>(dd_, flat_);
+        }
+    }
+    // test: with the convergence test of this iteration (in the tail)
+    void vcycle(bool test) {
         const int G = size();
         if constexpr (D == 3) {
             if (nrows_[0]) kb_rows_down0<2, S><<<nrows_[0], 640, 0, s_>>>(dd_, rows_[0]);
             if (nrows_[1]) kb_rows_down0<4, S><<<nrows_[1], 640, 0, s_>>>(dd_, rows_[1]);
+            if (nm0_) kb_march_down0<D, RX0, RY0, PPT0, S><<<nm0_, 256, 0, s_>>>(dd_, m0_);
+        } else {
+            kb_t2_down0<S><<<nm0_, T2_THREADS, 0, s_>>>(dd_, m0_);
         }
-        if (nm0_) kb_march_down0<D, RX0, RY0, PPT0, S><<<nm0_, 256, 0, s_>>>(dd_, m0_);
-        for (int l = 1; l < (int)nc_.size(); l++)
-            if (nc_[l]) kb_march_down<D, RXC, RYC, PPTC, S><<<nc_[l], 256, 0, s_>>>(dd_, c_[l], l);
-        kb_tail<D, S, NLMAX><<<G, TAIL_THREADS, 0, s_>>>(dd_);
-        for (int l = (int)nc_.size() - 1; l >= 1; l--)
-            if (nc_[l]) kb_march_up<D, RXC, RYC, PPTC, S><<<nc_[l], 256, 0, s_>>>(dd_, c_[l], l);
+        for (int l = 1; l < (int)nc_.size(); l++) {
+            if constexpr (D == 3) {
+                if (nt_[l]) kb_t3_down<S><<<nt_[l], T3_THREADS, 0, s_>>>(dd_, t_[l], l);
+                if (nc_[l]) kb_march_down<D, RXC, RYC, PPTC, S><<<nc_[l], 256, 0, s_>>>(dd_, c_[l], l);
+            } else {
+                if (nt_[l]) kb_t2_down<S><<<nt_[l], T2_THREADS, 0, s_>>>(dd_, t_[l], l);
+            }
+        }
+        kb_tail<D, S, NLMAX><<<G, TAIL_THREADS, 0, s_>>>(dd_, test);
+        for (int l = (int)nc_.size() - 1; l >= 1; l--) {
+            if constexpr (D == 3) {
+                if (nt_[l]) kb_t3_up<S><<<nt_[l], T3_THREADS, 0, s_>>>(dd_, t_[l], l);
+                if (nc_[l]) kb_march_up<D, RXC, RYC, PPTC, S><<<nc_[l], 256, 0, s_>>>(dd_, c_[l], l);
+            } else {
+                if (nt_[l]) kb_t2_up<S><<<nt_[l], T2_THREADS, 0, s_>>>(dd_, t_[l], l);
+            }
+        }
         if constexpr (D == 3) {
             if (nrows_[0]) kb_rows_up0<2, S><<<nrows_[0], 640, 0, s_>>>(dd_, rows_[0], prows_[0]);
             if (nrows_[1]) kb_rows_up0<4, S><<<nrows_[1], 640, 0, s_>>>(dd_, rows_[1], prows_[1]);
+            if (nm0_) kb_march_up0<D, RX0, RY0, PPT0, S><<<nm0_, 256, 0, s_>>>(dd_, m0_, pm0_);
+        } else {
+            kb_t2_up0<S><<<nm0_, T2_THREADS, 0, s_>>>(dd_, m0_, pm0_);
         }
-        if (nm0_) kb_march_up0<D, RX0, RY0, PPT0, S><<<nm0_, 256, 0, s_>>>(dd_, m0_, pm0_);
-        kb_fin_zsums<S><<<G, FIN_THREADS, 0, s_>>>(dd_);
     }
 
     // ---- descriptors and work-lists ----
@@ -282,11 +306,17 @@ private:
     void make_lists(long target) {
         const int G = size();
         std::vector<BItem> flat, rows[2], m0;
-        std::vector<std::vector<BItem>> cl;
+        std::vector<std::vector<BItem>> cl, tl;   // per level: march chunks, tiles
+        // flat phases: 4 cells x 256 threads x `trips` loop trips per workgroup,
+        // the fewest with which the chip holds all workgroups at once (2048);
+        // a trip is a memory round trip
+        long vecs = 0;
+        for (int g = 0; g < G; g++) vecs += hd_[g].N4 / 4;
+        const long trips = std::min<long>(4, std::max<long>(1, (vecs + 2048 * 256 - 1) / (2048 * 256)));
         for (int g = 0; g < G; g++) {
             BGrid<S>& d = hd_[g];
-            // flat phases: 4 cells x 256 threads x 4 loop trips per workgroup
-            const long nb = std::min<long>(2048, std::max<long>(1, (d.N4 / 4 + 1023) / 1024));
+            const long per = 256 * trips;
+            const long nb = std::min<long>(2048, std::max<long>(1, (d.N4 / 4 + per - 1) / per));
             d.flat_base = (int)flat.size();
             d.flat_cnt = (int)nb;
             for (long b = 0; b < nb; b++) flat.push_back(BItem{g, (int)b, (int)nb, 0});
@@ -298,6 +328,10 @@ private:
                 d.up_base = (int)L.size();
                 d.up_cnt = d.rgeo.ntiles;
                 for (int t = 0; t < d.rgeo.ntiles; t++) L.push_back(BItem{g, t, 0, 0});
+            } else if constexpr (D == 2) {
+                d.up_base = (int)m0.size();
+                d.up_cnt = t2_tiles(d.g0);
+                for (int t = 0; t < d.up_cnt; t++) m0.push_back(BItem{g, t, 0, 0});
             } else {
                 typename E::MLaunch m = E::march_launch(d.g0, RX0, RY0, target, kc_min_);
                 d.lKC[0] = m.KC;
@@ -307,9 +341,14 @@ private:
                     for (unsigned y = 0; y < m.grid.y; y++)
                         for (unsigned x = 0; x < m.grid.x; x++) m0.push_back(BItem{g, (int)x, (int)y, (int)z});
             }
-            // march levels 1 .. lt-1
+            // levels 1 .. lt-1: tiles, 3D levels of many tiles marching (Engine::t3_level)
             for (int l = 1; l < d.lt; l++) {
-                if ((int)cl.size() <= l) cl.resize(l + 1);
+                if ((int)cl.size() <= l) { cl.resize(l + 1); tl.resize(l + 1); }
+                if (D == 2 || eng_[g]->t3_level(l)) {
+                    const int nt = D == 2 ? t2_tiles(d.lg[l]) : t3_tiles(d.lg[l]);
+                    for (int t = 0; t < nt; t++) tl[l].push_back(BItem{g, t, 0, 0});
+                    continue;
+                }
                 typename E::MLaunch m = E::march_launch(d.lg[l], RXC, RYC, target, kc_min_);
                 d.lKC[l] = m.KC;
                 for (unsigned z = 0; z < m.grid.z; z++)
@@ -320,6 +359,7 @@ private:
         nflat_ = (int)flat.size();
         flat_ = upload(flat);
         pflat_ = dev<double>(3 * (size_t)nflat_ + 64);
+        pap_ = dev<double>((size_t)nflat_ + 64);   // of its own: the update reads these while it writes r.r partials
         for (int c = 0; c < 2; c++) {
             nrows_[c] = (int)rows[c].size();
             rows_[c] = nrows_[c] ? upload(rows[c]) : nullptr;
@@ -330,12 +370,20 @@ private:
         pm0_ = nm0_ ? dev<double>(3 * (size_t)nm0_ + 64) : nullptr;
         nc_.assign(cl.size(), 0);
         c_.assign(cl.size(), nullptr);
+        nt_.assign(tl.size(), 0);
+        t_.assign(tl.size(), nullptr);
         for (size_t l = 1; l < cl.size(); l++) {
+            nt_[l] = (int)tl[l].size();
+            t_[l] = nt_[l] ? upload(tl[l]) : nullptr;
             nc_[l] = (int)cl[l].size();
             c_[l] = nc_[l] ? upload(cl[l]) : nullptr;
         }
         for (int g = 0; g < G; g++) {
             BGrid<S>& d = hd_[g];
+            d.pap = pap_ + d.flat_base;
+            d.tail.rr = pflat_ + d.flat_base;   // one partial per workgroup of the update
+            d.tail.nrr = d.flat_cnt;
+            d.tail.ctrl = d.ctrl;
             if (D == 3 && d.cpl) {
                 const int c = d.cpl == 2 ? 0 : 1;
                 d.up_partials = prows_[c];
@@ -359,6 +407,7 @@ private:
     // arithmetic; only the tiling changes.
     void autotune() {
         tuned_ = true;
+        if (D == 2) return;   // every launch is on tiles of one shape
         const int G = size();
         bool any_rows = false;
         for (int g = 0; g < G; g++) any_rows = any_rows || (D == 3 && hd_[g].cpl);
@@ -370,9 +419,9 @@ private:
             free_lists();
             make_lists(target_);
             kb_ctrl_init<S><<<(G + 63) / 64, 64, 0, s_>>>(dd_, G, 1 << 30, 0.0, o_.tol_mode, 0, o_.project_mean);
-            vcycle();   // warm-up
+            vcycle(false);   // warm-up
             HIPCHK(hipEventRecord(e0, s_));
-            for (int k = 0; k < 3; k++) vcycle();
+            for (int k = 0; k < 3; k++) vcycle(false);
             HIPCHK(hipEventRecord(e1, s_));
             HIPCHK(hipEventSynchronize(e1));
             float ms = 0;
@@ -438,10 +487,10 @@ private:
             (void)hipFree(lists_.back());
             lists_.pop_back();
         }
-        flat_ = nullptr; m0_ = nullptr; pflat_ = nullptr; pm0_ = nullptr;
+        flat_ = nullptr; m0_ = nullptr; pflat_ = pap_ = nullptr; pm0_ = nullptr;
         for (int c = 0; c < 2; c++) { rows_[c] = nullptr; prows_[c] = nullptr; nrows_[c] = 0; }
         nflat_ = nm0_ = 0;
-        nc_.clear(); c_.clear();
+        nc_.clear(); c_.clear(); nt_.clear(); t_.clear();
     }
     void free_all() {
         if (!lists_.empty() || hctrl_) (void)hipStreamSynchronize(s_);
@@ -450,10 +499,10 @@ private:
         keep_ = 0;
         if (hctrl_) (void)hipHostFree(hctrl_);
         hctrl_ = nullptr; ctrl_ = nullptr; dd_ = nullptr;
-        flat_ = nullptr; m0_ = nullptr; pflat_ = nullptr; pm0_ = nullptr;
+        flat_ = nullptr; m0_ = nullptr; pflat_ = pap_ = nullptr; pm0_ = nullptr;
         for (int c = 0; c < 2; c++) { rows_[c] = nullptr; prows_[c] = nullptr; nrows_[c] = 0; }
         nflat_ = nm0_ = 0;
-        nc_.clear(); c_.clear();
+        nc_.clear(); c_.clear(); nt_.clear(); t_.clear();
         bytes_ = 0;
     }
 
@@ -470,10 +519,10 @@ private:
     Ctrl* ctrl_ = nullptr;
     Ctrl* hctrl_ = nullptr;
     BItem *flat_ = nullptr, *m0_ = nullptr, *rows_[2] = {nullptr, nullptr};
-    double *pflat_ = nullptr, *pm0_ = nullptr, *prows_[2] = {nullptr, nullptr};
+    double *pflat_ = nullptr, *pap_ = nullptr, *pm0_ = nullptr, *prows_[2] = {nullptr, nullptr};
     int nflat_ = 0, nm0_ = 0, nrows_[2] = {0, 0};
-    std::vector<int> nc_;
-    std::vector<BItem*> c_;
+    std::vector<int> nc_, nt_;   // per level: march chunks, tiles
+    std::vector<BItem*> c_, t_;
     std::vector<void*> lists_;
     size_t keep_ = 0;
     size_t bytes_ = 0;

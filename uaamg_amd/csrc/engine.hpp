@@ -598,7 +598,9 @@ public:
     // 256 x 128 x 128, 5120 tiles: 60 / 83 us down / up); in FP64 (one
     // workgroup per CU, the divisions) both take the same time (64 x 32 x 32:
     // 7.6 / 6.3 us on tiles, 7.4 / 5.7 marching).
-    bool t3_level(int l) const { return D == 3 && sizeof(SC) == 4 && t3_tiles(lv_[l].g) <= 512; }
+    // 16-bit records stay on the march kernels: their diagonals are formed
+    // from all six couplings, which a tile's border does not have.
+    bool t3_level(int l) const { return D == 3 && std::is_same<C4, float4>::value && t3_tiles(lv_[l].g) <= 512; }
 
     // ---- 2D tile kernels (kernels_tile.hpp) ----
     // The CG passes of 2D grids: p update, operator and the finish of the z

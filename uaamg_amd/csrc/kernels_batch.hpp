@@ -13,6 +13,7 @@
 #include "kernels_march.hpp"
 #include "kernels_rows.hpp"
 #include "kernels_tail.hpp"
+#include "kernels_tile3.hpp"
 
 namespace uaamg {
 
@@ -40,13 +41,14 @@ struct BGrid {
     S* lb[BATCH_MAXL];
     S* lx[BATCH_MAXL];
     C4* lcoef[BATCH_MAXL];
-    int lKC[BATCH_MAXL];               // march chunk per level (level 0 too, when not on rows)
+    int lKC[BATCH_MAXL];               // march chunk per level (3D; level 0 too, when not on rows)
     int cpl;                           // level-0 row kernels: cells per lane (0: march)
     RowTab rtab;
     RowGeo rgeo;
     TailArgs<C4> tail;
     // slices of the reducing launches
     int flat_base, flat_cnt;
+    const double* pap;                 // p.Ap partials of this grid (flat_cnt of them)
     const double* up_partials;
     int up_nbt, up_base, up_cnt;
 };
@@ -135,6 +137,70 @@ __global__ __launch_bounds__(256) void kb_update(BGrid<S>* G, const BItem* items
         return;
     }
     d_update<float, FLEX>(d.x, d.r, d.p, d.Ap, d.z, d.nbr0, d.N4, partials, d.ctrl, it.a, it.b);
+}
+// The finish of the operator (alpha, breakdown), x += alpha p, r -= alpha Ap
+// and the r.r partials: kb_fin_matvec and kb_update in one launch.  Every
+// workgroup adds its grid's p.Ap partials in the finish kernel's order; the
+// grid's first one stores the scalars and rsold for the next beta, which no
+// workgroup of this launch reads.  With the finish of the z sums in
+// kb_pupdate_f and the convergence test in the tail, an iteration has three
+// launches of one workgroup per grid less (4.2 to 4.7 us each).
+template <typename S>
+__global__ __launch_bounds__(FIN_THREADS) void kb_update_f(BGrid<S>* G, const BItem* items, double* partials) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    Ctrl* c = d.ctrl;
+    const int done = c->done, iter = c->iter;
+    const double rz = c->rz;
+    double tot[1] = {0.0};
+    for (int k = threadIdx.x; k < d.flat_cnt; k += FIN_THREADS) tot[0] += d.pap[k];
+    if (done) return;
+    __shared__ double s_pap;
+    block_sum<1>(tot);
+    if (threadIdx.x == 0) s_pap = tot[0];
+    __syncthreads();
+    const double pAp = s_pap;
+    const bool ok = isfinite(pAp) && pAp >= 1e-15;   // pcg.cpp:100 breakdown test
+    const double alpha = rz / pAp;
+    if (it.a == 0 && threadIdx.x == 0) {
+        c->pAp = pAp;
+        if (!ok) { c->done = 1; c->status = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE; c->iter = iter + 1; }
+        c->alpha = c->xalpha = ok ? alpha : 0.0;
+        c->rsold = rz;
+        c->first = 0;
+    }
+    if (!ok) return;
+    d_update_a<float, false>(d.x, d.r, d.p, d.Ap, d.z, d.nbr0, d.N4, partials, alpha, it.a, it.b);
+}
+// The finish of the z sums and the p update; rsold and the first flag are
+// read here and written by the next iteration's kb_update_f.
+template <typename S>
+__global__ __launch_bounds__(FIN_THREADS) void kb_pupdate_f(BGrid<S>* G, const BItem* items) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    Ctrl* c = d.ctrl;
+    const int done = c->done, project = c->project, first = c->first;
+    const double count = c->count, rsold = c->rsold;
+    double tot[3] = {0.0, 0.0, 0.0};
+    for (int k = threadIdx.x; k < d.up_cnt; k += FIN_THREADS)
+#pragma unroll
+        for (int q = 0; q < 3; q++) tot[q] += d.up_partials[(long)q * d.up_nbt + d.up_base + k];
+    if (done) return;
+    __shared__ double s_z[3];
+    block_sum<3>(tot);
+    if (threadIdx.x == 0) { s_z[0] = tot[0]; s_z[1] = tot[1]; s_z[2] = tot[2]; }
+    __syncthreads();
+    const double sz = s_z[0], srz = s_z[1], sr = s_z[2];
+    const double mean = (project && count > 0) ? sz / count : 0.0;
+    const double rz = srz - mean * sr;
+    const double beta = first ? 0.0 : rz / rsold;
+    if (it.a == 0 && threadIdx.x == 0) {
+        c->sum_z = sz; c->sum_rz = srz; c->sum_r = sr;
+        c->mean_z = mean; c->rz = rz; c->beta = beta;
+        if (!isfinite(rz)) { c->done = 1; c->status = ST_NONFINITE; }
+    }
+    if (!isfinite(rz)) return;
+    d_pupdate_a<float>(d.p, d.z, d.nbr0, d.N4, mean, beta, it.a, it.b);
 }
 template <typename S>
 __global__ __launch_bounds__(256) void kb_pupdate(BGrid<S>* G, const BItem* items) {
@@ -244,11 +310,61 @@ __global__ __launch_bounds__(256) void kb_march_up(BGrid<S>* G, const BItem* ite
                                                       &d.ctrl->done, nullptr, it.a, it.b, it.c);
 }
 
+// tile kernels: item = (grid, tile)
+template <typename S>
+__global__ __launch_bounds__(T2_THREADS) void kb_t2_down0(BGrid<S>* G, const BItem* items) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    if (d.ctrl->done) return;
+    const FusedArgs<2, true, float, typename Vec4<S>::type> A{d.g0, d.nbr0, nullptr, d.c0};
+    const int nx = t2_nx(d.g0);
+    d_t2_down<true, float, typename Vec4<S>::type, S>(d.r, A, d.lb[1], d.lg[1], it.a % nx, it.a / nx);
+}
+template <typename S>
+__global__ __launch_bounds__(T2_THREADS) void kb_t2_up0(BGrid<S>* G, const BItem* items, double* partials) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    if (d.ctrl->done) return;
+    const FusedArgs<2, true, float, typename Vec4<S>::type> A{d.g0, d.nbr0, nullptr, d.c0};
+    const int nx = t2_nx(d.g0);
+    d_t2_up<true, float, typename Vec4<S>::type, S>(d.r, A, d.lx[1], d.lg[1], d.z, it.a % nx, it.a / nx, partials + blockIdx.x, gridDim.x);
+}
+template <typename S>
+__global__ __launch_bounds__(T2_THREADS) void kb_t2_down(BGrid<S>* G, const BItem* items, int l) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    if (d.ctrl->done) return;
+    const FusedArgs<2, false, float, typename Vec4<S>::type> A{d.lg[l], nullptr, d.lcoef[l], Consts<float>{}};
+    const int nx = t2_nx(A.g);
+    d_t2_down<false, S, typename Vec4<S>::type, S>(d.lb[l], A, d.lb[l + 1], d.lg[l + 1], it.a % nx, it.a / nx);
+}
+template <typename S>
+__global__ __launch_bounds__(T2_THREADS) void kb_t2_up(BGrid<S>* G, const BItem* items, int l) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    if (d.ctrl->done) return;
+    const FusedArgs<2, false, float, typename Vec4<S>::type> A{d.lg[l], nullptr, d.lcoef[l], Consts<float>{}};
+    const int nx = t2_nx(A.g);
+    d_t2_up<false, S, typename Vec4<S>::type, S>(d.lb[l], A, d.lx[l + 1], d.lg[l + 1], d.lx[l], it.a % nx, it.a / nx);
+}
+template <typename S>
+__global__ __launch_bounds__(T3_THREADS) void kb_t3_down(BGrid<S>* G, const BItem* items, int l) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    d_t3_down<S, typename Vec4<S>::type>(d.lb[l], d.lcoef[l], d.lg[l], d.lb[l + 1], d.lg[l + 1], it.a, &d.ctrl->done);
+}
+template <typename S>
+__global__ __launch_bounds__(T3_THREADS) void kb_t3_up(BGrid<S>* G, const BItem* items, int l) {
+    const BItem it = items[blockIdx.x];
+    const BGrid<S>& d = G[it.g];
+    d_t3_up<S, typename Vec4<S>::type>(d.lb[l], d.lcoef[l], d.lg[l], d.lx[l + 1], d.lg[l + 1], d.lx[l], it.a, &d.ctrl->done);
+}
+
 // the small levels of every grid: one workgroup per grid
 template <int D, typename S, int NLMAX>
-__global__ __launch_bounds__(TAIL_THREADS) void kb_tail(BGrid<S>* G) {
+__global__ __launch_bounds__(TAIL_THREADS) void kb_tail(BGrid<S>* G, int test) {
     const BGrid<S>& d = G[blockIdx.x];
-    d_tail<D, S, typename Vec4<S>::type, NLMAX>(d.tail);
+    d_tail<D, S, typename Vec4<S>::type, NLMAX>(d.tail, test != 0);
 }
 
 }  // namespace uaamg

@@ -361,11 +361,9 @@ static __global__ void k_fin_init_warm(const double* partials, int nb, Ctrl* ctr
 // x += alpha p; r -= alpha Ap (fluid cells); r.r; convergence / iteration cap.
 // FLEX: also (r_new, z_old - mean_old) for the Polak-Ribiere beta.
 template <typename T, bool FLEX>
-__device__ __forceinline__ void d_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ Ap,
+__device__ __forceinline__ void d_update_a(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ Ap,
                          const T* __restrict__ z, const uint8_t* __restrict__ nbr, long N4, double* partials,
-                         Ctrl* ctrl, int fv_b, int fv_n) {
-    if (ctrl->done) return;
-    const double alpha = ctrl->alpha;
+                         double alpha, int fv_b, int fv_n) {
     double v[3] = {0.0, 0.0, 0.0};
     FLAT_LOOP(N4) {
         long c = 4 * v_;
@@ -389,6 +387,13 @@ __device__ __forceinline__ void d_update(T* __restrict__ x, T* __restrict__ r, c
     }
     if (FLEX) block_store<3>(v, partials);
     else { double v1[1] = {v[0]}; block_store<1>(v1, partials); }
+}
+template <typename T, bool FLEX>
+__device__ __forceinline__ void d_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ Ap,
+                         const T* __restrict__ z, const uint8_t* __restrict__ nbr, long N4, double* partials,
+                         Ctrl* ctrl, int fv_b, int fv_n) {
+    if (ctrl->done) return;
+    d_update_a<T, FLEX>(x, r, p, Ap, z, nbr, N4, partials, ctrl->alpha, fv_b, fv_n);
 }
 template <typename T, bool FLEX>
 __global__ void k_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ Ap,
@@ -521,10 +526,8 @@ __global__ void k_xupdate(T* __restrict__ x, const T* __restrict__ p, const uint
 
 // p = (z - mean) + beta p on fluid cells.
 template <typename T>
-__device__ __forceinline__ void d_pupdate(T* __restrict__ p, const T* __restrict__ z, const uint8_t* __restrict__ nbr, long N4,
-                          Ctrl* ctrl, int fv_b, int fv_n) {
-    if (ctrl->done) return;
-    const double mean = ctrl->mean_z, beta = ctrl->beta;
+__device__ __forceinline__ void d_pupdate_a(T* __restrict__ p, const T* __restrict__ z, const uint8_t* __restrict__ nbr, long N4,
+                          double mean, double beta, int fv_b, int fv_n) {
     FLAT_LOOP(N4) {
         long c = 4 * v_;
         uint32_t w = *(const uint32_t*)(nbr + c);
@@ -535,6 +538,12 @@ __device__ __forceinline__ void d_pupdate(T* __restrict__ p, const T* __restrict
             if (nbyte(w, q) & NB_FLUID) pv[q] = (T)(((double)zv[q] - mean) + beta * (double)pv[q]);
         *(vec4<T>*)(p + c) = pv;
     }
+}
+template <typename T>
+__device__ __forceinline__ void d_pupdate(T* __restrict__ p, const T* __restrict__ z, const uint8_t* __restrict__ nbr, long N4,
+                          Ctrl* ctrl, int fv_b, int fv_n) {
+    if (ctrl->done) return;
+    d_pupdate_a<T>(p, z, nbr, N4, ctrl->mean_z, ctrl->beta, fv_b, fv_n);
 }
 template <typename T>
 __global__ void k_pupdate(T* __restrict__ p, const T* __restrict__ z, const uint8_t* __restrict__ nbr, long N4,

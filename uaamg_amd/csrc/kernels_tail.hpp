@@ -51,7 +51,7 @@ struct TailArgs {
     const int* skip;               // stop flag (nullptr: never skip)
     const void* rec;               // pair records (compute type), TAIL_NSLOT slots at most
     // the convergence test of this iteration (k_fin_update), run before the
-    // levels: r.r partials (nullptr: no test here) and the scalars
+    // levels: r.r partials (k_tail: nullptr: no test here) and the scalars
     const double* rr;
     int nrr;
     Ctrl* ctrl;
@@ -298,7 +298,7 @@ __device__ __forceinline__ void tail_restrict(const CT* Rs, CT* BC, CT* XC, cons
 }
 
 template <int D, typename S, typename C4, int NLMAX>
-__device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag) {
+__device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     static_assert(NLMAX >= 2 && NLMAX <= TAIL_MAXL, "tail depth");
     using CT = typename CTOf<S>::type;
     __shared__ __align__(16) CT lds[TAIL_LDS_BYTES / sizeof(CT)];
@@ -348,8 +348,8 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag) {
     }
     double rs[1] = {0.0};
     FinState fs{};
-    if (A.rr && tid == 0) fs = fin_state(A.ctrl);
-    if (A.rr && tid < FIN_THREADS)   // the finish kernel's order
+    if (test && tid == 0) fs = fin_state(A.ctrl);
+    if (test && tid < FIN_THREADS)   // the finish kernel's order
         for (int e = tid; e < A.nrr; e += FIN_THREADS) rs[0] += gload(A.rr + e);
 
     // x = 0 on every level (ghosts included) while the loads are in flight
@@ -373,7 +373,7 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag) {
         }
     }
     __syncthreads();
-    if (A.rr) {   // one launch less per iteration than a finish kernel of its own (2.7 us)
+    if (test) {   // one launch less per iteration than a finish kernel of its own (2.7 us)
         __shared__ int s_stop;
         block_sum<1>(rs);
         if (tid == 0) s_stop = fin_update_scalars(A.ctrl, fs, rs[0]);
@@ -464,7 +464,7 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag) {
 
 template <int D, typename S, typename C4, int NLMAX>
 __global__ __launch_bounds__(TAIL_THREADS) void k_tail(TailArgs<C4> A) {
-    d_tail<D, S, C4, NLMAX>(A);
+    d_tail<D, S, C4, NLMAX>(A, A.rr != nullptr);
 }
 
 }  // namespace uaamg

@@ -186,11 +186,13 @@ __device__ __forceinline__ void d_t2_down(const VB* __restrict__ b, const FusedA
     }
 }
 
-// Up (levels >= 1): x' = x0 + 2 x_coarse, reverse sweep.
-template <typename VB, typename C4>
-__device__ __forceinline__ void d_t2_up(const VB* __restrict__ b, const FusedArgs<2, false, typename CTOf<VB>::type, C4>& A,
-                                        const VB* __restrict__ xc, const Geo& cg, VB* __restrict__ xout, int bx, int by) {
-    constexpr bool L0 = false;
+// Up: x' = x0 + 2 x_coarse, reverse sweep.  Level 0 (of batch members; single
+// grids: d_t2_up0): with the z sums (sum z, sum r z, sum r over fluid cells) of
+// the tile in partials[q np].
+template <bool L0, typename VB, typename C4, typename VCX>
+__device__ __forceinline__ void d_t2_up(const VB* __restrict__ b, const FusedArgs<2, L0, typename CTOf<VB>::type, C4>& A,
+                                        const VCX* __restrict__ xc, const Geo& cg, VB* __restrict__ xout, int bx, int by,
+                                        double* partials = nullptr, int np = 0) {
     using CT = typename CTOf<VB>::type;
     __shared__ T2LDS<CT> S;
     T2Pos t;
@@ -222,6 +224,14 @@ __device__ __forceinline__ void d_t2_up(const VB* __restrict__ b, const FusedArg
     __syncthreads();
     t2_sweep<L0, CT>(S, t, !t.left_odd, t.own, x0, x1, b0, b1, s0, s1);                     // odd cells
     if (t.own && t.in0) t2_put(xout + t.id, (VB)x0, (VB)x1, t.in1);
+    if constexpr (L0) {
+        double red[3] = {0.0, 0.0, 0.0};
+        if (t.own && s0.d >= CT(0)) { const double z = (double)(VB)x0, r = (double)b0; red[0] = z; red[1] = r * z; red[2] = r; }
+        if (t.own && s1.d >= CT(0)) { const double z = (double)(VB)x1, r = (double)b1; red[0] += z; red[1] += r * z; red[2] += r; }
+        block_sum<3>(red);
+        if (threadIdx.x == 0)
+            for (int q = 0; q < 3; q++) partials[(long)q * np] = red[q];
+    }
 }
 
 template <bool L0, typename VB, typename C4, typename VC>
@@ -237,7 +247,7 @@ __global__ __launch_bounds__(T2_THREADS) void k_t2_up(const VB* __restrict__ b, 
                                                       const VB* __restrict__ xc, Geo cg, VB* __restrict__ xout, const int* skip) {
     if (skip && *skip) return;
     const int t = tile_of_block();
-    if (t < t2_tiles(A.g)) d_t2_up<VB, C4>(b, A, xc, cg, xout, t % t2_nx(A.g), t / t2_nx(A.g));
+    if (t < t2_tiles(A.g)) d_t2_up<false, VB, C4, VB>(b, A, xc, cg, xout, t % t2_nx(A.g), t / t2_nx(A.g));
 }
 
 // ---------------------------------------------------------------- level 0, up

@@ -13,8 +13,7 @@
 //   * the left and right neighbours come from the lanes beside it by DPP, the
 //     other y and z neighbours through LDS, the restriction's second row from
 //     lane + 32 (a wave holds two rows of 32 pairs);
-//   * two barriers per launch, one for each colour (three with 16-bit records,
-//     whose diagonal is formed from all six couplings).
+//   * two barriers per launch, one for each colour.
 // In FP32: 64^3 down 10.0 -> 6.5 us, up 10.5 -> 8.9 (beside the x update),
 // 24 x 20 x 18 down 4.9 -> 4.0, up 4.0 (a launch with nothing in it takes 2.2).
 #pragma once
@@ -99,11 +98,8 @@ __device__ __forceinline__ void t3_load(const VB* __restrict__ b, const C4* __re
     }
 }
 
-// The couplings that other threads hold, through LDS.  16-bit records: the
-// cells at the region's lower borders, whose -x / -y / -z neighbours lie
-// outside it, read those couplings from memory, and the diagonals are formed
-// (snap_diag) as everywhere else.
-template <typename C4, typename CT>
+// The couplings that other threads hold, through LDS.
+template <typename CT>
 __device__ __forceinline__ void t3_couplings_put(T3LDS<CT>& S, const T3Pos& t, const T3St<CT> (&s)[2][2]) {
 #pragma unroll
     for (int q = 0; q < 2; q++) {
@@ -112,29 +108,14 @@ __device__ __forceinline__ void t3_couplings_put(T3LDS<CT>& S, const T3Pos& t, c
         S.cz[q][t.ec] = s[1][q].zp;
     }
 }
-template <typename C4, typename CT>
-__device__ __forceinline__ void t3_couplings_get(const T3LDS<CT>& S, const T3Pos& t, T3St<CT> (&s)[2][2], const C4* __restrict__ rec, const Geo& g) {
-    constexpr bool XD = std::is_same<C4, BF16x4>::value;
+template <typename CT>
+__device__ __forceinline__ void t3_couplings_get(const T3LDS<CT>& S, const T3Pos& t, T3St<CT> (&s)[2][2]) {
 #pragma unroll
     for (int q = 0; q < 2; q++) {
         s[0][q].ym = t.rj >= 1 ? S.cy[q][t.e - 32] : CT(0);
         s[1][q].ym = t.rj >= 1 ? S.cy[q][t.e + 256 - 32] : CT(0);
         s[0][q].zm = t.rk >= 1 ? S.cz[q][t.ec - 256] : CT(0);
         s[1][q].zm = s[0][q].zp;
-    }
-    if constexpr (XD) {
-#pragma unroll
-        for (int v = 0; v < 2; v++) {
-            if (t.hx == 0 && t.in0[v]) s[v][0].xm = (CT)rec[t.id[v] - 1].x;
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                if (!(q ? t.in1[v] : t.in0[v])) continue;
-                if (t.rj == 0) s[v][q].ym = (CT)rec[t.id[v] + q - g.sx].y;
-                if (t.rk == 0 && v == 0) s[v][q].zm = (CT)rec[t.id[v] + q - g.sy].z;
-                T3St<CT>& c = s[v][q];
-                if (c.d >= CT(0)) c.d = snap_diag<C4, CT>(c.d, c.xp + c.xm + c.yp + c.ym + c.zp + c.zm);
-            }
-        }
     }
 }
 
@@ -191,7 +172,6 @@ template <typename VB, typename C4>
 __device__ __forceinline__ void d_t3_down(const VB* __restrict__ b, const C4* __restrict__ rec, const Geo& g, VB* __restrict__ bc, const Geo& cg,
                                           int tile, const int* skip) {
     using CT = typename CTOf<VB>::type;
-    constexpr bool XD = std::is_same<C4, BF16x4>::value;
     __shared__ T3LDS<CT> S;
     const int stop = skip ? *skip : 0;
     T3Pos t;
@@ -202,14 +182,10 @@ __device__ __forceinline__ void d_t3_down(const VB* __restrict__ b, const C4* __
     if (stop) return;
 #pragma unroll
     for (int v = 0; v < 2; v++) { s[v][0].xm = t3_left(t, s[v][1].xp); s[v][1].xm = s[v][0].xp; }
-    t3_couplings_put<C4, CT>(S, t, s);
-    if constexpr (XD) {
-        __syncthreads();
-        t3_couplings_get<C4, CT>(S, t, s, rec, g);
-    }
+    t3_couplings_put<CT>(S, t, s);
     t3_first<false, CT>(S, t, x, bv, s, CT(0));
     __syncthreads();
-    if constexpr (!XD) t3_couplings_get<C4, CT>(S, t, s, rec, g);
+    t3_couplings_get<CT>(S, t, s);
     // A neighbour has the other colour, so every value that the even cells
     // read was written before the barrier, and every one that they write is
     // read after the next.
@@ -251,7 +227,6 @@ template <typename VB, typename C4>
 __device__ __forceinline__ void d_t3_up(const VB* __restrict__ b, const C4* __restrict__ rec, const Geo& g, const VB* __restrict__ xc, const Geo& cg,
                                         VB* __restrict__ xout, int tile, const int* skip) {
     using CT = typename CTOf<VB>::type;
-    constexpr bool XD = std::is_same<C4, BF16x4>::value;
     __shared__ T3LDS<CT> S;
     const int stop = skip ? *skip : 0;
     T3Pos t;
@@ -266,14 +241,10 @@ __device__ __forceinline__ void d_t3_up(const VB* __restrict__ b, const C4* __re
     if (stop) return;
 #pragma unroll
     for (int v = 0; v < 2; v++) { s[v][0].xm = t3_left(t, s[v][1].xp); s[v][1].xm = s[v][0].xp; }
-    t3_couplings_put<C4, CT>(S, t, s);
-    if constexpr (XD) {
-        __syncthreads();
-        t3_couplings_get<C4, CT>(S, t, s, rec, g);
-    }
+    t3_couplings_put<CT>(S, t, s);
     t3_first<true, CT>(S, t, x, bv, s, c);
     __syncthreads();
-    if constexpr (!XD) t3_couplings_get<C4, CT>(S, t, s, rec, g);
+    t3_couplings_get<CT>(S, t, s);
     t3_sweep<true, CT>(S, t, true, x, bv, s);      // even cells
     t3_put_even<CT>(S, t, x);
     __syncthreads();
