@@ -305,8 +305,8 @@ int uaamg_batch_solve(uaamg_batch* b, const double* const* rhs_dev, double* cons
  * resident while the HBM budget allows (least recently used idle simulations
  * are evicted), runs the active requests in batches and admits new requests
  * between chunks of iterations (continuous batching).  Simulations fall into
- * four size classes (2D / 3D, fewer / at least 2^18 padded cells), each
- * batched on a stream of its own, so small requests complete at the pace of
+ * three classes (fewer than 2^18 padded cells, larger 2D, larger 3D), each on
+ * a stream of its own, so small requests complete at the pace of
  * their own chunks, not of the largest grid's.  With warm_start = 1 the
  * request's p_dev holds the previous frame's pressure and receives the new
  * one.  precision: UAAMG_FP32 or UAAMG_MIXED_BF16. */

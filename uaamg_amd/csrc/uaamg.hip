@@ -847,12 +847,17 @@ struct Request {
 };
 }  // namespace
 
-// batch part of a simulation: 2D small, 2D large, 3D small, 3D large; the
-// size class (small 0, large 1) is the part's low bit
+// batch part of a simulation: 2D small, 2D large, 3D small, 3D large
 constexpr int kServeParts = 4;
 constexpr long kServeLarge = 1L << 18;   // padded cells from which a grid is large
 static int serve_part_of(int dim, long cells) { return (dim == 3 ? 2 : 0) + (cells >= kServeLarge ? 1 : 0); }
-static int serve_class_of(int part) { return part & 1; }
+// Classes: small grids of both dimensions, large 2D, large 3D.  A class has a
+// stream of its own; three and the caller's are the process's four hardware
+// queues (with a stream per part two parts shared a queue and ran in lockstep;
+// with one class for all large grids a 768 x 768 frame waited for each chunk
+// of a 128^3 one: 16 simulations, one frame each, 17.6 ms, now 14.8).
+constexpr int kServeClasses = 3;
+static int serve_class_of(int part) { return part == 1 ? 1 : (part == 3 ? 2 : 0); }
 
 struct uaamg_server {
     uaamg_opts o{};
@@ -863,9 +868,9 @@ struct uaamg_server {
     // inflight: a chunk of the class was launched and its event has not been
     // seen complete
     std::unique_ptr<uaamg::BatchBase> part[kServeParts];
-    hipStream_t cstream[2] = {};
-    hipEvent_t cev[2] = {};
-    bool inflight[2] = {};
+    hipStream_t cstream[kServeClasses] = {};
+    hipEvent_t cev[kServeClasses] = {};
+    bool inflight[kServeClasses] = {};
     std::vector<int> slot_sim[kServeParts];
     std::unordered_map<int, SimState> sims;
     std::vector<Request> reqs;
@@ -910,7 +915,7 @@ extern "C" int uaamg_server_create(uaamg_server** out, const uaamg_opts* o, size
     s->max_active = max_active;
     // the class streams are created together (default priority), so that
     // they land on different hardware queues
-    for (int c = 0; c < 2; c++)
+    for (int c = 0; c < kServeClasses; c++)
         if (hipStreamCreateWithFlags(&s->cstream[c], hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&s->cev[c], hipEventDisableTiming) != hipSuccess) {
             uaamg_server_destroy(s);
@@ -922,11 +927,11 @@ extern "C" int uaamg_server_create(uaamg_server** out, const uaamg_opts* o, size
 
 extern "C" void uaamg_server_destroy(uaamg_server* s) {
     if (!s) return;
-    for (int c = 0; c < 2; c++)
+    for (int c = 0; c < kServeClasses; c++)
         if (s->cstream[c]) (void)hipStreamSynchronize(s->cstream[c]);
     for (int pi = 0; pi < kServeParts; pi++) s->part[pi].reset();
     if (s->stage) (void)hipFree(s->stage);
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < kServeClasses; c++) {
         if (s->cev[c]) (void)hipEventDestroy(s->cev[c]);
         if (s->cstream[c]) (void)hipStreamDestroy(s->cstream[c]);
     }
@@ -1010,7 +1015,7 @@ static bool server_collect(uaamg_server* s, bool wait, std::vector<int>& fin) {
     bool any = false;
     for (;;) {
         bool inflight = false;
-        for (int cl = 0; cl < 2; cl++) {
+        for (int cl = 0; cl < kServeClasses; cl++) {
             if (!s->inflight[cl]) continue;
             inflight = true;
             const hipError_t q = hipEventQuery(s->cev[cl]);
@@ -1100,11 +1105,11 @@ static void server_admit_and_launch(uaamg_server* s) {
     }
     bool run[kServeParts] = {};
     for (int id : s->active) run[s->sims[s->reqs[id].sim].part] = true;
-    for (int cl = 0; cl < 2; cl++) {
+    for (int cl = 0; cl < kServeClasses; cl++) {
         if (s->inflight[cl]) continue;
         bool any = false;
-        for (int pi = cl; pi < kServeParts; pi += 2)
-            if (run[pi]) { s->part[pi]->run_chunk(); any = true; }
+        for (int pi = 0; pi < kServeParts; pi++)
+            if (serve_class_of(pi) == cl && run[pi]) { s->part[pi]->run_chunk(); any = true; }
         if (!any) continue;
         HIPCHK(hipEventRecord(s->cev[cl], s->cstream[cl]));
         s->inflight[cl] = true;
