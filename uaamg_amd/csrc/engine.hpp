@@ -562,10 +562,12 @@ public:
             const Level& L = lv_[tail_first_ + q];
             targs_.g[q] = L.g;
             targs_.coef[q] = L.coef;
+            targs_.np[q] = ((L.g.nx + 1) / 2) * L.g.ny * (D == 3 ? L.g.nz : 1);
             targs_.xo[q] = off; off += (int)L.g.N;
             targs_.bo[q] = off; off += (int)L.g.N;
         }
         targs_.ro = off;
+        targs_.N0 = (int)targs_.g[0].N;
         targs_.npass = (o_.coarsest_sweeps > 0) ? 2 * o_.coarsest_sweeps + 1 : 0;
         targs_.b = lv_[tail_first_].b;
         targs_.x = lv_[tail_first_].x;

@@ -407,12 +407,14 @@ struct FinState { int done, tol_mode, iter, max_iter; double tol, tolsq; double*
 __device__ __forceinline__ FinState fin_state(const Ctrl* c) {
     return FinState{c->done, c->tol_mode, c->iter, c->max_iter, c->tol, c->tolsq, c->hist};
 }
-// r.r of this iteration: history, convergence, iteration cap; whether the solve stops
+// r.r of this iteration: history, convergence, iteration cap; whether the solve
+// stops (ctrl == nullptr: the decision alone)
 __device__ __forceinline__ int fin_update_scalars(Ctrl* ctrl, const FinState& f, double rs) {
     if (f.done) return 1;
     const bool conv = (f.tol_mode == 1) ? (rs < f.tolsq) : (sqrt(rs) < f.tol);
     const int iter = f.iter + 1;
     const int status = conv ? ST_CONVERGED : (!isfinite(rs) ? ST_NONFINITE : (iter >= f.max_iter ? ST_MAXITER : ST_RUNNING));
+    if (!ctrl) return status != ST_RUNNING;
     ctrl->rsnew = rs;
     if (f.hist) f.hist[f.iter] = rs;
     ctrl->iter = iter;

@@ -15,6 +15,25 @@
 //
 // A thread owns pairs of x-adjacent cells (i odd, i+1): one cell of each
 // colour, so every RBGS pass keeps all lanes busy.
+//
+// One workgroup on one CU: the chain of dependent steps is what counts.
+//   * Everything a pair needs is built at set-up (k_tail_records): couplings,
+//     diagonal and 1 / diagonal by colour, and the pair's LDS index, its
+//     parent's and its first child's (integer divisions by the level's sides
+//     cost as much as the memory round trip).  Only existing pairs are loaded.
+//   * The kernel arguments that the loads depend on come first in the block,
+//     so one round trip of scalar loads starts all of them.
+//   * x = 0 before the first pass of a level, so that pass is b / d of the
+//     thread's own cell, in the step that restricts b: three barriers a level
+//     down, three up.
+//   * Levels of at most 64 pairs run in wave 0 alone, without barriers.
+//   * The convergence test costs no barrier of its own.
+// Measured against the form before (records of all 1024 threads loaded,
+// indices by division, four barriers a level, division in the chain): 16^3 to
+// 4^3 FP32 19.6 -> 15.9 us, 18 x 12 x 7 FP32
+// 13.4 -> 9.0, 16 x 8 x 8 FP64 24.0 -> 13.9, 2D 32 x 16 FP64 15.2 -> 13.8, 12 2D
+// grids of up to 5 levels 20.7 -> 16.3.  What is left is the 21 coarsest passes
+// (a chain of LDS reads and additions) and one memory round trip.
 #pragma once
 #include "kernels_cg.hpp"
 
@@ -24,153 +43,92 @@ constexpr int TAIL_THREADS = 1024;
 constexpr int TAIL_MAXL = 5;      // tail levels (3D: 16^3..4^3 is 3; 2D: 64^2..4^2 is 5)
 constexpr int TAIL_MAXP = 2;      // pairs per thread on the first tail level
 constexpr int TAIL_LDS_BYTES = 96 * 1024;   // x, b of every tail level + one residual array
-constexpr int TAIL_BMAX = 8;     // b elements per thread of the first tail level (padded cells <= 8192)
-constexpr int TAIL_NSLOT = TAIL_MAXP + TAIL_MAXL - 1;   // record slots: TAIL_MAXP on the first level, 1 below
+constexpr int TAIL_BMAX = 8;     // b elements per thread of the first tail level (padded cells <= 8192; FP64: 4, by the LDS)
 
-// Stencil records of the owned pairs, built at set-up in the compute type:
-// 14 values per pair (d, xp, xm, yp, ym, zp, zm of both cells), NQ 16-byte
-// quads per thread, stored [slot][quad][thread] so that every quad load of a
-// wave is one contiguous 1 KiB read.
+// A pair's record: 16 values (d, 1/d, xp, xm, yp, ym, zp, zm, each of the even
+// and the odd cell; 1/d = 0 where no pass updates the cell) and 4 indices, in
+// 16-byte quads stored [slot][quad][thread], so that every quad load of a
+// wave is one contiguous 1 KiB read.  Slots: TAIL_MAXP on the first level, 1
+// on every other.
 template <typename CT> struct TailRec;
-template <> struct TailRec<float> { static constexpr int NQ = 4; using Q = float4; };
-template <> struct TailRec<double> { static constexpr int NQ = 7; using Q = double2; };
-template <typename CT> constexpr int tail_rec_per_q() { return 16 / (int)sizeof(CT); }
+template <> struct TailRec<float> { static constexpr int NV = 4, NQ = 5, PER = 4; using Q = float4; };
+template <> struct TailRec<double> { static constexpr int NV = 8, NQ = 9, PER = 2; using Q = double2; };
 template <typename CT> constexpr long tail_rec_bytes(int nslots) { return (long)nslots * TailRec<CT>::NQ * TAIL_THREADS * 16; }
 __host__ __device__ constexpr int tail_slot(int l, int v) { return l == 0 ? v : TAIL_MAXP + l - 1; }
 
 template <typename C4>
 struct TailArgs {
-    int nl;                        // levels in the tail; the last one is the coarsest
-    Geo g[TAIL_MAXL];
-    const C4* coef[TAIL_MAXL];
-    int xo[TAIL_MAXL], bo[TAIL_MAXL];   // LDS offsets (elements) of x and b per level
-    int ro;                        // LDS offset of the residual scratch
-    int npass;                     // coarsest passes (2 * sweeps + 1)
+    // what the first loads depend on
+    const void* rec;               // pair records (compute type)
     const void* b;                 // b of the first tail level (level storage type)
     void* x;                       // x of the first tail level (written at the end)
     const int* skip;               // stop flag (nullptr: never skip)
-    const void* rec;               // pair records (compute type), TAIL_NSLOT slots at most
     // the convergence test of this iteration (k_fin_update), run before the
     // levels: r.r partials (k_tail: nullptr: no test here) and the scalars
     const double* rr;
-    int nrr;
     Ctrl* ctrl;
+    int nrr;
+    int nl;                        // levels in the tail; the last one is the coarsest
+    int ro;                        // LDS offset of the residual scratch (behind x and b of every level)
+    int N0;                        // padded cells of the first one
+    int np[TAIL_MAXL];             // pairs per level
+    int npass;                     // coarsest passes (2 * sweeps + 1)
+    int xo[TAIL_MAXL], bo[TAIL_MAXL];   // LDS offsets (elements) of x and b per level
+    Geo g[TAIL_MAXL];
+    const C4* coef[TAIL_MAXL];     // set-up
 };
 
-// Stencils of one owned pair of cells, in the reference channel order.
+// One owned pair: [0] the even cell, [1] the odd one.
 template <typename CT>
 struct TailPair {
-    CT d[2], xp[2], xm[2], yp[2], ym[2], zp[2], zm[2];
-    int id0;          // padded index of the first cell
-    int i0, j, k;
-    int par0;         // colour of the first cell
-    bool valid, ok1;  // pair exists; second cell inside the level
+    CT d[2], inv[2], xp[2], xm[2], yp[2], ym[2], zp[2], zm[2];
+    int id[2];        // padded indices (a second cell outside the level: d < 0)
+    int pid;          // padded index of the parent on the next level, -1: none
+    int ch;           // padded index of the first cell's first child on the level above
+    bool valid, ok1, first_odd;   // pair exists; its second cell is inside the level; colour of its first cell
 };
 
-// Record element type of a coefficient vector type.
-template <typename C4> struct TailE { using E = float; };
-template <> struct TailE<double4> { using E = double; };
-template <> struct TailE<BF16x4> { using E = __bf16; };
-
-// The record loads of one pair as they come from memory.  Every pair of
-// every tail level issues its loads before any of them is used, so that the
-// start of the kernel waits for one memory round trip instead of one per
-// pair; an absent pair reads the first interior cell (in bounds, discarded)
-// and the second cell of a pair at i = nx reads the ghost at nx + 1 (inside
-// the padded level, discarded).
-template <typename C4>
-struct TailRaw {
-    C4 c[2];
-    typename TailE<C4>::E xm[2], ym[2], zm[2];
-};
-
-template <int D, typename C4>
-__device__ __forceinline__ void tail_issue_pair(TailRaw<C4>& R, const C4* __restrict__ coef, const Geo& g, int p) {
-    const int npx = (g.nx + 1) >> 1;
-    const int npairs = npx * g.ny * (D == 3 ? g.nz : 1);
-    const int pp = p < npairs ? p : 0;
-    const int ip = pp % npx;
-    const int j = (pp / npx) % g.ny + 1, k = (D == 3) ? pp / (npx * g.ny) + 1 : 0;
-    const int id0 = (int)gidx(g, 2 * ip + 1, j, k);
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-        const int id = id0 + q;
-        using E = typename TailE<C4>::E;
-        const E* e = reinterpret_cast<const E*>(coef);   // {x, y, z, w} per record
-        R.c[q] = gload(coef + id);
-        R.xm[q] = gload(e + 4 * (id - 1));
-        R.ym[q] = gload(e + 4 * (id - g.sx) + 1);
-        if (D == 3) R.zm[q] = gload(e + 4 * (id - g.sy) + 2);
-    }
-}
-
-// The stencils of pair p from its loaded records, as sten_lc forms them.
-template <int D, typename CT, typename C4>
-__device__ __forceinline__ void tail_load_pair(TailPair<CT>& P, const TailRaw<C4>& R, const Geo& g, int p) {
-    const int npx = (g.nx + 1) >> 1;
-    const int npairs = npx * g.ny * (D == 3 ? g.nz : 1);
-    P.valid = p < npairs;
-    if (!P.valid) { P.id0 = 0; P.ok1 = false; P.par0 = 0; P.i0 = P.j = P.k = 0; return; }
-    const int ip = p % npx;
-    P.i0 = 2 * ip + 1;
-    P.j = (p / npx) % g.ny + 1;
-    P.k = (D == 3) ? p / (npx * g.ny) + 1 : 0;
-    P.ok1 = P.i0 + 1 <= g.nx;
-    P.par0 = (P.i0 + P.j + P.k) & 1;
-    P.id0 = (int)gidx(g, P.i0, P.j, P.k);
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-        if (q == 1 && !P.ok1) {
-            P.d[q] = CT(-1); P.xp[q] = P.xm[q] = P.yp[q] = P.ym[q] = P.zp[q] = P.zm[q] = CT(0);
-            continue;
-        }
-        const C4 c0 = R.c[q];
-        CT d = (CT)c0.w;
-        P.xp[q] = (CT)c0.x; P.yp[q] = (CT)c0.y;
-        P.xm[q] = (CT)R.xm[q]; P.ym[q] = (CT)R.ym[q];
-        if (D == 3) { P.zp[q] = (CT)c0.z; P.zm[q] = (CT)R.zm[q]; }
-        else { P.zp[q] = CT(0); P.zm[q] = CT(0); }
-        if (d >= CT(0)) d = snap_diag<C4, CT>(d, P.xp[q] + P.xm[q] + P.yp[q] + P.ym[q] + P.zp[q] + P.zm[q]);
-        P.d[q] = d;
-    }
-}
-
-// The 14 record values of one pair, as loaded.
-template <typename CT>
-struct TailRecV { CT v[TailRec<CT>::NQ * tail_rec_per_q<CT>()]; };
-
-template <typename CT>
-__device__ __forceinline__ void tail_issue_rec(TailRecV<CT>& R, const void* rec, int slot, int t) {
-    using Q = typename TailRec<CT>::Q;
-    constexpr int NQ = TailRec<CT>::NQ;
-    const Q* base = static_cast<const Q*>(rec) + (long)slot * NQ * TAIL_THREADS + t;
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        const Q x = gload(base + q * TAIL_THREADS);
-        if constexpr (sizeof(CT) == 4) { R.v[4 * q] = x.x; R.v[4 * q + 1] = x.y; R.v[4 * q + 2] = x.z; R.v[4 * q + 3] = x.w; }
-        else { R.v[2 * q] = x.x; R.v[2 * q + 1] = x.y; }
-    }
-}
-
-// Geometry of pair p (computed) and its stencils (from the record).
+// Record loads of a pair (undefined where the pair does not exist).
 template <int D, typename CT>
-__device__ __forceinline__ void tail_pair_from_rec(TailPair<CT>& P, const TailRecV<CT>& R, const Geo& g, int p) {
-    const int npx = (g.nx + 1) >> 1;
-    const int npairs = npx * g.ny * (D == 3 ? g.nz : 1);
-    P.valid = p < npairs;
-    const int pp = P.valid ? p : 0;
-    const int ip = pp % npx;
-    P.i0 = 2 * ip + 1;
-    P.j = (pp / npx) % g.ny + 1;
-    P.k = (D == 3) ? pp / (npx * g.ny) + 1 : 0;
-    P.ok1 = P.valid && P.i0 + 1 <= g.nx;
-    P.par0 = (P.i0 + P.j + P.k) & 1;
-    P.id0 = (int)gidx(g, P.i0, P.j, P.k);
+struct TailRecV {
+    typename TailRec<CT>::Q v[TailRec<CT>::NV];
+    int4 ix;
+};
+template <int D, typename CT>
+__device__ __forceinline__ void tail_issue_rec(TailRecV<D, CT>& R, const void* rec, int slot, int p, int np, int t) {
+    using Q = typename TailRec<CT>::Q;
+    constexpr int NQ = TailRec<CT>::NQ, NV = TailRec<CT>::NV;
+    const Q* base = static_cast<const Q*>(rec) + (long)slot * NQ * TAIL_THREADS + t;
+    R.ix = int4{0, -1, 0, 0};
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
-        P.d[q] = R.v[q]; P.xp[q] = R.v[2 + q]; P.xm[q] = R.v[4 + q]; P.yp[q] = R.v[6 + q];
-        P.ym[q] = R.v[8 + q]; P.zp[q] = R.v[10 + q]; P.zm[q] = R.v[12 + q];
+    for (int q = 0; q < NV; q++) R.v[q] = Q{};
+    if (p < np) {
+#pragma unroll
+        for (int q = 0; q < (D == 3 ? NV : NV * 3 / 4); q++) R.v[q] = gload(base + q * TAIL_THREADS);   // 2D: no z couplings
+        R.ix = __builtin_bit_cast(int4, gload(base + NV * TAIL_THREADS));
     }
+}
+template <int D, typename CT>
+__device__ __forceinline__ void tail_pair_from_rec(TailPair<CT>& P, const TailRecV<D, CT>& R, int p, int np) {
+    constexpr int PER = TailRec<CT>::PER;
+    auto val = [&](int e) -> CT {
+        const auto& q = R.v[e / PER];
+        if constexpr (sizeof(CT) == 4) return (e & 3) == 0 ? q.x : ((e & 3) == 1 ? q.y : ((e & 3) == 2 ? q.z : q.w));
+        else return (e & 1) ? q.y : q.x;
+    };
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        P.d[c] = val(c); P.inv[c] = val(2 + c);
+        P.xp[c] = val(4 + c); P.xm[c] = val(6 + c); P.yp[c] = val(8 + c); P.ym[c] = val(10 + c);
+        P.zp[c] = val(12 + c); P.zm[c] = val(14 + c);
+    }
+    P.valid = p < np;
+    P.first_odd = (R.ix.w & 1) != 0;
+    P.ok1 = (R.ix.w & 2) != 0;
+    P.id[0] = R.ix.x + (P.first_odd ? 1 : 0);
+    P.id[1] = R.ix.x + (P.first_odd ? 0 : 1);
+    P.pid = R.ix.y;
+    P.ch = R.ix.z;
 }
 
 // Set-up: the records of every slot of the tail (one workgroup per slot).
@@ -181,76 +139,74 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail_records(TailArgs<C4> A, C
     const int v = slot < TAIL_MAXP ? slot : 0;
     if (l >= A.nl) return;
     const int t = threadIdx.x, p = t + TAIL_THREADS * v;
-    TailRaw<C4> R;
-    tail_issue_pair<D, C4>(R, A.coef[l], A.g[l], p);
-    TailPair<CT> P;
-    tail_load_pair<D, CT, C4>(P, R, A.g[l], p);
-    constexpr int PER = tail_rec_per_q<CT>(), NQ = TailRec<CT>::NQ;
-    CT f[NQ * PER];
+    const Geo g = A.g[l];
+    if (p >= A.np[l]) return;
+    const int npx = (g.nx + 1) >> 1;
+    const int i0 = 2 * (p % npx) + 1, j = (p / npx) % g.ny + 1, k = (D == 3) ? p / (npx * g.ny) + 1 : 0;
+    const int id0 = (int)gidx(g, i0, j, k), par0 = (i0 + j + k) & 1;
+    const bool ok1 = i0 + 1 <= g.nx;
+    constexpr int PER = TailRec<CT>::PER, NQ = TailRec<CT>::NQ, NV = TailRec<CT>::NV;
+    CT f[NV * PER];
 #pragma unroll
-    for (int e = 0; e < NQ * PER; e++) f[e] = CT(0);
-    if (P.valid) {
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            f[q] = P.d[q]; f[2 + q] = P.xp[q]; f[4 + q] = P.xm[q]; f[6 + q] = P.yp[q];
-            f[8 + q] = P.ym[q]; f[10 + q] = P.zp[q]; f[12 + q] = P.zm[q];
-        }
+    for (int c = 0; c < 2; c++) {   // cell of colour c
+        const int q = c ^ par0;
+        Sten<CT> s;
+        s.d = CT(-1); s.xp = s.xm = s.yp = s.ym = s.zp = s.zm = CT(0);
+        if (q == 0 || ok1) s = sten_lc<D, CT>(A.coef[l], g, id0 + q);
+        f[c] = s.d;
+        f[2 + c] = s.d >= CT(1e-30) ? recip(s.d) : CT(0);
+        f[4 + c] = s.xp; f[6 + c] = s.xm; f[8 + c] = s.yp; f[10 + c] = s.ym;
+        f[12 + c] = D == 3 ? s.zp : CT(0); f[14 + c] = D == 3 ? s.zm : CT(0);
     }
+    const long at = (long)slot * NQ * TAIL_THREADS + t;
 #pragma unroll
-    for (int q = 0; q < NQ; q++)
+    for (int q = 0; q < NV; q++)
 #pragma unroll
-        for (int e = 0; e < PER; e++) rec[(((long)slot * NQ + q) * TAIL_THREADS + t) * PER + e] = f[q * PER + e];
-}
-
-// (b + nb) / d: exact division in FP64 (the parity path); in FP32 the
-// hardware reciprocal, as in the march kernels of the same levels, which
-// shortens the dependent chain of every pass
-template <typename CT>
-__device__ __forceinline__ CT tdiv(CT num, CT d) {
-    if constexpr (std::is_same<CT, double>::value) return num / d;
-    else return num * __builtin_amdgcn_rcpf(d);
+        for (int e = 0; e < PER; e++) rec[(at + (long)q * TAIL_THREADS) * PER + e] = f[q * PER + e];
+    int4 ix;
+    ix.x = id0;
+    ix.y = -1;
+    if (l + 1 < A.nl) {
+        const Geo cg = A.g[l + 1];
+        const int ic = (i0 + 1) >> 1, jc = (j + 1) >> 1, kc = (D == 3) ? (k + 1) >> 1 : 0;
+        if (ic <= cg.nx && jc <= cg.ny && (D != 3 || kc <= cg.nz)) ix.y = (int)gidx(cg, ic, jc, kc);
+    }
+    ix.z = l > 0 ? (int)gidx(A.g[l - 1], 2 * i0 - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0) : 0;
+    ix.w = par0 | (ok1 ? 2 : 0);
+    reinterpret_cast<int4*>(rec)[at + (long)NV * TAIL_THREADS] = ix;
 }
 
 // One RBGS colour on the owned pairs of one level.
-template <int D, typename CT, int NP>
-__device__ __forceinline__ void tail_smooth(const TailPair<CT> (&P)[NP], CT* X, const CT* Bv, const Geo& g, int colour) {
+template <int D, int C, typename CT, int NP>
+__device__ __forceinline__ void tail_smooth(const TailPair<CT> (&P)[NP], CT* X, const CT* Bv, int sx, int sy) {
 #pragma unroll
     for (int v = 0; v < NP; v++) {
         const TailPair<CT>& p = P[v];
-        if (!p.valid) continue;
-        const int q = (p.par0 == colour) ? 0 : 1;
-        if (q == 1 && !p.ok1) continue;
-        const CT d = q ? p.d[1] : p.d[0];
-        if (!(d >= CT(1e-30))) continue;           // solid (d < 0) or isolated
-        const int id = p.id0 + q;
-        const CT xp = q ? p.xp[1] : p.xp[0], xm = q ? p.xm[1] : p.xm[0];
-        const CT yp = q ? p.yp[1] : p.yp[0], ym = q ? p.ym[1] : p.ym[0];
-        CT nb = xp * X[id + 1] + xm * X[id - 1] + yp * X[id + g.sx] + ym * X[id - g.sx];
-        if (D == 3) {
-            const CT zp = q ? p.zp[1] : p.zp[0], zm = q ? p.zm[1] : p.zm[0];
-            nb = nb + zp * X[id + g.sy] + zm * X[id - g.sy];
-        }
-        X[id] = tdiv<CT>(Bv[id] + nb, d);
+        if (p.inv[C] == CT(0)) continue;           // absent, solid or isolated
+        const int id = p.id[C];
+        CT nb = p.xp[C] * X[id + 1] + p.xm[C] * X[id - 1] + p.yp[C] * X[id + sx] + p.ym[C] * X[id - sx];
+        if (D == 3) nb = nb + p.zp[C] * X[id + sy] + p.zm[C] * X[id - sy];
+        X[id] = rdiv(Bv[id] + nb, p.d[C], p.inv[C]);
     }
 }
 
 // b - A x on the owned fluid cells (0 elsewhere), formed as k_restrict forms it.
 template <int D, typename CT, int NP>
-__device__ __forceinline__ void tail_residual(const TailPair<CT> (&P)[NP], const CT* X, const CT* Bv, CT* Rs, const Geo& g) {
+__device__ __forceinline__ void tail_residual(const TailPair<CT> (&P)[NP], const CT* X, const CT* Bv, CT* Rs, int sx, int sy) {
 #pragma unroll
     for (int v = 0; v < NP; v++) {
         const TailPair<CT>& p = P[v];
         if (!p.valid) continue;
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            if (q == 1 && !p.ok1) continue;
-            const int id = p.id0 + q;
+        for (int c = 0; c < 2; c++) {
+            if (!p.ok1 && (p.first_odd ? c == 0 : c == 1)) continue;   // the second cell, outside the level
+            const int id = p.id[c];
             CT res = CT(0);
-            if (p.d[q] >= CT(0)) {
-                double Ax = (double)p.d[q] * (double)X[id] - (double)p.xp[q] * (double)X[id + 1]
-                          - (double)p.xm[q] * (double)X[id - 1] - (double)p.yp[q] * (double)X[id + g.sx]
-                          - (double)p.ym[q] * (double)X[id - g.sx];
-                if (D == 3) Ax = Ax - (double)p.zp[q] * (double)X[id + g.sy] - (double)p.zm[q] * (double)X[id - g.sy];
+            if (p.d[c] >= CT(0)) {
+                double Ax = (double)p.d[c] * (double)X[id] - (double)p.xp[c] * (double)X[id + 1]
+                          - (double)p.xm[c] * (double)X[id - 1] - (double)p.yp[c] * (double)X[id + sx]
+                          - (double)p.ym[c] * (double)X[id - sx];
+                if (D == 3) Ax = Ax - (double)p.zp[c] * (double)X[id + sy] - (double)p.zm[c] * (double)X[id - sy];
                 res = (CT)((double)Bv[id] - Ax);
             }
             Rs[id] = res;
@@ -259,42 +215,46 @@ __device__ __forceinline__ void tail_residual(const TailPair<CT> (&P)[NP], const
 }
 
 // x_f += 2 x_c on the owned fluid cells whose parent lies in the coarse level.
-template <int D, typename CT, int NP>
-__device__ __forceinline__ void tail_prolong(const TailPair<CT> (&P)[NP], CT* X, const CT* XC, const Geo& g, const Geo& cg) {
+template <typename CT, int NP>
+__device__ __forceinline__ void tail_prolong(const TailPair<CT> (&P)[NP], CT* X, const CT* XC) {
 #pragma unroll
     for (int v = 0; v < NP; v++) {
         const TailPair<CT>& p = P[v];
-        if (!p.valid) continue;
-        const int jc = (p.j + 1) >> 1, kc = (D == 3) ? (p.k + 1) >> 1 : 0;
-        const int ic = (p.i0 + 1) >> 1;              // both cells of the pair share the parent
-        if (ic > cg.nx || jc > cg.ny || (D == 3 && kc > cg.nz)) continue;
-        const CT xc = XC[gidx(cg, ic, jc, kc)];
+        if (p.pid < 0) continue;
+        const CT xc = XC[p.pid];
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            if (q == 1 && !p.ok1) continue;
-            if (!(p.d[q] >= CT(0))) continue;
-            X[p.id0 + q] = X[p.id0 + q] + CT(2) * xc;
-        }
+        for (int c = 0; c < 2; c++)
+            if (p.valid && p.d[c] >= CT(0)) X[p.id[c]] = X[p.id[c]] + CT(2) * xc;
     }
-    (void)g;
 }
 
-// b_c = sum of the children's residuals; x_c = 0 (every coarse interior cell).
+// b / d on the odd cells (the first pass of a level, whose x is 0)
+template <typename CT>
+__device__ __forceinline__ void tail_first(const TailPair<CT>& p, CT* X, CT b) {
+    if (p.inv[1] != CT(0)) X[p.id[1]] = rdiv(b + CT(0), p.d[1], p.inv[1]);
+}
+
+// b of the owned pair = sum of the children's residuals (all its cells in the
+// level), then the first pass (unless no pass is asked for on the coarsest).
 template <int D, typename CT>
-__device__ __forceinline__ void tail_restrict(const CT* Rs, CT* BC, CT* XC, const Geo& fg, const Geo& cg) {
-    const int n = cg.nx * cg.ny * (D == 3 ? cg.nz : 1);
-    for (int c = threadIdx.x; c < n; c += TAIL_THREADS) {
-        const int i = c % cg.nx + 1, j = (c / cg.nx) % cg.ny + 1, k = (D == 3) ? c / (cg.nx * cg.ny) + 1 : 0;
-        const int fi = 2 * i - 1, fj = 2 * j - 1, fk = (D == 3) ? 2 * k - 1 : 0;
+__device__ __forceinline__ void tail_restrict(const TailPair<CT>& p, const CT* Rs, CT* B, CT* X, int fsx, int fsy, bool first) {
+    if (!p.valid) return;
+    CT b[2];   // first and second cell
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
         double sum = 0;
-        for (int di = 0; di < 2; di++)
-            for (int dj = 0; dj < 2; dj++)
-                for (int dk = 0; dk < (D == 3 ? 2 : 1); dk++)
-                    sum += (double)Rs[gidx(fg, fi + di, fj + dj, fk + dk)];
-        const long cid = gidx(cg, i, j, k);
-        BC[cid] = (CT)sum;
-        XC[cid] = CT(0);
+        if (q == 0 || p.ok1) {
+            const CT* R = Rs + p.ch + 2 * q;
+            for (int di = 0; di < 2; di++)
+                for (int dj = 0; dj < 2; dj++)
+                    for (int dk = 0; dk < (D == 3 ? 2 : 1); dk++) sum += (double)R[di + dj * fsx + dk * fsy];
+        }
+        b[q] = (CT)sum;
     }
+    const int id0 = p.first_odd ? p.id[1] : p.id[0];
+    B[id0] = b[0];
+    if (p.ok1) B[id0 + 1] = b[1];
+    if (first) tail_first(p, X, p.first_odd ? b[0] : b[1]);
 }
 
 template <int D, typename S, typename C4, int NLMAX>
@@ -302,149 +262,153 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     static_assert(NLMAX >= 2 && NLMAX <= TAIL_MAXL, "tail depth");
     using CT = typename CTOf<S>::type;
     __shared__ __align__(16) CT lds[TAIL_LDS_BYTES / sizeof(CT)];
+    __shared__ TailArgs<C4> A;      // geometry and offsets (one vector load per dword)
+    __shared__ double s_rr[FIN_THREADS / WAVE];
     const int tid = threadIdx.x;
-    // The arguments sit in memory no cache has seen yet (a fresh kernel
-    // argument block, or the batch descriptor): scalar loads would fetch them
-    // line by line as the code first touches them, one memory round trip
-    // each.  One vector load per dword brings the block in one round trip.
-    // The skip flag is read beside the first data loads and tested before
-    // the first store to memory, not waited for up front.
-    __shared__ TailArgs<C4> A;
-    {
-        constexpr int NW = (int)(sizeof(TailArgs<C4>) / 4);
-        static_assert(NW <= TAIL_THREADS && sizeof(TailArgs<C4>) % 4 == 0, "tail arguments");
-        if (tid < NW) reinterpret_cast<uint32_t*>(&A)[tid] = reinterpret_cast<const uint32_t*>(&Ag)[tid];
-    }
-    __syncthreads();
-    const S* __restrict__ b_first = static_cast<const S*>(A.b);
-    S* __restrict__ x_first = static_cast<S*>(A.x);
-    const int nl = A.nl;   // 1 <= nl <= NLMAX (checked on the host); 1: the coarsest level only
+    const int nl = Ag.nl;   // 1 <= nl <= NLMAX (checked on the host); 1: the coarsest level only
+    const S* __restrict__ b_first = static_cast<const S*>(Ag.b);
+    S* __restrict__ x_first = static_cast<S*>(Ag.x);
+    int np[NLMAX];
+#pragma unroll
+    for (int l = 0; l < NLMAX; l++) np[l] = Ag.np[l];   // 0 past nl
 
     // every global load of the kernel's start first: the records of the
     // owned pairs (the first tail level has up to 2 pairs per thread, the
     // others 1) and b of the first level (at most TAIL_BMAX per thread,
     // checked on the host)
-    TailRecV<CT> R0[TAIL_MAXP], R1, R2, R3, R4;
+    TailRecV<D, CT> R0[TAIL_MAXP], R1, R2, R3, R4;
 #pragma unroll
-    for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<CT>(R0[v], A.rec, tail_slot(0, v), tid);
-    if (nl > 1) tail_issue_rec<CT>(R1, A.rec, tail_slot(1, 0), tid);
-    if constexpr (NLMAX > 2) { if (nl > 2) tail_issue_rec<CT>(R2, A.rec, tail_slot(2, 0), tid); }
-    if constexpr (NLMAX > 3) { if (nl > 3) tail_issue_rec<CT>(R3, A.rec, tail_slot(3, 0), tid); }
-    if constexpr (NLMAX > 4) { if (nl > 4) tail_issue_rec<CT>(R4, A.rec, tail_slot(4, 0), tid); }
-    S bt[TAIL_BMAX];
-    const int N0 = (int)A.g[0].N;
+    for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<D, CT>(R0[v], Ag.rec, tail_slot(0, v), tid + TAIL_THREADS * v, np[0], tid);
+    tail_issue_rec<D, CT>(R1, Ag.rec, tail_slot(1, 0), tid, np[1], tid);
+    if constexpr (NLMAX > 2) tail_issue_rec<D, CT>(R2, Ag.rec, tail_slot(2, 0), tid, np[2], tid);
+    if constexpr (NLMAX > 3) tail_issue_rec<D, CT>(R3, Ag.rec, tail_slot(3, 0), tid, np[3], tid);
+    if constexpr (NLMAX > 4) tail_issue_rec<D, CT>(R4, Ag.rec, tail_slot(4, 0), tid, np[4], tid);
+    constexpr int BMAX = sizeof(CT) == 8 ? TAIL_LDS_BYTES / 24 / TAIL_THREADS : TAIL_BMAX;
+    S bt[BMAX];
+    const int N0 = Ag.N0;
 #pragma unroll
-    for (int u = 0; u < TAIL_BMAX; u++) {
+    for (int u = 0; u < BMAX; u++) {
         const int e = tid + TAIL_THREADS * u;
         if (e < N0) bt[u] = gload(b_first + e);
     }
     // a vector load (the index lives in a VGPR), so that the flag is waited
     // for where it is tested, not at once by a scalar branch
     int skipped = 0;
-    if (A.skip) {
+    if (Ag.skip) {
         int z = 0;
         asm volatile("" : "+v"(z));
-        skipped = gload(A.skip + z);
+        skipped = gload(Ag.skip + z);
     }
-    double rs[1] = {0.0};
+    double rs = 0.0;
     FinState fs{};
-    if (test && tid == 0) fs = fin_state(A.ctrl);
-    if (test && tid < FIN_THREADS)   // the finish kernel's order
-        for (int e = tid; e < A.nrr; e += FIN_THREADS) rs[0] += gload(A.rr + e);
-
-    // x = 0 on every level (ghosts included) while the loads are in flight
-    for (int l = 0; l < nl; l++) {
-        CT* X = lds + A.xo[l];
-        for (int e = tid; e < A.g[l].N; e += TAIL_THREADS) X[e] = CT(0);
+    if (test) {
+        fs = fin_state(Ag.ctrl);
+        if (tid < FIN_THREADS)   // the finish kernel's order
+            for (int e = tid; e < Ag.nrr; e += FIN_THREADS) rs += gload(Ag.rr + e);
     }
-    TailPair<CT> P0[TAIL_MAXP], P1[1], P2[1], P3[1], P4[1];
-#pragma unroll
-    for (int v = 0; v < TAIL_MAXP; v++) tail_pair_from_rec<D, CT>(P0[v], R0[v], A.g[0], tid + TAIL_THREADS * v);
-    if (nl > 1) tail_pair_from_rec<D, CT>(P1[0], R1, A.g[1], tid); else P1[0].valid = false;
-    if constexpr (NLMAX > 2) { if (nl > 2) tail_pair_from_rec<D, CT>(P2[0], R2, A.g[2], tid); }
-    if constexpr (NLMAX > 3) { if (nl > 3) tail_pair_from_rec<D, CT>(P3[0], R3, A.g[3], tid); }
-    if constexpr (NLMAX > 4) { if (nl > 4) tail_pair_from_rec<D, CT>(P4[0], R4, A.g[4], tid); }
+    {
+        constexpr int NW = (int)(sizeof(TailArgs<C4>) / 4);
+        static_assert(NW <= TAIL_THREADS && sizeof(TailArgs<C4>) % 4 == 0, "tail arguments");
+        if (tid < NW) reinterpret_cast<uint32_t*>(&A)[tid] = reinterpret_cast<const uint32_t*>(&Ag)[tid];
+    }
+    // x = 0 on every level (ghosts included) while the loads are in flight;
+    // the other arrays lie behind or between and are written before they are read
+    for (int e = tid; e < Ag.ro; e += TAIL_THREADS) lds[e] = CT(0);
+    __syncthreads();
     {
         CT* B0 = lds + A.bo[0];
 #pragma unroll
-        for (int u = 0; u < TAIL_BMAX; u++) {
+        for (int u = 0; u < BMAX; u++) {
             const int e = tid + TAIL_THREADS * u;
             if (e < N0) B0[e] = (CT)bt[u];
         }
     }
+    if (test && tid < FIN_THREADS) {
+        rs = wave_sum(rs);
+        if ((tid & (WAVE - 1)) == 0) s_rr[tid / WAVE] = rs;
+    }
+    TailPair<CT> P0[TAIL_MAXP], P1[1], P2[1], P3[1], P4[1];
+#pragma unroll
+    for (int v = 0; v < TAIL_MAXP; v++) tail_pair_from_rec<D, CT>(P0[v], R0[v], tid + TAIL_THREADS * v, np[0]);
+    tail_pair_from_rec<D, CT>(P1[0], R1, tid, np[1]);
+    if constexpr (NLMAX > 2) tail_pair_from_rec<D, CT>(P2[0], R2, tid, np[2]);
+    if constexpr (NLMAX > 3) tail_pair_from_rec<D, CT>(P3[0], R3, tid, np[3]);
+    if constexpr (NLMAX > 4) tail_pair_from_rec<D, CT>(P4[0], R4, tid, np[4]);
     __syncthreads();
-    if (test) {   // one launch less per iteration than a finish kernel of its own (2.7 us)
-        __shared__ int s_stop;
-        block_sum<1>(rs);
-        if (tid == 0) s_stop = fin_update_scalars(A.ctrl, fs, rs[0]);
-        __syncthreads();
-        skipped |= s_stop;
+    if (test) {   // every thread takes the same decision from the same values, thread 0 stores it
+        double tot = s_rr[0];
+        for (int w = 1; w < FIN_THREADS / WAVE; w++) tot += s_rr[w];
+        skipped |= fin_update_scalars(tid == 0 ? Ag.ctrl : nullptr, fs, tot);
     }
     if (skipped) return;   // uniform: every thread read the same flag
 
-    auto level_down = [&](auto& P, int l) {
-        // geometry and offsets copied to registers once: read through the
-        // LDS copy of the arguments they would be fetched again after every
-        // barrier
-        const Geo g = A.g[l], gc = A.g[l + 1];
-        CT* X = lds + A.xo[l];
-        const CT* Bv = lds + A.bo[l];
-        CT* Rs = lds + A.ro;
-        CT* BC = lds + A.bo[l + 1];
-        CT* XC = lds + A.xo[l + 1];
-        tail_smooth<D>(P, X, Bv, g, 1);
-        __syncthreads();
-        tail_smooth<D>(P, X, Bv, g, 0);
-        __syncthreads();
-        tail_residual<D>(P, X, Bv, Rs, g);
-        __syncthreads();
-        tail_restrict<D, CT>(Rs, BC, XC, g, gc);
-        __syncthreads();
+    // per-level offsets and strides, uniform
+    auto u32 = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    struct Lev { CT *X, *B; int sx, sy; };
+    auto level = [&](int l) { return Lev{lds + u32(A.xo[l]), lds + u32(A.bo[l]), u32((int)A.g[l].sx), u32((int)A.g[l].sy)}; };
+    CT* Rs = lds + u32(A.ro);
+    const bool w0 = u32(tid >> 6) == 0;
+    // levels of at most 64 pairs (every one after the first such level): all
+    // pairs belong to wave 0, whose LDS accesses complete in program order;
+    // the fences keep the compiler from moving them across passes
+    auto wave = [&](int l) { return np[l] <= WAVE; };
+    auto sync = [&](bool w) {
+        if (w) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        } else {
+            __syncthreads();
+        }
     };
-    auto level_coarsest = [&](auto& P, int l) {
-        CT* X = lds + A.xo[l];
-        const CT* Bv = lds + A.bo[l];
-        const Geo g = A.g[l];
-        const int npass = A.npass;
-        const int npairs = ((g.nx + 1) >> 1) * g.ny * (D == 3 ? g.nz : 1);
-        if (npairs <= 64) {
-            // every pair is owned by a lane of wave 0 (thread = pair): the
-            // passes need no workgroup barrier, only wave order (LDS accesses
-            // of one wave complete in program order; the fences keep the
-            // compiler from moving them across passes)
-            if (tid < 64) {
-                for (int s = 0; s < npass; s++) {
-                    tail_smooth<D>(P, X, Bv, g, (s & 1) ? 0 : 1);
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                }
-            }
-            __syncthreads();
-            return;
+    // the first pass of level l is done; leaves the first pass of level l + 1 done
+    auto level_down = [&](auto& P, auto& PC, int l) {
+        const bool w = wave(l);
+        if (w && !w0) return;
+        const Lev L = level(l), C = level(l + 1);
+        sync(w);
+        tail_smooth<D, 0>(P, L.X, L.B, L.sx, L.sy);
+        sync(w);
+        tail_residual<D>(P, L.X, L.B, Rs, L.sx, L.sy);
+        sync(w);
+        tail_restrict<D>(PC[0], Rs, C.B, C.X, L.sx, L.sy, l + 2 < nl || A.npass > 0);
+    };
+    auto level_coarsest = [&](auto& P, int l) {   // odd, even, odd, ... (forward/reverse pairs collapsed)
+        const bool w = wave(l);
+        if (w && !w0) return;
+        const Lev L = level(l);
+        const int npass = u32(A.npass);
+        int s = 1;                                 // the first pass is done
+        for (; s + 1 < npass; s += 2) {
+            sync(w);
+            tail_smooth<D, 0>(P, L.X, L.B, L.sx, L.sy);
+            sync(w);
+            tail_smooth<D, 1>(P, L.X, L.B, L.sx, L.sy);
         }
-        for (int s = 0; s < npass; s++) {     // odd, even, odd, ... (forward/reverse pairs collapsed)
-            tail_smooth<D>(P, X, Bv, g, (s & 1) ? 0 : 1);
-            __syncthreads();
-        }
+        if (s < npass) { sync(w); tail_smooth<D, 0>(P, L.X, L.B, L.sx, L.sy); }
     };
     auto level_up = [&](auto& P, int l) {
-        const Geo g = A.g[l], gc = A.g[l + 1];
-        CT* X = lds + A.xo[l];
-        const CT* Bv = lds + A.bo[l];
-        const CT* XC = lds + A.xo[l + 1];
-        tail_prolong<D>(P, X, XC, g, gc);
-        __syncthreads();
-        tail_smooth<D>(P, X, Bv, g, 0);
-        __syncthreads();
-        tail_smooth<D>(P, X, Bv, g, 1);
-        __syncthreads();
+        const bool w = wave(l);
+        if (w && !w0) return;
+        const Lev L = level(l);
+        sync(w);
+        tail_prolong(P, L.X, lds + u32(A.xo[l + 1]));
+        sync(w);
+        tail_smooth<D, 0>(P, L.X, L.B, L.sx, L.sy);
+        sync(w);
+        tail_smooth<D, 1>(P, L.X, L.B, L.sx, L.sy);
     };
+    if (nl > 1 || A.npass > 0) {
+        const CT* B0 = lds + u32(A.bo[0]);
+#pragma unroll
+        for (int v = 0; v < TAIL_MAXP; v++)
+            if (P0[v].valid) tail_first(P0[v], lds + u32(A.xo[0]), B0[P0[v].id[1]]);
+    }
     // down
-    if (nl > 1) level_down(P0, 0);
-    if constexpr (NLMAX > 2) { if (nl > 2) level_down(P1, 1); }
-    if constexpr (NLMAX > 3) { if (nl > 3) level_down(P2, 2); }
-    if constexpr (NLMAX > 4) { if (nl > 4) level_down(P3, 3); }
+    if (nl > 1) level_down(P0, P1, 0);
+    if constexpr (NLMAX > 2) { if (nl > 2) level_down(P1, P2, 1); }
+    if constexpr (NLMAX > 3) { if (nl > 3) level_down(P2, P3, 2); }
+    if constexpr (NLMAX > 4) { if (nl > 4) level_down(P3, P4, 3); }
     // coarsest
     if (nl == 1) level_coarsest(P0, 0);
     if (nl == 2) level_coarsest(P1, 1);
@@ -456,9 +420,15 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     if constexpr (NLMAX > 3) { if (nl > 3) level_up(P2, 2); }
     if constexpr (NLMAX > 2) { if (nl > 2) level_up(P1, 1); }
     if (nl > 1) level_up(P0, 0);
-    {
-        const CT* X0 = lds + A.xo[0];
-        for (int e = tid; e < A.g[0].N; e += TAIL_THREADS) gstore(x_first + e, (S)X0[e]);
+    // a thread stores its own cells (its last pass wrote the odd ones, the
+    // pass before the even ones); ghosts of x are 0 from its allocation
+    const CT* X0 = lds + u32(A.xo[0]);
+#pragma unroll
+    for (int v = 0; v < TAIL_MAXP; v++) {
+        if (!P0[v].valid) continue;
+        const int id0 = P0[v].first_odd ? P0[v].id[1] : P0[v].id[0];
+        gstore(x_first + id0, (S)X0[id0]);
+        if (P0[v].ok1) gstore(x_first + id0 + 1, (S)X0[id0 + 1]);
     }
 }
 

@@ -257,22 +257,10 @@ __global__ __launch_bounds__(T2_THREADS) void k_t2_up(const VB* __restrict__ b, 
 // each column is added from the top down and the columns as block_store adds
 // them.  512 threads, 128 pairs a row, row rj + 4 u for u < U (KC + 4 <= 4 U);
 // all neighbours come from LDS here (a row spans two waves).  1/d comes from a
-// table of the 16 neighbour patterns (rdiv).  Chunks of more than 12 rows
+// table of the 16 neighbour patterns (rdiv, kernels_vcycle.hpp).  Chunks of more than 12 rows
 // (grids of about 2.5 million cells and more) stay on the march kernel, whose
 // halo rows then cost little.
 constexpr int T2U_RX = 256, T2U_HX = 128, T2U_MAXU = 4;
-
-// n / d from d's correctly rounded reciprocal: the product, its exact
-// remainder (FMA) and the remainder's share, which is the correctly rounded
-// quotient (Markstein, IBM J. Res. Dev. 34, 1990) in 3 operations instead of
-// the division's 10 or so.  FP32 divides by the hardware reciprocal (mdiv).
-__device__ __forceinline__ double rdiv(double n, double d, double rinv) {
-    const double q = n * rinv;
-    return fma(fma(-q, d, n), rinv, q);
-}
-__device__ __forceinline__ float rdiv(float n, float, float rinv) { return n * rinv; }
-__device__ __forceinline__ double recip(double d) { return 1.0 / d; }
-__device__ __forceinline__ float recip(float d) { return __builtin_amdgcn_rcpf(d); }
 
 template <int U, typename VB, typename VCX>
 __device__ __forceinline__ void d_t2_up0(const VB* __restrict__ b, const uint8_t* __restrict__ nbr, const Geo& g,

@@ -13,6 +13,18 @@
 
 namespace uaamg {
 
+// n / d from d's correctly rounded reciprocal: the product, its exact
+// remainder (FMA) and the remainder's share, which is the correctly rounded
+// quotient (Markstein, IBM J. Res. Dev. 34, 1990) in 3 operations instead of
+// the division's 10 or so.  FP32 divides by the hardware reciprocal (mdiv).
+__device__ __forceinline__ double rdiv(double n, double d, double rinv) {
+    const double q = n * rinv;
+    return fma(fma(-q, d, n), rinv, q);
+}
+__device__ __forceinline__ float rdiv(float n, float, float rinv) { return n * rinv; }
+__device__ __forceinline__ double recip(double d) { return 1.0 / d; }
+__device__ __forceinline__ float recip(float d) { return __builtin_amdgcn_rcpf(d); }
+
 // The 7-point (5-point in 2D) stencil of one cell in compute type CT.
 template <typename CT>
 struct Sten {

@@ -817,13 +817,12 @@ extern "C" int uaamg_batch_solve(uaamg_batch* b, const double* const* rhs_dev, d
 // completes the converged ones.  Requests that arrive while others run join
 // at the next chunk.
 //
-// Simulations are split into two size classes (below / from 2^18 padded
-// cells), each with a stream of its own and one batch per dimension: a class
-// whose chunk has finished is completed, refilled and relaunched while the
-// other runs, so a 64^2 request does not wait for the chunks of 256^3
-// members (a chunk of the large class takes milliseconds, one of the small
-// class tens of microseconds).  Two streams besides the caller's keep the
-// classes on hardware queues of their own (a process has four).
+// Simulations are split into classes by size (below / from 2^18 padded
+// cells), the large ones by dimension too, each class with a stream of its
+// own: a class whose chunk has finished is completed, refilled and relaunched
+// while the others run, so a 64^2 request does not wait for the chunks of
+// 256^3 members (a chunk of a large class takes milliseconds, one of the small
+// class tens of microseconds).
 
 namespace {
 struct SimState {
@@ -864,7 +863,7 @@ struct uaamg_server {
     std::string err;
     size_t budget = 0, used = 0;
     int max_active = 0;
-    // one batch per part; one stream and completion event per size class;
+    // one batch per part; one stream and completion event per class;
     // inflight: a chunk of the class was launched and its event has not been
     // seen complete
     std::unique_ptr<uaamg::BatchBase> part[kServeParts];
