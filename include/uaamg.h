@@ -75,10 +75,12 @@ typedef struct {
      * _TAIL, _PMV) or rows_kc / march_* through uaamg_set_opts drops the grid
      * (set it again). */
     int forms;                 /* bitmask of UAAMG_FORM_* allowed (default UAAMG_FORM_DEFAULT) */
-    int xfork_level;           /* side-stream x update forked after this level's down kernel
-                                  (>= the tail's first level: right before the tail); default 2 */
-    int xblocks, xthreads;     /* x update launch: at most xblocks workgroups of xthreads (default 256 x 256) */
-    int rows_kc;               /* planes per level-0 row-kernel tile, multiple of 4 (0: auto) */
+    int xfork_level;           /* side-stream x update (grids of more than 6 * 2^20 cells) forked
+                                  after this level's down kernel (>= the tail's first level: right
+                                  before the tail); default 2 */
+    int xblocks, xthreads;     /* its launch: at most xblocks workgroups of xthreads (default 256 x 256) */
+    int rows_kc;               /* planes per level-0 row-kernel tile, multiple of 4 (0: auto, which
+                                  may also take 2) */
     int march_kc_min;          /* fewest planes per march-kernel chunk, even (default 2) */
     int march_target;          /* workgroups a march-kernel launch aims at (default 1024) */
     int trace;                 /* 1: relative residual history of each solve to stderr */

@@ -323,7 +323,7 @@ private:
             // level 0
             if (D == 3 && d.cpl) {
                 // row tiles of rows_kc_ planes (0: the engine's own choice)
-                d.rgeo = E::make_rowgeo(d.g0.ny, d.g0.nz, E::ROWS_NW * E::ROWS_RW - 4, rows_kc_);
+                d.rgeo = E::make_rowgeo(d.g0.ny, d.g0.nz, E::ROWS_NW * E::ROWS_RW - 4, rows_kc_, 1, 64, false);
                 std::vector<BItem>& L = rows[d.cpl == 2 ? 0 : 1];
                 d.up_base = (int)L.size();
                 d.up_cnt = d.rgeo.ntiles;

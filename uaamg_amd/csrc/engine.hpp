@@ -205,7 +205,7 @@ public:
             pmv_blocks_ = flat_blocks(2048);
         }
         timer_.s = stream_;
-        if (D == 3 && pmv_on_) {   // the x update's stream, created before any capture
+        if (D == 3 && pmv_on_ && !xinline()) {   // the x update's stream, created before any capture
             HIPCHK(hipStreamCreateWithFlags(&xs_, hipStreamNonBlocking));
             HIPCHK(hipEventCreateWithFlags(&xfork_, hipEventDisableTiming));
             HIPCHK(hipEventCreateWithFlags(&xjoin_, hipEventDisableTiming));
@@ -697,12 +697,24 @@ public:
     RowGeo rgeo_{};
     unsigned rows_blocks_ = 0;
     // cells per lane and windows of rows of nx cells (0: no row kernels)
-    static int row_lanes(int nx, int& nwx, int& wl) {
-        const int cpl = sizeof(T) == 8 || nx <= 128 ? 2 : 4;
+    static int row_lanes(int nx, int& nwx, int& wl, int cpl = 0) {
+        if (!cpl) cpl = sizeof(T) == 8 || nx <= 128 ? 2 : 4;
         const int lanes = (nx + cpl - 1) / cpl;
         nwx = lanes <= 64 ? 1 : (lanes <= 126 ? 2 : (lanes + 61) / 62);
         wl = nwx == 1 ? 64 : (lanes + nwx - 1) / nwx;
         return cpl;
+    }
+    // FP32 rows of 129 to 256 cells in two or three windows of 2 cells a lane
+    // instead of whole with 4: where the chip holds the tiles of 4 planes at
+    // once a plane step's latency counts, not its bytes, and a step of half
+    // the cells takes half the time (151 x 97 x 63: 11.4 -> 9.7 ms per solve,
+    // 250 x 64 x 64 3.45 -> 2.74).  Larger grids are slower so (160^3 4.7 ->
+    // 4.9, 256^3 11.6 -> 14.6) or the same (200 x 120 x 80).
+    static bool narrow_rows(int nx, int ny, int nz) {
+        int nwx, wl;
+        if (sizeof(T) != 4 || nx <= 128 || nx > 256) return false;
+        row_lanes(nx, nwx, wl, 2);
+        return (long)nwx * ((ny + 15) / 16) * ((nz + 3) / 4) <= 256;
     }
     // the row kernels address a level by 32-bit element offsets
     static bool rows_addressable(const Geo& g) { return g.N < (1L << 31) - 1024; }
@@ -713,6 +725,7 @@ public:
             if (nlevels() < 2 || !rows_addressable(g0_)) return;
             int nwx, wl;
             rows_cpl_ = row_lanes(n_[0], nwx, wl);
+            if (narrow_rows(n_[0], n_[1], n_[2])) rows_cpl_ = row_lanes(n_[0], nwx, wl, 2);
             rows_win_ = nwx > 1;
             const double ix = 1.0 / (h[0] * h[0]), iy = 1.0 / (h[1] * h[1]), iz = 1.0 / (h[2] * h[2]);
             for (int m = 0; m < 64; m++) {
@@ -742,24 +755,28 @@ public:
             pmv_blocks_ = 8u * (unsigned)pgeo_.per_xcd;
         }
     }
-    // Tiles of the row kernels: TY rows by KC planes, KC a multiple of 4, unless
-    // kc_force > 0 sets it
-    static RowGeo make_rowgeo(int ny, int nz, int TY = ROWS_NW * ROWS_RW - 4, int kc_force = 0, int nwx = 1, int wl = 64) {
+    // Tiles of the row kernels: TY rows by KC planes, KC 2 or a multiple of 4,
+    // unless kc_force > 0 sets it; alone: no other grid shares the launch
+    static RowGeo make_rowgeo(int ny, int nz, int TY = ROWS_NW * ROWS_RW - 4, int kc_force = 0, int nwx = 1, int wl = 64, bool alone = true) {
         RowGeo rg{};
         rg.nwx = nwx;
         rg.wl = wl;
         rg.nty = (ny + TY - 1) / TY;
+        auto tiles = [&](int k) { return (long)rg.nty * nwx * ((nz + k - 1) / k); };
         // fewest plane steps in sequence on a CU: rounds of 256 workgroups
         // (one per CU: ten waves of about 145 VGPRs) times the planes of a
         // chunk, its 4 halo planes and about 2 steps' time to start
         int KC = 4;
         long best = 0;
         for (int k = 4; k <= 64; k += 4) {
-            const long tiles = (long)rg.nty * nwx * ((nz + k - 1) / k);
-            const long cost = (tiles + 255) / 256 * (k + 6);
+            const long cost = (tiles(k) + 255) / 256 * (k + 6);
             if (k == 4 || cost < best) { best = cost; KC = k; }
-            if (tiles <= (long)rg.nty * nwx) break;
+            if (tiles(k) <= (long)rg.nty * nwx) break;
         }
+        // 2 planes (6 steps for 8) where the chip holds those tiles too: 64^3
+        // FP32 1.77 -> 1.64 ms per solve, 160 x 100 x 60 4.02 -> 3.59, 128 x 64
+        // x 64 FP64 2.26 -> 2.14; in two rounds slower (96^3 2.36 -> 2.79)
+        if (alone && KC == 4 && tiles(2) <= 256) KC = 2;
         if (kc_force > 0) KC = std::max(4, kc_force / 4 * 4);
         rg.KC = KC;
         rg.nkc = (nz + KC - 1) / KC;
@@ -780,7 +797,7 @@ public:
                 // two cells per lane (64 < nx <= 128): smaller levels stay on the
                 // march kernels (too few rows to fill the chip), wider ones would
                 // need four cells per lane and more registers than the workgroup has
-                if (g.nx <= 64 || g.nx > 128) continue;
+                if (g.nx <= 64 || g.nx > 128 || t3_level(l)) continue;
                 rcpl_[l] = 2;
                 rgl_[l] = make_rowgeo(g.ny, g.nz);
             }
@@ -828,12 +845,13 @@ public:
                 // UAAMG_FORM_NT_D plain): 34.5 vs 33.5 solves/s at 256^3 in three paired runs
                 const bool dnt = rows_nt(UAAMG_FORM_NT_D);
                 forms_used_ |= dnt ? UAAMG_FORM_NT_D : 0;
-                auto kern = rows_win_ ? (dnt ? k_rows_down0r<ROWS_CPL, ROWS_NW, ROWS_RW, S, true, false, true, T>
-                                             : k_rows_down0r<ROWS_CPL, ROWS_NW, ROWS_RW, S, false, false, true, T>)
+                auto kern = rows_win_ ? (dnt ? k_rows_down0r<2, ROWS_NW, ROWS_RW, S, true, false, true, T>
+                                             : k_rows_down0r<2, ROWS_NW, ROWS_RW, S, false, false, true, T>)
                                       : k_rows_down0r<2, ROWS_NW, ROWS_RW, S, false, false, false, T>;
                 if constexpr (ROWS_CPL == 4)
-                    if (!rows_win_ && rows_cpl_ == 4)
-                        kern = dnt ? (rows_full() ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true>)
+                    if (rows_cpl_ == 4)
+                        kern = rows_win_ ? (dnt ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, false, true> : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, false, false, true>)
+                             : dnt ? (rows_full() ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true>)
                                    : k_rows_down0r<4, ROWS_NW, ROWS_RW, S>;
                 tlaunch(timer_, UAAMG_K_DOWN0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, (const T*)fr_old_,
                         (const uint8_t*)nbr0_, g0_, rtab_, rgeo_, C.b, C.g, skip, (const T*)Ap_, (T*)r, partials_,
@@ -843,9 +861,9 @@ public:
                 else if (!fin_fold_) k_fin_update<false><<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)rows_blocks_, ctrl_);
                 return;
             }
-            auto kern = rows_win_ ? k_rows_down0<ROWS_CPL, ROWS_NW, ROWS_RW, S, true, T> : k_rows_down0<2, ROWS_NW, ROWS_RW, S, false, T>;
+            auto kern = rows_win_ ? k_rows_down0<2, ROWS_NW, ROWS_RW, S, true, T> : k_rows_down0<2, ROWS_NW, ROWS_RW, S, false, T>;
             if constexpr (ROWS_CPL == 4)
-                if (!rows_win_ && rows_cpl_ == 4) kern = k_rows_down0<4, ROWS_NW, ROWS_RW, S>;
+                if (rows_cpl_ == 4) kern = rows_win_ ? k_rows_down0<4, ROWS_NW, ROWS_RW, S, true> : k_rows_down0<4, ROWS_NW, ROWS_RW, S>;
             tlaunch(timer_, UAAMG_K_DOWN0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, (const uint8_t*)nbr0_, g0_, rtab_,
                     rgeo_, C.b, C.g, skip);
         }
@@ -856,12 +874,13 @@ public:
             // 33.9 solves/s at 256^3 in three paired runs
             const bool unt = rows_nt(UAAMG_FORM_NT_U);
             forms_used_ |= unt ? UAAMG_FORM_NT_U : 0;
-            auto kern = rows_win_ ? (unt ? k_rows_up0<ROWS_CPL, ROWS_NW, ROWS_RW, S, true, false, true, T>
-                                         : k_rows_up0<ROWS_CPL, ROWS_NW, ROWS_RW, S, false, false, true, T>)
+            auto kern = rows_win_ ? (unt ? k_rows_up0<2, ROWS_NW, ROWS_RW, S, true, false, true, T>
+                                         : k_rows_up0<2, ROWS_NW, ROWS_RW, S, false, false, true, T>)
                                   : k_rows_up0<2, ROWS_NW, ROWS_RW, S, false, false, false, T>;
             if constexpr (ROWS_CPL == 4)
-                if (!rows_win_ && rows_cpl_ == 4)
-                    kern = unt ? (rows_full() ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_up0<4, ROWS_NW, ROWS_RW, S, true>)
+                if (rows_cpl_ == 4)
+                    kern = rows_win_ ? (unt ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, false, true> : k_rows_up0<4, ROWS_NW, ROWS_RW, S, false, false, true>)
+                         : unt ? (rows_full() ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_up0<4, ROWS_NW, ROWS_RW, S, true>)
                                : k_rows_up0<4, ROWS_NW, ROWS_RW, S>;
             tlaunch(timer_, UAAMG_K_UP0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, (const uint8_t*)nbr0_, g0_, rtab_, rgeo_,
                     (const S*)C.x, C.g, z, skip, partials_);
@@ -905,7 +924,8 @@ public:
             Level& C = lv_[l + 1];
             if (l == 0 && rows_cpl_) {
                 rows_down0(r, C, skip);
-                if (fr_old_ && xfork_level() == 0) fork_x();
+                if (fr_old_ && xinline()) { launch_x(stream_, 256, 2048); xforked_ = true; }
+                else if (fr_old_ && xfork_level() == 0) fork_x();
             } else if (l == 0) {
                 MLaunch m = mlaunch(g0_, RX0, RY0);
                 tlaunch(timer_, UAAMG_K_DOWN0, k_down_m<D, true, RX0, RY0, PPT0, T, C4, S, C4>, m.grid, dim3(256), stream_,
@@ -919,7 +939,7 @@ public:
                 FusedArgs<D, false, SC, C4> A{F.g, nullptr, F.coef, Consts<SC>{}};
                 MLaunch m = mlaunch(F.g, RXC, RYC);
                 auto launch = [&](auto kern, dim3 grid, int threads, auto... args) {
-                    if (fr_old_ && xfork_level() == l && !timer_.on && !capturing_) {
+                    if (fr_old_ && !xforked_ && xfork_level() == l && !timer_.on && !capturing_) {
                         // the fork event rides on this dispatch's completion: no
                         // marker packet between it and the next kernel on stream_
                         hipExtLaunchKernelGGL(kern, grid, dim3(threads), 0, stream_, nullptr, xfork_, 0, args...);
@@ -932,7 +952,7 @@ public:
                 else launch(k_down_m<D, false, RXC, RYC, PPTC, S, C4, S, C4>, m.grid, 256, (const S*)F.b, A, C.b, (const C4*)C.coef, C.g, m.KC, skip);
             }
             HIPCHK(hipGetLastError());
-            if (fr_old_ && l > 0 && xfork_level() == l) fork_x();
+            if (fr_old_ && !xforked_ && l > 0 && xfork_level() == l) fork_x();
         }
         if (fr_old_ && !xforked_ && xfork_level() >= lt) fork_x();   // before the tail / coarsest solve
         coarse_solve(skip, nrr_);
@@ -1203,13 +1223,16 @@ public:
                 // UAAMG_FORM_NT_P plain): 33.6 vs 33.0 solves/s at 256^3 in three paired runs
                 const bool pnt = rows_nt(UAAMG_FORM_NT_P) && fr_;
                 forms_used_ |= pnt ? UAAMG_FORM_NT_P : 0;
-                auto kern = rows_win_ ? (fr_ ? (pnt ? k_rows_pmv<ROWS_CPL, PMV_NW, PMV_RW, true, true, false, true, T>
-                                                    : k_rows_pmv<ROWS_CPL, PMV_NW, PMV_RW, true, false, false, true, T>)
-                                             : k_rows_pmv<ROWS_CPL, PMV_NW, PMV_RW, false, false, false, true, T>)
+                auto kern = rows_win_ ? (fr_ ? (pnt ? k_rows_pmv<2, PMV_NW, PMV_RW, true, true, false, true, T>
+                                                    : k_rows_pmv<2, PMV_NW, PMV_RW, true, false, false, true, T>)
+                                             : k_rows_pmv<2, PMV_NW, PMV_RW, false, false, false, true, T>)
                                       : (fr_ ? k_rows_pmv<2, PMV_NW, PMV_RW, true, false, false, false, T>
                                              : k_rows_pmv<2, PMV_NW, PMV_RW, false, false, false, false, T>);
                 if constexpr (ROWS_CPL == 4)
-                    if (!rows_win_ && rows_cpl_ == 4)
+                    if (rows_cpl_ == 4 && rows_win_)
+                        kern = fr_ ? (pnt ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, false, true> : k_rows_pmv<4, PMV_NW, PMV_RW, true, false, false, true>)
+                                   : k_rows_pmv<4, PMV_NW, PMV_RW, false, false, false, true>;
+                    else if (rows_cpl_ == 4)
                         kern = fr_ ? (pnt ? (rows_full() ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, true> : k_rows_pmv<4, PMV_NW, PMV_RW, true, true>)
                                           : k_rows_pmv<4, PMV_NW, PMV_RW, true>)
                                    : k_rows_pmv<4, PMV_NW, PMV_RW, false>;
@@ -1417,21 +1440,33 @@ private:
     bool xforked_ = false;         // this iteration's x pass was forked
     int xslot_ = 0;                // Ctrl::xa slot (p buffer) of this iteration's x pass
     bool capturing_ = false;       // a hipGraph capture of stream_ is open
-    void fork_x() {
-        if (!fork_recorded_) HIPCHK(hipEventRecord(xfork_, stream_));
-        fork_recorded_ = false;
-        HIPCHK(hipStreamWaitEvent(xs_, xfork_, 0));
-        const unsigned xthreads = (unsigned)std::min(1024, std::max(64, o_.xthreads / 64 * 64));
-        const long xneed = (N4_ / 4 + xthreads - 1) / xthreads;
-        const unsigned xb = (unsigned)std::max<long>(1, std::min<long>(xneed, std::max(8, o_.xblocks)));
+    // Grids of up to kInlineCells padded cells run the update on the main
+    // stream, right behind the level-0 down kernel: the fork and the join cost
+    // 12 us of barrier packets per iteration and as many host calls, the update
+    // itself 3 to 11 (FP32, per solve: 48 x 40 x 36 1.29 -> 1.13 ms, 64^3 1.63 ->
+    // 1.44, 128^3 2.77 -> 2.65, 160^3 4.48 -> 4.42, but 200^3 8.13 -> 8.32 and
+    // 256^3 11.6 -> 12.0; FP64 128 x 64 x 64 2.11 -> 1.96, 256 x 128 x 128 6.03 ->
+    // 5.93).
+    static constexpr long kInlineCells = 6L << 20;
+    bool xinline() const { return N4_ <= kInlineCells; }
+    void launch_x(hipStream_t s, unsigned threads, long blocks) {
         // nontemporal loads and stores (without UAAMG_FORM_NT_X plain): x and p
         // are used once here, and the kernels running beside the update keep
         // their working set in the caches (33.3 vs 32.9 solves/s at 256^3)
         const bool xnb = (o_.forms & UAAMG_FORM_XMASK) != 0;
         const bool xnt = !xnb && (o_.forms & UAAMG_FORM_NT_X);
         forms_used_ |= (xnb ? UAAMG_FORM_XMASK : 0) | (xnt ? UAAMG_FORM_NT_X : 0);
-        tlaunch(timer_, UAAMG_K_UPDATE, xnb ? k_xupdate<T, true> : (xnt ? k_xupdate<T, false, true> : k_xupdate<T, false>), dim3(xb),
-                dim3(xthreads), xs_, xfork_x_, xfork_p_, (const uint8_t*)nbr0_, N4_, (const double*)&ctrl_->xa[xslot_]);
+        const long need = (N4_ / 4 + threads - 1) / threads;
+        tlaunch(timer_, UAAMG_K_UPDATE, xnb ? k_xupdate<T, true> : (xnt ? k_xupdate<T, false, true> : k_xupdate<T, false>),
+                dim3((unsigned)std::max<long>(1, std::min(need, blocks))), dim3(threads), s, xfork_x_, xfork_p_, (const uint8_t*)nbr0_, N4_,
+                (const double*)&ctrl_->xa[xslot_]);
+    }
+    void fork_x() {
+        if (!fork_recorded_) HIPCHK(hipEventRecord(xfork_, stream_));
+        fork_recorded_ = false;
+        HIPCHK(hipStreamWaitEvent(xs_, xfork_, 0));
+        const unsigned xthreads = (unsigned)std::min(1024, std::max(64, o_.xthreads / 64 * 64));
+        launch_x(xs_, xthreads, std::max(8, o_.xblocks));
         HIPCHK(hipEventRecord(xjoin_, xs_));
         xpend_ = true;
         xforked_ = true;

@@ -73,7 +73,7 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
     const int dir = (th.kc & 1) ? -1 : 1;
     const int lane = th.lane, w = th.w;
 
-    F PN[4][RW][CPL];        // p_new of planes (slot = plane & 3)
+    F PN[4][RW][CPL];        // p_new of the last four planes
     uint8_t NB[4][RW][CPL];
     F pfz[2][RW][CPL], pfp[2][RW][CPL];
     uint8_t pfn[2][RW][CPL];

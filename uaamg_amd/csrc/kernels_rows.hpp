@@ -60,7 +60,7 @@ using RowTab = RowTabOf<float>;
 struct RowGeo {
     int nty;       // tiles in y
     int nkc;       // chunks in z
-    int KC;        // planes per chunk (multiple of 4)
+    int KC;        // planes per chunk (even)
     int ntiles;    // nwx * nty * nkc
     int per_xcd;   // ceil(ntiles / 8)
     int nwx;       // windows in x (1: a wave owns whole rows)
@@ -375,7 +375,8 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
     issue(1, th.m0 - 2);
     issue(0, th.m0 - 1);
 
-    // one plane step: plane P enters the window; S = P & 3
+    // one plane step: plane P enters the window, in slot S (the first plane in
+    // slot 3, so S and P have the same parity: chunks have an even number of planes)
     auto step = [&](auto Sc, int P) {
         constexpr int S = decltype(Sc)::value;
         constexpr int S1 = (S + 3) & 3, S2 = (S + 2) & 3, S3 = (S + 1) & 3;   // planes P-1, P-2, P-3
@@ -501,7 +502,7 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
         }
         __syncthreads();
     };
-    for (int P = th.m0 - 2; P <= th.last + 2; P += 4) {   // m0 - 2 = 3 (mod 4)
+    for (int P = th.m0 - 2; P <= th.last + 2; P += 4) {   // m0 - 2 is odd
         step(IC<3>{}, P);
         if (P + 1 > th.last + 2) break;
         step(IC<0>{}, P + 1);
@@ -978,7 +979,7 @@ __device__ __forceinline__ void d_rows_downc(const SV* __restrict__ b, const C4*
         for (int c = 0; c < CPL / 2; c++) acc[a][c] = 0.0f;
     rec_prev_cz<CPL, NW, RW, C4>(Q, rec, th, g);
     // planes m0 - 2 .. m0 + REC_PD - 3 in flight before the first step, each
-    // in the buffer of its slot (m0 = 1 mod 4: plane m0 - 2 + d has slot 3 + d)
+    // in the buffer of its slot (plane m0 - 2 + d has slot 3 + d)
     sfor<REC_PD>([&](auto dc) {
         constexpr int d = decltype(dc)::value;
         rec_issue<CPL, NW, RW, SV, C4>(pf[(3 + d) & (REC_PD - 1)], b, rec, th, g, th.m0 - 2 + d);

@@ -471,7 +471,8 @@ extern "C" size_t uaamg_bytes_required(const uaamg_grid* g, const uaamg_opts* o)
     const bool gmg = o->preconditioner == UAAMG_PRECOND_GMG || o->preconditioner == UAAMG_PRECOND_AMG;
     size_t bytes = N0 + N4 + kRowSlack + 8 + sizeof(uaamg::Ctrl) + (pmv ? (d3 ? 7 : 6) : (gmg ? 6 : 5)) * uaamg::vec_stride((long)N4, (long)margin) * sv;
     if (pmv && !d3) bytes += (2048 + 64) * 8;
-    if (pmv && d3) bytes += (size_t)(8 * (((long)nwx * ((g0.ny + 15) / 16) * ((g0.nz + 3) / 4) + 7) / 8) + 64) * 8;   // p.Ap partials
+    if (pmv && d3)   // p.Ap partials; 256 tiles at most where a chunk has 2 planes or rows are narrow
+        bytes += (size_t)(8 * ((std::max(256L, (long)nwx * ((g0.ny + 15) / 16) * ((g0.nz + 3) / 4)) + 7) / 8) + 64) * 8;
     long maxb = std::max<long>(cells_launch(g0, g->dim).nblocks(), 2048);
     for (size_t l = 1; l < shape.size(); l++) {
         bytes += (size_t)shape[l].N * (3 * sl + 4 * sr + 1) + (size_t)kRowSlack * 6 * std::max(sl, sr);
