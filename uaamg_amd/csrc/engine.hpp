@@ -17,6 +17,7 @@
 #include "kernels_cg.hpp"
 #include "kernels_march.hpp"
 #include "kernels_rows.hpp"
+#include "kernels_rows64.hpp"
 #include "kernels_tail.hpp"
 #include "kernels_pmv.hpp"
 #include "kernels_tile.hpp"
@@ -200,12 +201,10 @@ public:
             throw HipError{hipErrorInvalidValue, "GMG / AMG preconditioners: 2D grids, FP64 or FP32 levels"};
         if (gmg_) { gmg_setup(); gmg_tail_setup(); }
         if (!ident_ && !gmg_) rows_setup(h, wall);   // the identity and GMG / AMG forms run the flat kernels only
-        if (D == 2) {
-            pmv_on_ = t2_pmv(o, shape_);
-            pmv_blocks_ = flat_blocks(2048);
-        }
+        if (D == 2) pmv_on_ = t2_pmv(o, shape_);
+        if (FLATCG) pmv_blocks_ = flat_blocks(2048);
         timer_.s = stream_;
-        if (D == 3 && pmv_on_ && !xinline()) {   // the x update's stream, created before any capture
+        if (!FLATCG && pmv_on_ && !xinline()) {   // the x update's stream, created before any capture
             HIPCHK(hipStreamCreateWithFlags(&xs_, hipStreamNonBlocking));
             HIPCHK(hipEventCreateWithFlags(&xfork_, hipEventDisableTiming));
             HIPCHK(hipEventCreateWithFlags(&xjoin_, hipEventDisableTiming));
@@ -605,7 +604,7 @@ public:
     bool t3_level(int l) const { return D == 3 && std::is_same<C4, float4>::value && t3_tiles(lv_[l].g) <= 512; }
 
     // ---- 2D tile kernels (kernels_tile.hpp) ----
-    // The CG passes of 2D grids: p update, operator and the finish of the z
+    // The CG passes of 2D grids and of 3D grids with FP64 vectors: p update, operator and the finish of the z
     // sums in one launch, alpha and the CG update in the next, the
     // convergence test in the tail (kernel_set 2).
     static bool t2_pmv(const uaamg_opts& o, const std::vector<Geo>& shape) {
@@ -617,7 +616,7 @@ public:
     // partials of the z sums (GMG / AMG: of the flat pass)
     int nzp() const {
         const MLaunch m = up0_launch();
-        return gmg_ ? (int)flat_blocks(2048) : (int)(m.grid.x * m.grid.z);
+        return gmg_ ? (int)flat_blocks(2048) : (int)(m.grid.x * m.grid.y * m.grid.z);
     }
     int nrr_ = 0;                // r.r partials that the tail finishes (0: none pending)
     void vcycle_t2(const T* r, T* z, const int* skip) {
@@ -661,12 +660,14 @@ public:
             HIPCHK(hipGetLastError());
         }
     }
-    // one CG iteration of the fused 2D form
+    // FP32 vectors in 3D run the fused passes on rows instead (k_rows_pmv, k_rows_down0r)
+    static constexpr bool FLATCG = D == 2 || sizeof(T) == 8;
+    // one CG iteration of the fused flat form
     void iteration_t2(T* x, const int* skip) {
-        if constexpr (D == 2) {
+        if constexpr (FLATCG) {
             const T* pold = pbuf(pcur_);
             T* pnew = pbuf(pcur_ ^ 1);
-            tlaunch(timer_, UAAMG_K_MATVEC, vlap_.d ? k_t2_pmv<T, true> : k_t2_pmv<T, false>, dim3(pmv_blocks_), dim3(FIN_THREADS),
+            tlaunch(timer_, UAAMG_K_MATVEC, D == 2 && vlap_.d ? k_t2_pmv<D, T, D == 2> : k_t2_pmv<D, T, false>, dim3(pmv_blocks_), dim3(FIN_THREADS),
                     stream_, (const T*)z_, pold, pnew, Ap_, (const uint8_t*)nbr0_, g0_, c0d_, N4_, ctrl_, (const double*)partials_,
                     nzp(), partials_m_, vlap_);
             pcur_ ^= 1;
@@ -686,10 +687,8 @@ public:
     // nx <= 128 with 2 cells a lane, <= 256 with 4; FP64: 2 cells, nx <= 128,
     // which is the same bytes and registers per lane as FP32 with 4), wider
     // rows in windows.  Against the march kernels and flat CG passes that ran
-    // here before: 128 x 64 x 64 FP64 projection 3.02 -> 2.22 ms, 256 x 128 x
-    // 128 FP64 solve (3 windows) 4.98 -> 4.02, 512 x 256 x 256 FP32 solve (3
-    // windows) 57.7 -> 37.5; down / up kernel at 256 x 128 x 128 FP64 66 -> 49
-    // / 75 -> 39 us.
+    // here before: 512 x 256 x 256 FP32 solve (3 windows) 57.7 -> 37.5 ms; FP64:
+    // kernels_rows64.hpp.
     static constexpr int ROWS_NW = 10, ROWS_RW = 2, ROWS_CPL = sizeof(T) == 8 ? 2 : 4;   // ROWS_CPL: of wide rows
     int rows_cpl_ = 0;          // cells per lane (0: row kernels not used)
     bool rows_win_ = false;     // rows are cut into windows
@@ -751,7 +750,7 @@ public:
             rgeo_ = make_rowgeo(n_[1], n_[2], ROWS_NW * ROWS_RW - 4, o_.rows_kc, nwx, wl);
             rows_blocks_ = 8u * (unsigned)rgeo_.per_xcd;
             pmv_on_ = (o_.forms & UAAMG_FORM_PMV) != 0;
-            pgeo_ = make_rowgeo(n_[1], n_[2], PMV_NW * PMV_RW - 2, o_.rows_kc, nwx, wl);
+            pgeo_ = make_rowgeo(n_[1], n_[2], PMV_NW * PMV_RW - 2, o_.rows_kc, nwx, wl);   // FP32 vectors (FP64: flat)
             pmv_blocks_ = 8u * (unsigned)pgeo_.per_xcd;
         }
     }
@@ -839,7 +838,10 @@ public:
     // is allowed: rows of more than 128 cells
     bool rows_nt(int form) const { return (o_.forms & form) && (rows_cpl_ == 4 || rows_win_); }
     void rows_down0(const T* r, Level& C, const int* skip) {
-        if constexpr (D == 3) {
+        if constexpr (D == 3 && sizeof(T) == 8) {
+            tlaunch(timer_, UAAMG_K_DOWN0, rows_win_ ? k_rows64_down0<true, S> : k_rows64_down0<false, S>, dim3(rows_blocks_), dim3(R64_NW * 64),
+                    stream_, r, (const uint8_t*)nbr0_, g0_, c0d_, rgeo_, C.b, C.g, skip);
+        } else if constexpr (D == 3) {
             if (fr_old_) {   // alpha from the operator's partials; r = r_old - alpha Ap written to r; r.r -> convergence
                 // nontemporal loads of r_old and Ap (last use of both; without
                 // UAAMG_FORM_NT_D plain): 34.5 vs 33.5 solves/s at 256^3 in three paired runs
@@ -869,7 +871,13 @@ public:
         }
     }
     void rows_up0(const T* r, Level& C, T* z, const int* skip) {
-        if constexpr (D == 3) {
+        if constexpr (D == 3 && sizeof(T) == 8) {
+            const MLaunch m = up0_launch();
+            tlaunch(timer_, UAAMG_K_UP0, rows_win_ ? k_rows64_up0<true, S> : k_rows64_up0<false, S>, dim3(rows_blocks_), dim3(R64_NW * 64),
+                    stream_, r, (const uint8_t*)nbr0_, g0_, c0d_, rgeo_, (const S*)C.x, C.g, z, skip);
+            k_zsums_m3<RX0, RY0, PPT0><<<m.grid, 256, 0, stream_>>>(z, r, nbr0_, g0_, m.KC, skip, partials_);
+            if (!fr_) k_fin_zsums<<<1, FIN_THREADS, 0, stream_>>>(partials_, nzp(), ctrl_);
+        } else if constexpr (D == 3) {
             // nontemporal loads of r (without UAAMG_FORM_NT_U plain): 34.6 vs
             // 33.9 solves/s at 256^3 in three paired runs
             const bool unt = rows_nt(UAAMG_FORM_NT_U);
@@ -1052,7 +1060,7 @@ public:
         forms_used_ = 0;
         // the split update needs the fused V-cycle (its level-0 row kernels)
         fr_ = pmv_on_ && !o_.flexible && (gmg_ || (o_.fused && o_.nu_pre == 1 && o_.nu_post == 1 && fused_ok_));
-        pmv_now_ = pmv_on_ && (D == 3 || fr_);   // 2D: with the split update only
+        pmv_now_ = pmv_on_ && (!FLATCG || fr_);   // flat passes: with the split update only
         start(rhs_dev, p_dev, warm, max_iter, tol, pmv_now_);
         const int* skip = &ctrl_->done;
         int it_cap = max_iter;
@@ -1199,7 +1207,7 @@ public:
     }
 
     void iteration(T* x, const int* skip) {
-        if (D == 2 && fr_) { iteration_t2(x, skip); return; }
+        if (FLATCG && fr_) { iteration_t2(x, skip); return; }
         const unsigned fb = flat_blocks(2048);
         const T* pv = p_;        // the p of this iteration's operator and update
         unsigned mb = fb;        // workgroups of the operator launch (its partials)
@@ -1218,7 +1226,7 @@ public:
             // p.Ap partials in their own buffer: the down kernel that sums
             // them writes its r.r partials while other workgroups still read
             // (with the split update it also finishes the level-0 up kernel's z sums)
-            if constexpr (D == 3) {
+            if constexpr (D == 3 && sizeof(T) == 4) {
                 // nontemporal loads of z and p_old (last use of both; without
                 // UAAMG_FORM_NT_P plain): 33.6 vs 33.0 solves/s at 256^3 in three paired runs
                 const bool pnt = rows_nt(UAAMG_FORM_NT_P) && fr_;

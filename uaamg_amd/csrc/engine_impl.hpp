@@ -42,9 +42,9 @@ void Engine<D, T, S, R>::allocate() {
     HIPCHK(hipHostMalloc((void**)&ctrl_host_, sizeof(Ctrl), hipHostMallocDefault));
     // the level-0 vectors in one allocation: r, z, p, Ap, x and, where the CG
     // passes are fused, the second p (GMG / AMG have it in any case, for x of
-    // the coarse levels' way down) and in 3D the second r
+    // the coarse levels' way down) and in 3D with FP32 vectors the second r
     T** vec[] = {&r_, &z_, &p_, &Ap_, &x_, &p2_, &r2_};
-    const int nv = pmv_on_ ? (D == 3 ? 7 : 6) : (gmg_ ? 6 : 5);
+    const int nv = pmv_on_ ? (FLATCG ? 6 : 7) : (gmg_ ? 6 : 5);
     const size_t stride = vec_stride(N4_, margin_);
     T* base = dalloc<T>(nv * stride);
     for (int q = 0; q < nv; q++) *vec[q] = base + q * stride + margin_;

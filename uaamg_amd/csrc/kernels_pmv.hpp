@@ -1,5 +1,5 @@
-// kernels_pmv.hpp -- level-0 search direction and operator in one pass (3D;
-// vectors of type F: float, or double).
+// kernels_pmv.hpp -- level-0 search direction and operator in one pass (3D,
+// FP32 vectors: F = float; FP64: k_t2_pmv).
 //
 // One pass replaces the p update of iteration k-1 and the operator of
 // iteration k (pcg_3d.cpp:116-122 and 94-96):

@@ -1,5 +1,5 @@
-// kernels_rows.hpp -- level-0 V(1,1) kernels in 3D, in the vectors' type F
-// (float, or double for the forms with FP64 vectors).
+// kernels_rows.hpp -- level-0 V(1,1) kernels in 3D for FP32 vectors (F =
+// float; FP64 vectors: kernels_rows64.hpp).
 //
 // The same preconditioner as the reference's level-0 smooth /
 // restrictResidual / prolongateAdd (uaamg_preconditioner_3d.cpp:123-181).
@@ -14,8 +14,7 @@
 //   odd  cells: z = (r + sum_nb c z_nb) / d     (reverse sweep, odd colour)
 //   isolated cells keep x'.
 // These are identities in exact arithmetic; they round differently from the
-// per-pass and march kernels (which keep the reference's order), in FP64 by a
-// few units of its last place (the parity bar of a V-cycle is 1e-12).
+// per-pass and march kernels (which keep the reference's order).
 // Level-0 couplings are 1/h^2 on every face between two fluid interior cells
 // and 0 otherwise, and x is 0 on every non-fluid cell, so the neighbour sums
 // use the per-axis constants.
@@ -67,10 +66,8 @@ struct RowGeo {
     int wl;        // lanes a window owns (the last one: the rest)
 };
 
-// a b + c: one FMA on FP32 vectors; FP64 vectors keep the separate roundings
-// of the flat kernels
+// a b + c in one FMA
 __device__ __forceinline__ float rfma(float a, float b, float c) { return fmaf(a, b, c); }
-__device__ __forceinline__ double rfma(double a, double b, double c) { return a * b + c; }
 
 // Whole-wave shifts by one lane with DPP (wave_shr:1 = 0x138, wave_shl:1 =
 // 0x130; all rows and banks enabled, lanes with no source keep old = 0):

@@ -402,15 +402,20 @@ __global__ __launch_bounds__(512) void k_t2_up0(const VB* __restrict__ b, const 
 // issued before the partials are added: one memory round trip, not three
 // (1024 x 512 FP64: operator 12.2 -> 9.9 us, update 7.9 -> 6.8 us).
 
-// what the operator reads of z or p_old around the vector at c0
-template <typename T>
-struct T2Nb { vec4<T> c, b, t; T l, r; };
-template <typename T>
-__device__ __forceinline__ T2Nb<T> t2_nb(const T* __restrict__ v, long c0, long sx) {
-    T2Nb<T> o;
+// what the operator reads of z or p_old around the vector at c0 (3D: f, k:
+// the planes below and above)
+template <int D, typename T>
+struct T2Nb { vec4<T> c, b, t, f, k; T l, r; };
+template <int D, typename T>
+__device__ __forceinline__ T2Nb<D, T> t2_nb(const T* __restrict__ v, long c0, const Geo& g) {
+    T2Nb<D, T> o;
     o.c = *(const vec4<T>*)(v + c0);
-    o.b = *(const vec4u<T>*)(v + c0 - sx);
-    o.t = *(const vec4u<T>*)(v + c0 + sx);
+    o.b = *(const vec4u<T>*)(v + c0 - g.sx);
+    o.t = *(const vec4u<T>*)(v + c0 + g.sx);
+    if constexpr (D == 3) {
+        o.f = *(const vec4u<T>*)(v + c0 - g.sy);
+        o.k = *(const vec4u<T>*)(v + c0 + g.sy);
+    }
     o.l = v[c0 - 1];
     o.r = v[c0 + 4];
     return o;
@@ -419,7 +424,7 @@ __device__ __forceinline__ T2Nb<T> t2_nb(const T* __restrict__ v, long c0, long 
 // The finish of the z sums, p (written to the other p buffer: neighbours form
 // theirs from p_old) and Ap with its p.Ap partials.  rsold and the first flag
 // are read here and only written by the next launch.
-template <typename T, bool VAR>
+template <int D, typename T, bool VAR>
 __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z, const T* __restrict__ pold, T* __restrict__ pnew,
                                                         T* __restrict__ Ap, const uint8_t* __restrict__ nbr, Geo g,
                                                         Consts<double> c, long N4, Ctrl* ctrl, const double* zp, int nz, double* pap,
@@ -439,7 +444,10 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z,
     const long step = (long)(xcd ? (fv_n >> 3) : fv_n) * FIN_THREADS;
     const long first_v = min(beg, n - 1);          // a thread without a vector loads the last one
     uint32_t w = *(const uint32_t*)(nbr + 4 * first_v);
-    T2Nb<T> zv = t2_nb<T>(z, 4 * first_v, g.sx), pv = t2_nb<T>(pold, 4 * first_v, g.sx);
+    // vectors of the first and the last plane, which hold no fluid cell, load
+    // one whose neighbour planes lie in the array
+    const long first_c = D == 3 ? min(max(4 * first_v, (g.sy + 3) / 4 * 4), (N4 - g.sy - 4) / 4 * 4) : 4 * first_v;
+    T2Nb<D, T> zv = t2_nb<D, T>(z, first_c, g), pv = t2_nb<D, T>(pold, first_c, g);
     if (done) return;
     __shared__ double s_z[3];
     block_sum<3>(tot);
@@ -461,7 +469,7 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z,
         const long c0 = 4 * k;
         if (k != beg) {
             w = *(const uint32_t*)(nbr + c0);
-            if (w & 0x01010101u) { zv = t2_nb<T>(z, c0, g.sx); pv = t2_nb<T>(pold, c0, g.sx); }
+            if (w & 0x01010101u) { zv = t2_nb<D, T>(z, c0, g); pv = t2_nb<D, T>(pold, c0, g); }
         }
         vec4<T> out = (T)0;
         if (w & 0x01010101u) {
@@ -477,13 +485,15 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z,
                 if (!(nb & NB_FLUID)) continue;
                 const double pm = (double)pc[q + 1], vl = (double)pc[q], vr = (double)pc[q + 2];
                 const double vb = (double)at(zv.b[q], pv.b[q]), vt = (double)at(zv.t[q], pv.t[q]);
+                double vf = 0.0, vk = 0.0;
+                if constexpr (D == 3) { vf = (double)at(zv.f[q], pv.f[q]); vk = (double)at(zv.k[q], pv.k[q]); }
                 double o;
                 if constexpr (VAR) {
                     int i = 0, j = 0, kk = 0;
                     if (c.any_dirichlet) coords<2>(g, c0 + q, i, j, kk);
                     o = apply_A_var(i, j, c0 + q, nb, pm, vl, vr, vb, vt, g, c, L);
                 } else {
-                    o = apply_A<2>(c0 + q, nb, pm, vl, vr, vb, vt, 0.0, 0.0, g, c);
+                    o = apply_A<D>(c0 + q, nb, pm, vl, vr, vb, vt, vf, vk, g, c);
                 }
                 const T oq = (T)o;
                 out[q] = oq;

@@ -460,8 +460,8 @@ extern "C" size_t uaamg_bytes_required(const uaamg_grid* g, const uaamg_opts* o)
     const size_t N0 = (size_t)g0.N, N4 = (N0 + 3) / 4 * 4;
     const size_t margin = (size_t)((g0.sx + 8 + 63) / 64) * 64;
     // level-0 vectors r, z, p, Ap, x and the second buffers of the fused CG
-    // kernels (3D, on the level-0 row kernels: p and r; 2D: p, which GMG / AMG
-    // have in any case)
+    // kernels (3D with FP32 vectors, on the level-0 row kernels: p and r; others:
+    // p, which GMG / AMG have in any case)
     int nwx = 1, wl = 64;
     if (v64) Engine<3, double, double>::row_lanes(g0.nx, nwx, wl);
     else Engine<3, float, float>::row_lanes(g0.nx, nwx, wl);
@@ -469,9 +469,9 @@ extern "C" size_t uaamg_bytes_required(const uaamg_grid* g, const uaamg_opts* o)
                               (o->forms & UAAMG_FORM_ROWS) && (o->forms & UAAMG_FORM_PMV)
                         : Engine<2, float, float>::t2_pmv(*o, shape);
     const bool gmg = o->preconditioner == UAAMG_PRECOND_GMG || o->preconditioner == UAAMG_PRECOND_AMG;
-    size_t bytes = N0 + N4 + kRowSlack + 8 + sizeof(uaamg::Ctrl) + (pmv ? (d3 ? 7 : 6) : (gmg ? 6 : 5)) * uaamg::vec_stride((long)N4, (long)margin) * sv;
-    if (pmv && !d3) bytes += (2048 + 64) * 8;
-    if (pmv && d3)   // p.Ap partials; 256 tiles at most where a chunk has 2 planes or rows are narrow
+    size_t bytes = N0 + N4 + kRowSlack + 8 + sizeof(uaamg::Ctrl) + (pmv ? (d3 && !v64 ? 7 : 6) : (gmg ? 6 : 5)) * uaamg::vec_stride((long)N4, (long)margin) * sv;
+    if (pmv && (!d3 || v64)) bytes += (2048 + 64) * 8;
+    if (pmv && d3 && !v64)   // p.Ap partials; 256 tiles at most where a chunk has 2 planes or rows are narrow
         bytes += (size_t)(8 * ((std::max(256L, (long)nwx * ((g0.ny + 15) / 16) * ((g0.nz + 3) / 4)) + 7) / 8) + 64) * 8;
     long maxb = std::max<long>(cells_launch(g0, g->dim).nblocks(), 2048);
     for (size_t l = 1; l < shape.size(); l++) {
