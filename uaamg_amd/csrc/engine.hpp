@@ -747,7 +747,7 @@ public:
                 rtab_.any_dirichlet |= on;
             }
             ptab_.any_dirichlet = rtab_.any_dirichlet;
-            rgeo_ = make_rowgeo(n_[1], n_[2], ROWS_NW * ROWS_RW - 4, o_.rows_kc, nwx, wl);
+            rgeo_ = make_rowgeo(n_[1], n_[2], (sizeof(T) == 8 ? R64_NW * R64_RW : ROWS_NW * ROWS_RW) - 4, o_.rows_kc, nwx, wl);
             rows_blocks_ = 8u * (unsigned)rgeo_.per_xcd;
             pmv_on_ = (o_.forms & UAAMG_FORM_PMV) != 0;
             pgeo_ = make_rowgeo(n_[1], n_[2], PMV_NW * PMV_RW - 2, o_.rows_kc, nwx, wl);   // FP32 vectors (FP64: flat)

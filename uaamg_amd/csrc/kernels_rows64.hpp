@@ -1,7 +1,7 @@
 // kernels_rows64.hpp -- level-0 V(1,1) kernels in 3D for FP64 vectors.
 //
 // The mapping of kernels_rows.hpp (whole rows or windows of two cells a lane,
-// 10 waves of 2 rows, a march along z), the arithmetic and order per cell of
+// waves of 2 rows, a march along z), the arithmetic and order per cell of
 // the per-pass and march kernels (and so the reference's smooth /
 // restrictResidual / prolongateAdd, uaamg_preconditioner_3d.cpp:123-181), bit
 // for bit: an FP64 solve of some ten iterations carries a changed last digit
@@ -15,15 +15,17 @@
 // A lane keeps d (< 0: not fluid) of its cells on four planes; the rows that
 // waves share go through LDS, one slot per plane of the window and colour.
 //
-// 256 x 128 x 128 (three windows): down 62 -> 36 us, up 70 -> 26 and 15 for the
-// sums; 128 x 64 x 64: 25 -> 13, 30 -> 10 and 6.
+// Eight waves a workgroup, two per SIMD: with ten (168 VGPRs) the down kernel
+// spilled 47 registers (36 us at 256 x 128 x 128, 13 at 128 x 64 x 64).  256 x 128
+// x 128 (three windows): down 62 -> 26 us, up 70 -> 25 and 15 for the sums; 128 x
+// 64 x 64: 25 -> 8.1, 30 -> 8.5 and 6.
 #pragma once
 #include "kernels_march.hpp"
 #include "kernels_rows.hpp"
 
 namespace uaamg {
 
-constexpr int R64_NW = 10, R64_RW = 2, R64_CPL = 2;
+constexpr int R64_NW = 8, R64_RW = 2, R64_CPL = 2;
 
 struct Row64LDS {
     double d[64];                         // d per neighbour pattern, without walls

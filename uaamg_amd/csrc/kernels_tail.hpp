@@ -31,7 +31,7 @@
 // Measured against the form before (records of all 1024 threads loaded,
 // indices by division, four barriers a level, division in the chain): 16^3 to
 // 4^3 FP32 19.6 -> 15.9 us, 18 x 12 x 7 FP32
-// 13.4 -> 9.0, 16 x 8 x 8 FP64 24.0 -> 13.9, 2D 32 x 16 FP64 15.2 -> 13.8, 12 2D
+// 13.4 -> 9.0, 16 x 8 x 8 FP64 24.0 -> 12.2, 2D 32 x 16 FP64 15.2 -> 13.3, 12 2D
 // grids of up to 5 levels 20.7 -> 16.3.  What is left is the 21 coarsest passes
 // (a chain of LDS reads and additions) and one memory round trip.
 #pragma once
@@ -279,10 +279,17 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     TailRecV<D, CT> R0[TAIL_MAXP], R1, R2, R3, R4;
 #pragma unroll
     for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<D, CT>(R0[v], Ag.rec, tail_slot(0, v), tid + TAIL_THREADS * v, np[0], tid);
+    // FP64 (twice the registers): the levels below the second are loaded after
+    // the first is done, and the first again for its way up (16 x 8 x 8: 13.9 ->
+    // 12.2 us; a fourth 2D level still spilled 92 registers, 28 us)
+    constexpr bool LATE = sizeof(CT) == 8;
     tail_issue_rec<D, CT>(R1, Ag.rec, tail_slot(1, 0), tid, np[1], tid);
-    if constexpr (NLMAX > 2) tail_issue_rec<D, CT>(R2, Ag.rec, tail_slot(2, 0), tid, np[2], tid);
-    if constexpr (NLMAX > 3) tail_issue_rec<D, CT>(R3, Ag.rec, tail_slot(3, 0), tid, np[3], tid);
-    if constexpr (NLMAX > 4) tail_issue_rec<D, CT>(R4, Ag.rec, tail_slot(4, 0), tid, np[4], tid);
+    auto issue_rest = [&]() {
+        if constexpr (NLMAX > 2) tail_issue_rec<D, CT>(R2, Ag.rec, tail_slot(2, 0), tid, np[2], tid);
+        if constexpr (NLMAX > 3) tail_issue_rec<D, CT>(R3, Ag.rec, tail_slot(3, 0), tid, np[3], tid);
+        if constexpr (NLMAX > 4) tail_issue_rec<D, CT>(R4, Ag.rec, tail_slot(4, 0), tid, np[4], tid);
+    };
+    if constexpr (!LATE) issue_rest();
     constexpr int BMAX = sizeof(CT) == 8 ? TAIL_LDS_BYTES / 24 / TAIL_THREADS : TAIL_BMAX;
     S bt[BMAX];
     const int N0 = Ag.N0;
@@ -328,12 +335,18 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
         if ((tid & (WAVE - 1)) == 0) s_rr[tid / WAVE] = rs;
     }
     TailPair<CT> P0[TAIL_MAXP], P1[1], P2[1], P3[1], P4[1];
+    auto pairs_first = [&]() {
 #pragma unroll
-    for (int v = 0; v < TAIL_MAXP; v++) tail_pair_from_rec<D, CT>(P0[v], R0[v], tid + TAIL_THREADS * v, np[0]);
+        for (int v = 0; v < TAIL_MAXP; v++) tail_pair_from_rec<D, CT>(P0[v], R0[v], tid + TAIL_THREADS * v, np[0]);
+    };
+    pairs_first();
     tail_pair_from_rec<D, CT>(P1[0], R1, tid, np[1]);
-    if constexpr (NLMAX > 2) tail_pair_from_rec<D, CT>(P2[0], R2, tid, np[2]);
-    if constexpr (NLMAX > 3) tail_pair_from_rec<D, CT>(P3[0], R3, tid, np[3]);
-    if constexpr (NLMAX > 4) tail_pair_from_rec<D, CT>(P4[0], R4, tid, np[4]);
+    auto pairs_rest = [&]() {
+        if constexpr (NLMAX > 2) tail_pair_from_rec<D, CT>(P2[0], R2, tid, np[2]);
+        if constexpr (NLMAX > 3) tail_pair_from_rec<D, CT>(P3[0], R3, tid, np[3]);
+        if constexpr (NLMAX > 4) tail_pair_from_rec<D, CT>(P4[0], R4, tid, np[4]);
+    };
+    if constexpr (!LATE) pairs_rest();
     __syncthreads();
     if (test) {   // every thread takes the same decision from the same values, thread 0 stores it
         double tot = s_rr[0];
@@ -406,6 +419,7 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     }
     // down
     if (nl > 1) level_down(P0, P1, 0);
+    if constexpr (LATE) { issue_rest(); pairs_rest(); }
     if constexpr (NLMAX > 2) { if (nl > 2) level_down(P1, P2, 1); }
     if constexpr (NLMAX > 3) { if (nl > 3) level_down(P2, P3, 2); }
     if constexpr (NLMAX > 4) { if (nl > 4) level_down(P3, P4, 3); }
@@ -418,6 +432,13 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     // up
     if constexpr (NLMAX > 4) { if (nl > 4) level_up(P3, 3); }
     if constexpr (NLMAX > 3) { if (nl > 3) level_up(P2, 2); }
+    if constexpr (LATE) {
+        if (nl > 1) {
+#pragma unroll
+            for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<D, CT>(R0[v], Ag.rec, tail_slot(0, v), tid + TAIL_THREADS * v, np[0], tid);
+            pairs_first();
+        }
+    }
     if constexpr (NLMAX > 2) { if (nl > 2) level_up(P1, 1); }
     if (nl > 1) level_up(P0, 0);
     // a thread stores its own cells (its last pass wrote the odd ones, the
