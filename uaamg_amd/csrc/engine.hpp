@@ -557,11 +557,14 @@ public:
         if (!tail_first_) return;
         targs_.nl = nl - tail_first_;
         int off = 0;
+        long rec = 0;
         for (int q = 0; q < targs_.nl; q++) {
             const Level& L = lv_[tail_first_ + q];
             targs_.g[q] = L.g;
             targs_.coef[q] = L.coef;
-            targs_.np[q] = ((L.g.nx + 1) / 2) * L.g.ny * (D == 3 ? L.g.nz : 1);
+            targs_.np[q] = tail_pairs(L.g);
+            targs_.rq[q] = (int)(rec / 16);
+            rec += tail_rec_bytes<SC>(targs_.np[q]);
             targs_.xo[q] = off; off += (int)L.g.N;
             targs_.bo[q] = off; off += (int)L.g.N;
         }
@@ -571,9 +574,8 @@ public:
         targs_.b = lv_[tail_first_].b;
         targs_.x = lv_[tail_first_].x;
         targs_.skip = nullptr;
-        // per-thread stencil records (filled by tail_build once the level
-        // records exist)
-        tail_rec_ = dalloc<char>((size_t)tail_rec_bytes<SC>(TAIL_MAXP + targs_.nl - 1));
+        // the pairs' records (filled by tail_build once the level records exist)
+        tail_rec_ = dalloc<char>((size_t)rec);
         targs_.rec = tail_rec_;
     }
     char* tail_rec_ = nullptr;

@@ -47,14 +47,15 @@ constexpr int TAIL_BMAX = 8;     // b elements per thread of the first tail leve
 
 // A pair's record: 16 values (d, 1/d, xp, xm, yp, ym, zp, zm, each of the even
 // and the odd cell; 1/d = 0 where no pass updates the cell) and 4 indices, in
-// 16-byte quads stored [slot][quad][thread], so that every quad load of a
-// wave is one contiguous 1 KiB read.  Slots: TAIL_MAXP on the first level, 1
-// on every other.
+// 16-byte quads stored [level][quad][pair], a level's pairs padded to whole
+// waves, so that every quad load of a wave is one contiguous 1 KiB read.
 template <typename CT> struct TailRec;
 template <> struct TailRec<float> { static constexpr int NV = 4, NQ = 5, PER = 4; using Q = float4; };
 template <> struct TailRec<double> { static constexpr int NV = 8, NQ = 9, PER = 2; using Q = double2; };
-template <typename CT> constexpr long tail_rec_bytes(int nslots) { return (long)nslots * TailRec<CT>::NQ * TAIL_THREADS * 16; }
-__host__ __device__ constexpr int tail_slot(int l, int v) { return l == 0 ? v : TAIL_MAXP + l - 1; }
+__host__ __device__ constexpr int tail_rec_stride(int np) { return (np + 63) / 64 * 64; }
+template <typename CT> constexpr long tail_rec_bytes(int np) { return (long)tail_rec_stride(np) * TailRec<CT>::NQ * 16; }   // of a level
+// pairs of a level (D = 3: nz planes; 2D levels have nz = 1)
+inline int tail_pairs(const Geo& g) { return ((g.nx + 1) / 2) * g.ny * g.nz; }
 
 template <typename C4>
 struct TailArgs {
@@ -71,7 +72,8 @@ struct TailArgs {
     int nl;                        // levels in the tail; the last one is the coarsest
     int ro;                        // LDS offset of the residual scratch (behind x and b of every level)
     int N0;                        // padded cells of the first one
-    int np[TAIL_MAXL];             // pairs per level
+    int np[TAIL_MAXL];             // pairs per level (0 past nl)
+    int rq[TAIL_MAXL];             // a level's first quad in rec
     int npass;                     // coarsest passes (2 * sweeps + 1)
     int xo[TAIL_MAXL], bo[TAIL_MAXL];   // LDS offsets (elements) of x and b per level
     Geo g[TAIL_MAXL];
@@ -95,17 +97,18 @@ struct TailRecV {
     int4 ix;
 };
 template <int D, typename CT>
-__device__ __forceinline__ void tail_issue_rec(TailRecV<D, CT>& R, const void* rec, int slot, int p, int np, int t) {
+__device__ __forceinline__ void tail_issue_rec(TailRecV<D, CT>& R, const void* rec, int rq, int p, int np) {
     using Q = typename TailRec<CT>::Q;
-    constexpr int NQ = TailRec<CT>::NQ, NV = TailRec<CT>::NV;
-    const Q* base = static_cast<const Q*>(rec) + (long)slot * NQ * TAIL_THREADS + t;
+    constexpr int NV = TailRec<CT>::NV;
+    const Q* base = static_cast<const Q*>(rec) + rq + p;
+    const int st = tail_rec_stride(np);
     R.ix = int4{0, -1, 0, 0};
 #pragma unroll
     for (int q = 0; q < NV; q++) R.v[q] = Q{};
     if (p < np) {
 #pragma unroll
-        for (int q = 0; q < (D == 3 ? NV : NV * 3 / 4); q++) R.v[q] = gload(base + q * TAIL_THREADS);   // 2D: no z couplings
-        R.ix = __builtin_bit_cast(int4, gload(base + NV * TAIL_THREADS));
+        for (int q = 0; q < (D == 3 ? NV : NV * 3 / 4); q++) R.v[q] = gload(base + q * st);   // 2D: no z couplings
+        R.ix = __builtin_bit_cast(int4, gload(base + NV * st));
     }
 }
 template <int D, typename CT>
@@ -131,7 +134,8 @@ __device__ __forceinline__ void tail_pair_from_rec(TailPair<CT>& P, const TailRe
     P.ch = R.ix.z;
 }
 
-// Set-up: the records of every slot of the tail (one workgroup per slot).
+// Set-up: the records of the tail (TAIL_MAXP workgroups for the first level, one
+// for every other).
 template <int D, typename CT, typename C4>
 __global__ __launch_bounds__(TAIL_THREADS) void k_tail_records(TailArgs<C4> A, CT* __restrict__ rec) {
     const int slot = blockIdx.x;
@@ -145,7 +149,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail_records(TailArgs<C4> A, C
     const int i0 = 2 * (p % npx) + 1, j = (p / npx) % g.ny + 1, k = (D == 3) ? p / (npx * g.ny) + 1 : 0;
     const int id0 = (int)gidx(g, i0, j, k), par0 = (i0 + j + k) & 1;
     const bool ok1 = i0 + 1 <= g.nx;
-    constexpr int PER = TailRec<CT>::PER, NQ = TailRec<CT>::NQ, NV = TailRec<CT>::NV;
+    constexpr int PER = TailRec<CT>::PER, NV = TailRec<CT>::NV;
     CT f[NV * PER];
 #pragma unroll
     for (int c = 0; c < 2; c++) {   // cell of colour c
@@ -158,11 +162,11 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail_records(TailArgs<C4> A, C
         f[4 + c] = s.xp; f[6 + c] = s.xm; f[8 + c] = s.yp; f[10 + c] = s.ym;
         f[12 + c] = D == 3 ? s.zp : CT(0); f[14 + c] = D == 3 ? s.zm : CT(0);
     }
-    const long at = (long)slot * NQ * TAIL_THREADS + t;
+    const long at = A.rq[l] + p, st = tail_rec_stride(A.np[l]);
 #pragma unroll
     for (int q = 0; q < NV; q++)
 #pragma unroll
-        for (int e = 0; e < PER; e++) rec[(at + (long)q * TAIL_THREADS) * PER + e] = f[q * PER + e];
+        for (int e = 0; e < PER; e++) rec[(at + q * st) * PER + e] = f[q * PER + e];
     int4 ix;
     ix.x = id0;
     ix.y = -1;
@@ -173,7 +177,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail_records(TailArgs<C4> A, C
     }
     ix.z = l > 0 ? (int)gidx(A.g[l - 1], 2 * i0 - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0) : 0;
     ix.w = par0 | (ok1 ? 2 : 0);
-    reinterpret_cast<int4*>(rec)[at + (long)NV * TAIL_THREADS] = ix;
+    reinterpret_cast<int4*>(rec)[at + NV * st] = ix;
 }
 
 // One RBGS colour on the owned pairs of one level.
@@ -278,16 +282,16 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     // checked on the host)
     TailRecV<D, CT> R0[TAIL_MAXP], R1, R2, R3, R4;
 #pragma unroll
-    for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<D, CT>(R0[v], Ag.rec, tail_slot(0, v), tid + TAIL_THREADS * v, np[0], tid);
+    for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<D, CT>(R0[v], Ag.rec, Ag.rq[0], tid + TAIL_THREADS * v, np[0]);
     // FP64 (twice the registers): the levels below the second are loaded after
     // the first is done, and the first again for its way up (16 x 8 x 8: 13.9 ->
     // 12.2 us; a fourth 2D level still spilled 92 registers, 28 us)
     constexpr bool LATE = sizeof(CT) == 8;
-    tail_issue_rec<D, CT>(R1, Ag.rec, tail_slot(1, 0), tid, np[1], tid);
+    tail_issue_rec<D, CT>(R1, Ag.rec, Ag.rq[1], tid, np[1]);
     auto issue_rest = [&]() {
-        if constexpr (NLMAX > 2) tail_issue_rec<D, CT>(R2, Ag.rec, tail_slot(2, 0), tid, np[2], tid);
-        if constexpr (NLMAX > 3) tail_issue_rec<D, CT>(R3, Ag.rec, tail_slot(3, 0), tid, np[3], tid);
-        if constexpr (NLMAX > 4) tail_issue_rec<D, CT>(R4, Ag.rec, tail_slot(4, 0), tid, np[4], tid);
+        if constexpr (NLMAX > 2) tail_issue_rec<D, CT>(R2, Ag.rec, Ag.rq[2], tid, np[2]);
+        if constexpr (NLMAX > 3) tail_issue_rec<D, CT>(R3, Ag.rec, Ag.rq[3], tid, np[3]);
+        if constexpr (NLMAX > 4) tail_issue_rec<D, CT>(R4, Ag.rec, Ag.rq[4], tid, np[4]);
     };
     if constexpr (!LATE) issue_rest();
     constexpr int BMAX = sizeof(CT) == 8 ? TAIL_LDS_BYTES / 24 / TAIL_THREADS : TAIL_BMAX;
@@ -435,7 +439,7 @@ __device__ __forceinline__ void d_tail(const TailArgs<C4>& Ag, bool test) {
     if constexpr (LATE) {
         if (nl > 1) {
 #pragma unroll
-            for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<D, CT>(R0[v], Ag.rec, tail_slot(0, v), tid + TAIL_THREADS * v, np[0], tid);
+            for (int v = 0; v < TAIL_MAXP; v++) tail_issue_rec<D, CT>(R0[v], Ag.rec, Ag.rq[0], tid + TAIL_THREADS * v, np[0]);
             pairs_first();
         }
     }

@@ -497,10 +497,11 @@ extern "C" size_t uaamg_bytes_required(const uaamg_grid* g, const uaamg_opts* o)
         int lt;
         if (g->dim == 3) lt = l64 ? Engine<3, double, double>::choose_tail(shape) : Engine<3, float, float>::choose_tail(shape);
         else lt = l64 ? Engine<2, double, double>::choose_tail(shape) : Engine<2, float, float>::choose_tail(shape);
-        if (lt > 0) {
-            const int nslots = uaamg::TAIL_MAXP + (int)shape.size() - lt - 1;
-            bytes += (size_t)(l64 ? uaamg::tail_rec_bytes<double>(nslots) : uaamg::tail_rec_bytes<float>(nslots));
-        }
+        if (lt > 0)
+            for (size_t l = lt; l < shape.size(); l++) {
+                const int np = uaamg::tail_pairs(shape[l]);
+                bytes += (size_t)(l64 ? uaamg::tail_rec_bytes<double>(np) : uaamg::tail_rec_bytes<float>(np));
+            }
     }
     return bytes;
 }
