@@ -118,9 +118,25 @@ __device__ __forceinline__ int n_blocks() { return gridDim.x * gridDim.y * gridD
 __device__ __forceinline__ int lin_thread() { return threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z); }
 __device__ __forceinline__ int n_threads() { return blockDim.x * blockDim.y * blockDim.z; }
 
+// v of lane l + N within a row of 16 lanes (DPP row_shl:N; 0 past the row)
+template <int N>
+__device__ __forceinline__ double row_down(double v) {
+    struct I2 { int a, b; } x = __builtin_bit_cast(I2, v);
+    x.a = __builtin_amdgcn_update_dpp(0, x.a, 0x100 + N, 0xF, 0xF, false);
+    x.b = __builtin_amdgcn_update_dpp(0, x.b, 0x100 + N, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, x);
+}
+// Sum of the wave in lane 0: the tree v += v of lane + 32, 16, 8, 4, 2, 1.  The
+// last four steps stay within a row of lanes and are register moves; through
+// the LDS unit, as the first two, they cost a level-0 up kernel of many small
+// tiles (three sums of eight waves each) a quarter of its time.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_down(v, o, WAVE);
+    v += __shfl_down(v, 32, WAVE);
+    v += __shfl_down(v, 16, WAVE);
+    v += row_down<8>(v);
+    v += row_down<4>(v);
+    v += row_down<2>(v);
+    v += row_down<1>(v);
     return v;
 }
 
