@@ -15,7 +15,7 @@
 //   * two barriers per launch, one for each colour.
 // The march kernels that ran here before went through the level row by row
 // with four barriers a row.  At 1024 x 512 FP64: down 11.9 -> 6.1 us, level-0 up
-// 13.2 -> 11.0, the four coarse levels above the tail 5.5 -> 4.0 each way (a
+// 13.2 -> 9.3, the four coarse levels above the tail 5.5 -> 4.0 each way (a
 // launch with nothing in it takes 2.2); with the fused CG passes 17 launches
 // and 108 us per iteration became 11 and 80.
 #pragma once
