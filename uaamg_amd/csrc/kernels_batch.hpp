@@ -141,8 +141,8 @@ __global__ __launch_bounds__(256) void kb_update(BGrid<S>* G, const BItem* items
 // The finish of the operator (alpha, breakdown), x += alpha p, r -= alpha Ap
 // and the r.r partials: kb_fin_matvec and kb_update in one launch.  Every
 // workgroup adds its grid's p.Ap partials in the finish kernel's order; the
-// grid's first one stores the scalars and rsold for the next beta, which no
-// workgroup of this launch reads.  With the finish of the z sums in
+// grid's first one stores the scalars, rsold for the next beta and a
+// breakdown (Ctrl::brk), which no workgroup of this launch reads.  With the finish of the z sums in
 // kb_pupdate_f and the convergence test in the tail, an iteration has three
 // launches of one workgroup per grid less (4.2 to 4.7 us each).
 template <typename S>
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(FIN_THREADS) void kb_update_f(BGrid<S>* G, const BI
     const BItem it = items[blockIdx.x];
     const BGrid<S>& d = G[it.g];
     Ctrl* c = d.ctrl;
-    const int done = c->done, iter = c->iter;
+    const int done = c->done;
     const double rz = c->rz;
     double tot[1] = {0.0};
     for (int k = threadIdx.x; k < d.flat_cnt; k += FIN_THREADS) tot[0] += d.pap[k];
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(FIN_THREADS) void kb_update_f(BGrid<S>* G, const BI
     const double alpha = rz / pAp;
     if (it.a == 0 && threadIdx.x == 0) {
         c->pAp = pAp;
-        if (!ok) { c->done = 1; c->status = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE; c->iter = iter + 1; }
+        if (!ok) c->brk = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE;
         c->alpha = c->xalpha = ok ? alpha : 0.0;
         c->rsold = rz;
         c->first = 0;
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(FIN_THREADS) void kb_pupdate_f(BGrid<S>* G, const B
         c->mean_z = mean; c->rz = rz; c->beta = beta;
         if (!isfinite(rz)) { c->done = 1; c->status = ST_NONFINITE; }
     }
-    if (!isfinite(rz)) return;
+    if (!isfinite(rz)) return;   // as in k_t2_pmv
     d_pupdate_a<float>(d.p, d.z, d.nbr0, d.N4, mean, beta, it.a, it.b);
 }
 template <typename S>

@@ -462,7 +462,9 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z,
         ctrl->mean_z = mean; ctrl->rz = rz; ctrl->beta = beta;
         if (!isfinite(rz)) { ctrl->done = 1; ctrl->status = ST_NONFINITE; }
     }
-    if (!isfinite(rz)) return;   // the whole solve stops; the launches after this one see done
+    // the whole solve stops: the launches after this one see done, and what a
+    // workgroup that saw it half way wrote to p and Ap is read by none
+    if (!isfinite(rz)) return;
     auto at = [&](T zz, T pp) { return (T)(((double)zz - mean) + beta * (double)pp); };
     double v[1] = {0.0};
     for (long k = beg; k < end; k += step) {
@@ -508,13 +510,14 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z,
 }
 
 // The operator's finish (alpha, breakdown), x += alpha p, r -= alpha Ap and
-// the r.r partials.  Workgroup 0 stores the scalars and rsold for the next
-// beta; no workgroup of this launch reads those.
+// the r.r partials.  Workgroup 0 stores the scalars, rsold for the next beta
+// and a breakdown for the convergence test (Ctrl::brk); no workgroup of this
+// launch reads those.
 template <typename T>
 __global__ __launch_bounds__(FIN_THREADS) void k_t2_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p,
                                                            const T* __restrict__ Ap, const uint8_t* __restrict__ nbr, long N4,
                                                            int nvb, double* rr, const double* pap, int npap, Ctrl* ctrl) {
-    const int done = ctrl->done, iter = ctrl->iter;
+    const int done = ctrl->done;
     const double rz = ctrl->rz;
     double tot[1] = {0.0};
     for (int k = threadIdx.x; k < npap; k += FIN_THREADS) tot[0] += pap[k];
@@ -535,7 +538,7 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_update(T* __restrict__ x, T*
     const double alpha = rz / pAp;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctrl->pAp = pAp;
-        if (!ok) { ctrl->done = 1; ctrl->status = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE; ctrl->iter = iter + 1; }
+        if (!ok) ctrl->brk = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE;
         ctrl->alpha = ctrl->xalpha = ok ? alpha : 0.0;
         ctrl->rsold = rz;
         ctrl->first = 0;
