@@ -10,7 +10,7 @@
 //   partial sums of p_new . Ap             (deterministic, per workgroup)
 // p_old and p_new are separate buffers: a workgroup recomputes p_new on its
 // halo row and planes from z and p_old, so no workgroup reads what another
-// one writes.  p_new is k_pupdate's formula (in F); the operator is k_matvec_dot's
+// one writes.  p_new is k_pupdate's formula (in RowCG's arithmetic); the operator is k_matvec_dot's
 // (apply_A) in the stencil form of the row kernels: p_new is 0 on every
 // non-fluid cell, so a face to a solid cell or a Neumann wall drops out of
 // both d and the sum, and a Dirichlet wall face adds 2/h^2 to d (apply_A's
@@ -109,10 +109,11 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
         if (threadIdx.x == 0) { s_zs[0] = zs[0]; s_zs[1] = zs[1]; s_zs[2] = zs[2]; }
     }
     __syncthreads();
-    // FP32 vectors: the p update runs in FP32 (one FMA) with the FP64 scalars
-    // rounded once: it differs from k_pupdate's FP64 form by the rounding of
-    // the scalars, far below the FP32 storage of the vectors
-    F mean, beta;
+    // A = FP32: the p update is one FMA with the FP64 scalars rounded once: it
+    // differs from k_pupdate's FP64 form by the rounding of the scalars, far
+    // below the FP32 storage of the vectors
+    using A = RowCG<CPL, WIN, F>;
+    A mean, beta;
     if constexpr (FZ) {
         const double sz = s_zs[0], srz = s_zs[1], sr = s_zs[2];
         const double m = (ctrl->project && ctrl->count > 0) ? sz / ctrl->count : 0.0;
@@ -124,9 +125,9 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
             if (!isfinite(rz)) { ctrl->done = 1; ctrl->status = ST_NONFINITE; }
         }
         if (!isfinite(rz)) return;   // the whole solve stops; the down kernel sees done
-        mean = (F)m; beta = (F)b;
+        mean = (A)m; beta = (A)b;
     } else {
-        mean = (F)ctrl->mean_z; beta = (F)ctrl->beta;
+        mean = (A)ctrl->mean_z; beta = (A)ctrl->beta;
     }
 
     if (active) {
@@ -150,7 +151,7 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
                     const uint8_t nb = pin ? pfn[PB][t][q] : (uint8_t)0;
                     NB[S][t][q] = nb;
                     PN[S][t][q] = (nb & NB_FLUID)
-                        ? rfma(beta, pfp[PB][t][q], pfz[PB][t][q] - mean) : F(0);
+                        ? (F)rfma(beta, (A)pfp[PB][t][q], (A)pfz[PB][t][q] - mean) : F(0);
                 }
             // the last plane to enter is last + 1 (upwards) or m0 - 1 (downwards);
             // beyond it the loads repeat that cached plane (no memory traffic), so
@@ -192,7 +193,7 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
                     const F el = lane_from_left(PN[S1][t][CPL - 1]);
                     const F er = lane_from_right(PN[S1][t][0]);
                     F out[CPL];
-                    F pap = F(0);   // the row's p.Ap in F, accumulated in FP64
+                    A pap = A(0);   // the row's p.Ap, accumulated in FP64
                     sfor<CPL>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
                         const F vc = PN[S1][t][q];
@@ -207,7 +208,7 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
                                          + K.idz2 * ((double)PN[S2][t][q] + (double)PN[S][t][q]);
                         const bool fl = nb & NB_FLUID;
                         const F o = fl ? (F)(d * (double)vc - sum) : F(0);
-                        pap = rfma(th.okw[q] ? vc : F(0), o, pap);
+                        pap = rfma((A)(th.okw[q] ? vc : F(0)), (A)o, pap);
                         out[q] = o;
                     });
                     if (th.tile_row[t]) acc[0] += (double)pap;

@@ -68,6 +68,17 @@ struct RowGeo {
 
 // a b + c in one FMA
 __device__ __forceinline__ float rfma(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double rfma(double a, double b, double c) { return fma(a, b, c); }
+
+// Arithmetic of the CG work that the level-0 row kernels take over (p, r and
+// the dot products of FP32 vectors).  Whole rows and their narrow windows form
+// p and r in one FP32 FMA with FP32 scalars and add a lane's products in FP32
+// before the FP64 sum.  Rows of more than 256 cells (windows of four cells a
+// lane) do it all in FP64, as the flat passes that such grids have with the
+// fused passes switched off (512 x 256 x 256 35.0 -> 36.8 ms a solve for it,
+// 300^3 51.6 -> 57.4; on march kernels and flat passes 57 and 80).
+template <int CPL, bool WIN, typename F>
+using RowCG = std::conditional_t<WIN && CPL == 4, double, F>;
 
 // Whole-wave shifts by one lane with DPP (wave_shr:1 = 0x138, wave_shl:1 =
 // 0x130; all rows and banks enabled, lanes with no source keep old = 0):
@@ -301,7 +312,8 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
         return;
     }
     __shared__ RowLDS<CPL, NW, RW, F> L;
-    F alpha = F(0);   // FP32: r update in FP32 (one FMA), as in k_rows_pmv
+    using A = RowCG<CPL, WIN, F>;
+    A alpha = A(0);
     if constexpr (FR) {
         __shared__ double s_pap;
         double tot[1];
@@ -323,7 +335,7 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
             c->first = 0;
         }
         if (!ok) return;   // the whole solve stops; the finish after this kernel sees done
-        alpha = (F)(u.ctrl->rz / pAp);
+        alpha = (A)(u.ctrl->rz / pAp);
     }
     if (tile >= rg.ntiles) {   // the whole workgroup leaves together
         if constexpr (FR) { double z0[1] = {0.0}; block_store<1>(z0, u.partials); }
@@ -386,13 +398,13 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
             const bool pin = P >= th.m0 && P <= th.last;
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
-                F rs = F(0);   // the row's r.r in F, accumulated in FP64
+                A rs = A(0);   // the row's r.r, accumulated in FP64
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     const bool fl = pfn[PB][t][q] & NB_FLUID;
-                    const F rn = fl ? rfma(-alpha, pfa[PB][t][q], pfr[PB][t][q]) : F(0);
+                    const F rn = fl ? (F)rfma(-alpha, (A)pfa[PB][t][q], (A)pfr[PB][t][q]) : F(0);
                     pfr[PB][t][q] = rn;
-                    rs = rfma(th.okw[q] ? rn : F(0), rn, rs);
+                    rs = rfma((A)(th.okw[q] ? rn : F(0)), (A)rn, rs);
                 });
                 if (pin && th.tile_row[t]) rr[0] += (double)rs;
                 if (pin && th.tile_row[t]) {
@@ -658,12 +670,13 @@ __device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_
                         }
                     });
                     if (th.tile_row[t]) {
-                        // the row's CPL cells summed in F (FP32: one FMA each),
-                        // the row sums accumulated in FP64
-                        F s0 = F(0), s1 = F(0), s2 = F(0);
+                        // the row's CPL cells summed (FP32: one FMA each), the
+                        // row sums accumulated in FP64
+                        using A = RowCG<CPL, WIN, F>;
+                        A s0 = A(0), s1 = A(0), s2 = A(0);
                         sfor<CPL>([&](auto qc) {
                             constexpr int q = decltype(qc)::value;
-                            const F zv = th.okw[q] ? X[S2][t][q] : F(0), rv = th.okw[q] ? Rq[S2][t][q] : F(0);
+                            const A zv = (A)(th.okw[q] ? X[S2][t][q] : F(0)), rv = (A)(th.okw[q] ? Rq[S2][t][q] : F(0));
                             s0 += zv;
                             s1 = rfma(rv, zv, s1);
                             s2 += rv;
