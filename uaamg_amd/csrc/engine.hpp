@@ -493,7 +493,16 @@ public:
     double alg_bytes_of(int iters) const { return alg_bytes(iters); }
     long padded_cells() const { return g0_.N; }
     long n4() const { return N4_; }
-    int rows_cpl() const { return rows_win_ ? 0 : rows_cpl_; }   // of the batched row kernels (whole rows only)
+    // Cells per lane of the batched row kernels, which have whole rows only (0:
+    // the march kernels).  narrow_rows() is about a grid that has the chip to
+    // itself: members of 129 to 256 cells keep whole rows of four cells a lane
+    // (160 x 64 x 64, 256 x 64 x 64 and 160 x 80 x 80 in one batch, FP32: 162 us an
+    // iteration on the march kernels, 120 on these; BF16 levels 188 and 131).
+    int rows_cpl() const {
+        int nwx, wl;
+        const int cpl = row_lanes(n_[0], nwx, wl);
+        return rows_cpl_ && nwx == 1 ? cpl : 0;
+    }
     int tail_first() const { return tail_first_; }
     // fill the batch descriptor (ctrl: the batch's scalar slot for this grid)
     void fill_batch(BGrid<S>& d, Ctrl* ctrl) const {
