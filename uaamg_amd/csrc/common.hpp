@@ -90,10 +90,11 @@ struct Ctrl {
     double xalpha;         // alpha of this iteration's x update; 0 when the operator finish found the solve stopped
     double xa[2];          // the same for the split update's x pass, per p buffer: the x pass of one
                            // iteration may still run while the next iteration forms its alpha
+    // A breakdown in a CG update that other workgroups of the launch still run
+    // is status alone: a wave that started late would see done and leave, while
+    // the others of its workgroup add sums that need it.  The convergence test
+    // sets done from it.
     int iter, max_iter, done, status, first, tol_mode, project, flexible;
-    int brk;               // ST_* of a breakdown that this iteration's CG update found (0: none).  Not done itself:
-                           // a wave of that launch that started late would see it and leave, while the others of
-                           // its workgroup add sums that need it; the convergence test sets done from it
     double* hist;          // optional per-iteration r.r history (nullptr: off)
 };
 

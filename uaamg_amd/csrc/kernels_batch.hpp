@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void kb_update(BGrid<S>* G, const BItem* items
 // and the r.r partials: kb_fin_matvec and kb_update in one launch.  Every
 // workgroup adds its grid's p.Ap partials in the finish kernel's order; the
 // grid's first one stores the scalars, rsold for the next beta and a
-// breakdown (Ctrl::brk), which no workgroup of this launch reads.  With the finish of the z sums in
+// breakdown (Ctrl::status), which no workgroup of this launch reads.  With the finish of the z sums in
 // kb_pupdate_f and the convergence test in the tail, an iteration has three
 // launches of one workgroup per grid less (4.2 to 4.7 us each).
 template <typename S>
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(FIN_THREADS) void kb_update_f(BGrid<S>* G, const BI
     const double alpha = rz / pAp;
     if (it.a == 0 && threadIdx.x == 0) {
         c->pAp = pAp;
-        if (!ok) c->brk = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE;
+        if (!ok) c->status = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE;
         c->alpha = c->xalpha = ok ? alpha : 0.0;
         c->rsold = rz;
         c->first = 0;

@@ -403,16 +403,16 @@ __global__ void k_update(T* __restrict__ x, T* __restrict__ r, const T* __restri
 }
 // What the convergence test reads of the scalars.  Read before anything is
 // stored, they are one memory round trip.
-struct FinState { int done, brk, tol_mode, iter, max_iter; double tol, tolsq; double* hist; };
+struct FinState { int done, status, tol_mode, iter, max_iter; double tol, tolsq; double* hist; };
 __device__ __forceinline__ FinState fin_state(const Ctrl* c) {
-    return FinState{c->done, c->brk, c->tol_mode, c->iter, c->max_iter, c->tol, c->tolsq, c->hist};
+    return FinState{c->done, c->status, c->tol_mode, c->iter, c->max_iter, c->tol, c->tolsq, c->hist};
 }
 // a breakdown, or r.r of this iteration: history, convergence, iteration cap;
 // whether the solve stops (ctrl == nullptr: the decision alone)
 __device__ __forceinline__ int fin_update_scalars(Ctrl* ctrl, const FinState& f, double rs) {
     if (f.done) return 1;
-    if (f.brk) {
-        if (ctrl) { ctrl->iter = f.iter + 1; ctrl->done = 1; ctrl->status = f.brk; }
+    if (f.status != ST_RUNNING) {
+        if (ctrl) { ctrl->iter = f.iter + 1; ctrl->done = 1; }
         return 1;
     }
     const bool conv = (f.tol_mode == 1) ? (rs < f.tolsq) : (sqrt(rs) < f.tol);

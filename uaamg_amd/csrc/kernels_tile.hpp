@@ -511,7 +511,7 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_pmv(const T* __restrict__ z,
 
 // The operator's finish (alpha, breakdown), x += alpha p, r -= alpha Ap and
 // the r.r partials.  Workgroup 0 stores the scalars, rsold for the next beta
-// and a breakdown for the convergence test (Ctrl::brk); no workgroup of this
+// and a breakdown for the convergence test (Ctrl::status); no workgroup of this
 // launch reads those.
 template <typename T>
 __global__ __launch_bounds__(FIN_THREADS) void k_t2_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p,
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(FIN_THREADS) void k_t2_update(T* __restrict__ x, T*
     const double alpha = rz / pAp;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctrl->pAp = pAp;
-        if (!ok) ctrl->brk = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE;
+        if (!ok) ctrl->status = isfinite(pAp) ? ST_BREAKDOWN : ST_NONFINITE;
         ctrl->alpha = ctrl->xalpha = ok ? alpha : 0.0;
         ctrl->rsold = rz;
         ctrl->first = 0;
