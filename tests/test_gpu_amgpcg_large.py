@@ -1,0 +1,26 @@
+"""GPU: amgpcg at sides with more partial sums than a workgroup has threads
+(operator 256, level-0 down 512) and at the first sides whose partials are
+folded by a launch of their own.  The CG iterates of a fixed count equal the
+oracle's to the repository's FP64 bar (1e-9 of max|x|); FP32 runs the same
+launches and is held to the FP32 rounding of r over the smallest eigenvalue,
+6e-8 x 4 N^2 / (2 pi^2)."""
+import numpy as np
+import pytest
+
+import oracle_bind as ob
+import uaamg_amd as U
+from test_gpu_amgpcg import _rhs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N", [545, 700, 1024, 1025, 1100])
+def test_fixed_count(gpu, N):
+    b = _rhs(N)
+    print(f"[amgpcg large] N={N}", flush=True)
+    xo, ito = ob.amgpcg(N, b, 5, 1e-300)
+    for prec in (U.FP64, U.FP32):
+        x, it = gpu.amgpcg(N, b, 5, 1e-300, prec)
+        assert it == ito == 5
+        bar = 1e-9 if prec == U.FP64 else 6e-8 * 4 * N * N / (2 * np.pi ** 2)
+        assert np.abs(x - xo).max() <= bar * np.abs(xo).max()

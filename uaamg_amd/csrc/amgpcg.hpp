@@ -10,6 +10,7 @@
 // x += h^2/4 (b - A x).  PCG with absolute tolerance, out_iters = k+1.
 #pragma once
 #include <functional>
+#include "amgpcg_plan.hpp"
 #include "engine.hpp"
 
 namespace uaamg {
@@ -50,6 +51,19 @@ __device__ __forceinline__ double ag_total(const double* partials, int nb) {
     return all;
 }
 
+// n partials in fixed shares to AG_FOLD sums, one workgroup each (ag_plan).
+// With every workgroup adding all partials, an iteration of a large solve
+// went mostly into that (us an iteration, FP64: N = 1500 158 -> 150, 2048 384 -> 329,
+// 4096 1306 -> 805, 6144 4378 -> 1685; N = 1024 99, with the fold 111).
+__global__ __launch_bounds__(256) void k_ag_fold(const double* __restrict__ in, int n, double* __restrict__ out, const int* done) {
+    if (*done) return;
+    const int len = (n + AG_FOLD - 1) / AG_FOLD, beg = (int)blockIdx.x * len, end = min(n, beg + len);
+    double v[1] = {0.0};
+    for (int k = beg + (int)threadIdx.x; k < end; k += 256) v[0] += in[k];
+    block_sum<1>(v);
+    if (threadIdx.x == 0) out[blockIdx.x] = v[0];
+}
+
 // ---- tile kernels: one launch down and one up per level ----
 //
 // A workgroup owns AT_X x AT_Y cells of a level plus a halo of AT_H cells;
@@ -62,7 +76,7 @@ __device__ __forceinline__ double ag_total(const double* partials, int nb) {
 // These levels are latency-bound (a 256^2 FP64 level is 0.5 MB): with every
 // colour pass, restriction and prolongation a launch of its own an N = 256
 // FP64 solve took 6.6 ms with the GPU busy for 12 % of it, now 1.1 ms.
-constexpr int AT_X = 32, AT_Y = 16, AT_H = 4, AT_THREADS = 512;
+constexpr int AT_H = 4, AT_THREADS = 512;
 constexpr int AT_RX = AT_X + 2 * AT_H, AT_RY = AT_Y + 2 * AT_H, AT_HX = AT_RX / 2, AT_SX = AT_HX + 2;
 constexpr int AT_N = AT_SX * (AT_RY + 2);   // one side's LDS array: the pairs and a ring that stays 0
 static_assert(AT_HX * AT_RY <= AT_THREADS && AT_H % 2 == 0 && AT_X % 2 == 0 && AT_Y % 2 == 0, "pairs are the coarse cells' children");
@@ -211,7 +225,7 @@ __global__ __launch_bounds__(AT_THREADS) void k_ag_up(const T* __restrict__ xd, 
 }
 
 // ---- the levels of at most AG_TAIL cells a side, in one workgroup ----
-constexpr int AG_TAIL = 64, AG_TAIL_THREADS = 1024, AG_TAIL_MAXL = 8;
+constexpr int AG_TAIL_THREADS = 1024, AG_TAIL_MAXL = 8;
 constexpr int AG_TAIL_CELLS = 6016;   // >= the padded cells of 64, 32, 16, 8, 4, 2
 
 struct AgTail {
@@ -365,7 +379,7 @@ __global__ __launch_bounds__(AG_TAIL_THREADS) void k_ag_tail(AgTail A, const T* 
 
 // p = z + beta p (written to the other p buffer: neighbours still read p) and
 // Ap, p.Ap partials.  beta = r.z / the last iteration's (k = 0: 0, p is 0).
-constexpr int AP_X = 64, AP_Y = 16, AP_ROWS = 4;
+constexpr int AP_ROWS = 4;
 template <typename T>
 __global__ __launch_bounds__(AP_X * AP_Y / AP_ROWS) void k_ag_pmv(const T* __restrict__ z, const T* __restrict__ p, T* __restrict__ pn,
                                                                   T* __restrict__ Ap, int N, T inv_h2, const double* rz, int nrz,
@@ -422,7 +436,6 @@ inline std::vector<int> amgpcg_levels(int N) {
 // between the down leg and the next operator pass.)
 constexpr size_t kAgAlign = 256;
 inline size_t ag_round(size_t b) { return (b + kAgAlign - 1) / kAgAlign * kAgAlign; }
-inline dim3 ag_grid(int n) { return dim3((n + 63) / 64, (n + 3) / 4); }
 inline dim3 ag_tiles(int n) { return dim3((n + AT_X - 1) / AT_X, (n + AT_Y - 1) / AT_Y); }
 
 template <typename T>
@@ -431,8 +444,7 @@ size_t amgpcg_arena_bytes(int N) {
     for (int n : amgpcg_levels(N)) bytes += 2 * ag_round((size_t)(n + 2) * (n + 2) * sizeof(T));
     const size_t NN = (size_t)(N + 2) * (N + 2);
     bytes += 5 * ag_round(NN * sizeof(T));
-    const long maxb = (long)ag_grid(N).x * ag_grid(N).y;
-    bytes += ag_round((maxb + 64) * sizeof(double)) + ag_round(64);
+    bytes += ag_round(ag_partials_room(N) * sizeof(double)) + ag_round(64);
     return bytes;
 }
 
@@ -468,16 +480,22 @@ int amgpcg_core(int N, const double* b_dev, double* x_dev, int max_iter, double 
     T* rb[2] = {r, B[0]};
     T* pb[2] = {p, X[0]};
     const dim3 mgrid((N + AP_X - 1) / AP_X, (N + AP_Y - 1) / AP_Y), mblk(AP_X, AP_Y / AP_ROWS);
-    const int nm = (int)(mgrid.x * mgrid.y);
-    const long maxb = (long)ag_grid(N).x * ag_grid(N).y;
-    double* part_m = (double*)take((maxb + 64) * sizeof(double));
+    const AgPlan plan = ag_plan(N);
+    const int nm = plan.nm, nu = plan.nu;
+    if (plan.doubles > ag_partials_room(N)) throw HipError{hipErrorInvalidValue, "amgpcg: partial sums do not fit"};
+    double* part_m = (double*)take(ag_partials_room(N) * sizeof(double));
     AgCtrl* ctrl = (AgCtrl*)take(64);
     double* part_z = part_m + nm;    // r.r partials first, then r.z (the tail has read the former before the last up launch)
+    // what the consumers add
+    double* sum_m = plan.fold ? part_z + nu : part_m;
+    double* sum_z = plan.fold ? sum_m + AG_FOLD : part_z;
+    auto fold = [&](const double* part, int n, double* sum) {
+        if (plan.fold) k_ag_fold<<<AG_FOLD, 256, 0, s>>>(part, n, sum, &ctrl->done);
+    };
 
     int lt = 0;                      // first level of the tail
     while (lv[lt] > AG_TAIL) lt++;
     const dim3 tgrid = ag_tiles(N);
-    const int nu = lt ? (int)(tgrid.x * tgrid.y) : std::min(64, (N * N + 255) / 256);
     AgTail tail{};
     tail.nl = nl - lt;
     for (int l = lt, off = 0; l < nl; l++) {
@@ -506,7 +524,7 @@ int amgpcg_core(int N, const double* b_dev, double* x_dev, int max_iter, double 
         const T* rr = rb[(k + 1) & 1];
         T* zd = pb[k & 1];
         AgUpdate<T> u{};
-        if (k >= 0) u = AgUpdate<T>{x, pb[(k + 1) & 1], rb[k & 1], Ap, rb[(k + 1) & 1], part_m, nm, part_z, ctrl, k & 1};
+        if (k >= 0) u = AgUpdate<T>{x, pb[(k + 1) & 1], rb[k & 1], Ap, rb[(k + 1) & 1], sum_m, plan.sum_m, part_z, ctrl, k & 1};
         for (int l = 0; l < lt; l++) {
             T* xl = l ? X[l] : zd;
             const T* bl = l ? B[l] : rr;
@@ -516,8 +534,9 @@ int amgpcg_core(int N, const double* b_dev, double* x_dev, int max_iter, double 
                 k_ag_down<T, false><<<ag_tiles(lv[l]), AT_THREADS, 0, s>>>(xl, bl, lv[l], ih2(lv[l]), idg(lv[l]), B[l + 1], lv[l + 1], nc_of(l), u, &ctrl->done);
         }
         if (lt == 0 && k >= 0) k_ag_update<T><<<nu, 256, 0, s>>>(u, N, &ctrl->done);
-        tail.rr = k >= 0 ? part_z : nullptr;
-        tail.nrr = nu;
+        if (k >= 0) fold(part_z, nu, sum_z);
+        tail.rr = k >= 0 ? sum_z : nullptr;
+        tail.nrr = plan.fold ? AG_FOLD : nu;
         tail.iter = k + 1;
         tail.dot = lt == 0 ? part_z : nullptr;
         k_ag_tail<T><<<1, AG_TAIL_THREADS, 0, s>>>(tail, lt ? B[lt] : rr, lt ? X[lt] : z);
@@ -528,13 +547,15 @@ int amgpcg_core(int N, const double* b_dev, double* x_dev, int max_iter, double 
             else
                 k_ag_up<T, false><<<ag_tiles(lv[l]), AT_THREADS, 0, s>>>(X[l], X2[l], B[l], lv[l], ih2(lv[l]), idg(lv[l]), xc, lv[l + 1], nullptr, &ctrl->done);
         }
+        fold(part_z, nu, sum_z);
     };
     precond(-1);
     int it_out = max_iter;
     for (int k = 0; k < max_iter;) {
         const int k1 = std::min(max_iter, k + AG_CHECK);
         for (; k < k1; k++) {
-            k_ag_pmv<T><<<mgrid, mblk, 0, s>>>(z, pb[k & 1], pb[(k + 1) & 1], Ap, N, ih2(N), part_z, lt ? nu : 1, ctrl, k, part_m);
+            k_ag_pmv<T><<<mgrid, mblk, 0, s>>>(z, pb[k & 1], pb[(k + 1) & 1], Ap, N, ih2(N), sum_z, plan.sum_z, ctrl, k, part_m);
+            fold(part_m, nm, sum_m);
             precond(k);
         }
         HIPCHK(hipGetLastError());
