@@ -700,10 +700,10 @@ public:
     // rows in windows.  Against the march kernels and flat CG passes that ran
     // here before: 512 x 256 x 256 FP32 solve (3 windows) 57.7 -> 37.5 ms; FP64:
     // kernels_rows64.hpp.
-    static constexpr int ROWS_NW = 10, ROWS_RW = 2, ROWS_CPL = sizeof(T) == 8 ? 2 : 4;   // ROWS_CPL: of wide rows
+    static constexpr int ROWS_NW = 10, ROWS_RW = 2;
     int rows_cpl_ = 0;          // cells per lane (0: row kernels not used)
     bool rows_win_ = false;     // rows are cut into windows
-    RowTabOf<T> rtab_{};
+    RowTab rtab_{};             // FP32 vectors
     RowGeo rgeo_{};
     unsigned rows_blocks_ = 0;
     // cells per lane and windows of rows of nx cells (0: no row kernels)
@@ -737,33 +737,37 @@ public:
             rows_cpl_ = row_lanes(n_[0], nwx, wl);
             if (narrow_rows(n_[0], n_[1], n_[2])) rows_cpl_ = row_lanes(n_[0], nwx, wl, 2);
             rows_win_ = nwx > 1;
-            const double ix = 1.0 / (h[0] * h[0]), iy = 1.0 / (h[1] * h[1]), iz = 1.0 / (h[2] * h[2]);
-            for (int m = 0; m < 64; m++) {
-                double d = ix * (((m >> 0) & 1) + ((m >> 1) & 1)) + iy * (((m >> 2) & 1) + ((m >> 3) & 1))
-                         + iz * (((m >> 4) & 1) + ((m >> 5) & 1));
-                rtab_.d[m] = (T)d;
-                rtab_.rinv[m] = d >= 1e-30 ? (T)(1.0 / d) : T(0);
-            }
-            rtab_.idx2 = (T)ix; rtab_.idy2 = (T)iy; rtab_.idz2 = (T)iz;
-            for (int m = 0; m < 64; m++)
-                ptab_.d[m] = ix * (((m >> 0) & 1) + ((m >> 1) & 1)) + iy * (((m >> 2) & 1) + ((m >> 3) & 1))
-                           + iz * (((m >> 4) & 1) + ((m >> 5) & 1));
-            ptab_.idx2 = ix; ptab_.idy2 = iy; ptab_.idz2 = iz;
-            const double e[6] = {2 * ix, 2 * ix, 2 * iy, 2 * iy, 2 * iz, 2 * iz};
-            rtab_.any_dirichlet = 0;
-            for (int f = 0; f < 6; f++) {
-                const bool on = wall[f] == UAAMG_WALL_DIRICHLET;
-                rtab_.ex[f] = on ? (T)e[f] : T(0);
-                ptab_.ex[f] = on ? e[f] : 0.0;
-                rtab_.any_dirichlet |= on;
-            }
-            ptab_.any_dirichlet = rtab_.any_dirichlet;
             rgeo_ = make_rowgeo(n_[1], n_[2], (sizeof(T) == 8 ? R64_NW * R64_RW : ROWS_NW * ROWS_RW) - 4, o_.rows_kc, nwx, wl);
             rows_blocks_ = 8u * (unsigned)rgeo_.per_xcd;
             pmv_on_ = (o_.forms & UAAMG_FORM_PMV) != 0;
-            pgeo_ = make_rowgeo(n_[1], n_[2], PMV_NW * PMV_RW - 2, o_.rows_kc, nwx, wl);   // FP32 vectors (FP64: flat)
-            pmv_blocks_ = 8u * (unsigned)pgeo_.per_xcd;
+            if constexpr (sizeof(T) == 4) {
+                pgeo_ = make_rowgeo(n_[1], n_[2], PMV_NW * PMV_RW - 2, o_.rows_kc, nwx, wl);
+                pmv_blocks_ = 8u * (unsigned)pgeo_.per_xcd;
+                rows_tables(h, wall);
+            }
         }
+    }
+    // level-0 constants of the FP32 row kernels (rtab_) and of their operator (ptab_, in FP64)
+    void rows_tables(const double h[3], const int wall[6]) {
+        const double ix = 1.0 / (h[0] * h[0]), iy = 1.0 / (h[1] * h[1]), iz = 1.0 / (h[2] * h[2]);
+        for (int m = 0; m < 64; m++) {
+            const double d = ix * (((m >> 0) & 1) + ((m >> 1) & 1)) + iy * (((m >> 2) & 1) + ((m >> 3) & 1))
+                           + iz * (((m >> 4) & 1) + ((m >> 5) & 1));
+            ptab_.d[m] = d;
+            rtab_.d[m] = (float)d;
+            rtab_.rinv[m] = d >= 1e-30 ? (float)(1.0 / d) : 0.0f;
+        }
+        ptab_.idx2 = ix; ptab_.idy2 = iy; ptab_.idz2 = iz;
+        rtab_.idx2 = (float)ix; rtab_.idy2 = (float)iy; rtab_.idz2 = (float)iz;
+        const double e[6] = {2 * ix, 2 * ix, 2 * iy, 2 * iy, 2 * iz, 2 * iz};
+        rtab_.any_dirichlet = 0;
+        for (int f = 0; f < 6; f++) {
+            const bool on = wall[f] == UAAMG_WALL_DIRICHLET;
+            ptab_.ex[f] = on ? e[f] : 0.0;
+            rtab_.ex[f] = (float)ptab_.ex[f];
+            rtab_.any_dirichlet |= on;
+        }
+        ptab_.any_dirichlet = rtab_.any_dirichlet;
     }
     // Tiles of the row kernels: TY rows by KC planes, KC 2 or a multiple of 4,
     // unless kc_force > 0 sets it; alone: no other grid shares the launch
@@ -858,12 +862,11 @@ public:
                 // UAAMG_FORM_NT_D plain): 34.5 vs 33.5 solves/s at 256^3 in three paired runs
                 const bool dnt = rows_nt(UAAMG_FORM_NT_D);
                 forms_used_ |= dnt ? UAAMG_FORM_NT_D : 0;
-                auto kern = rows_win_ ? (dnt ? k_rows_down0r<2, ROWS_NW, ROWS_RW, S, true, false, true, T>
-                                             : k_rows_down0r<2, ROWS_NW, ROWS_RW, S, false, false, true, T>)
-                                      : k_rows_down0r<2, ROWS_NW, ROWS_RW, S, false, false, false, T>;
-                if constexpr (ROWS_CPL == 4)
-                    if (rows_cpl_ == 4)
-                        kern = rows_win_ ? (dnt ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, false, true> : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, false, false, true>)
+                auto kern = rows_win_ ? (dnt ? k_rows_down0r<2, ROWS_NW, ROWS_RW, S, true, false, true>
+                                             : k_rows_down0r<2, ROWS_NW, ROWS_RW, S, false, false, true>)
+                                      : k_rows_down0r<2, ROWS_NW, ROWS_RW, S>;
+                if (rows_cpl_ == 4)
+                    kern = rows_win_ ? (dnt ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, false, true> : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, false, false, true>)
                              : dnt ? (rows_full() ? k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_down0r<4, ROWS_NW, ROWS_RW, S, true>)
                                    : k_rows_down0r<4, ROWS_NW, ROWS_RW, S>;
                 tlaunch(timer_, UAAMG_K_DOWN0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, (const T*)fr_old_,
@@ -874,9 +877,8 @@ public:
                 else if (!fin_fold_) k_fin_update<false><<<1, FIN_THREADS, 0, stream_>>>(partials_, (int)rows_blocks_, ctrl_);
                 return;
             }
-            auto kern = rows_win_ ? k_rows_down0<2, ROWS_NW, ROWS_RW, S, true, T> : k_rows_down0<2, ROWS_NW, ROWS_RW, S, false, T>;
-            if constexpr (ROWS_CPL == 4)
-                if (rows_cpl_ == 4) kern = rows_win_ ? k_rows_down0<4, ROWS_NW, ROWS_RW, S, true> : k_rows_down0<4, ROWS_NW, ROWS_RW, S>;
+            auto kern = rows_win_ ? k_rows_down0<2, ROWS_NW, ROWS_RW, S, true> : k_rows_down0<2, ROWS_NW, ROWS_RW, S>;
+            if (rows_cpl_ == 4) kern = rows_win_ ? k_rows_down0<4, ROWS_NW, ROWS_RW, S, true> : k_rows_down0<4, ROWS_NW, ROWS_RW, S>;
             tlaunch(timer_, UAAMG_K_DOWN0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, (const uint8_t*)nbr0_, g0_, rtab_,
                     rgeo_, C.b, C.g, skip);
         }
@@ -893,12 +895,11 @@ public:
             // 33.9 solves/s at 256^3 in three paired runs
             const bool unt = rows_nt(UAAMG_FORM_NT_U);
             forms_used_ |= unt ? UAAMG_FORM_NT_U : 0;
-            auto kern = rows_win_ ? (unt ? k_rows_up0<2, ROWS_NW, ROWS_RW, S, true, false, true, T>
-                                         : k_rows_up0<2, ROWS_NW, ROWS_RW, S, false, false, true, T>)
-                                  : k_rows_up0<2, ROWS_NW, ROWS_RW, S, false, false, false, T>;
-            if constexpr (ROWS_CPL == 4)
-                if (rows_cpl_ == 4)
-                    kern = rows_win_ ? (unt ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, false, true> : k_rows_up0<4, ROWS_NW, ROWS_RW, S, false, false, true>)
+            auto kern = rows_win_ ? (unt ? k_rows_up0<2, ROWS_NW, ROWS_RW, S, true, false, true>
+                                         : k_rows_up0<2, ROWS_NW, ROWS_RW, S, false, false, true>)
+                                  : k_rows_up0<2, ROWS_NW, ROWS_RW, S>;
+            if (rows_cpl_ == 4)
+                kern = rows_win_ ? (unt ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, false, true> : k_rows_up0<4, ROWS_NW, ROWS_RW, S, false, false, true>)
                          : unt ? (rows_full() ? k_rows_up0<4, ROWS_NW, ROWS_RW, S, true, true> : k_rows_up0<4, ROWS_NW, ROWS_RW, S, true>)
                                : k_rows_up0<4, ROWS_NW, ROWS_RW, S>;
             tlaunch(timer_, UAAMG_K_UP0, kern, dim3(rows_blocks_), dim3(ROWS_NW * 64), stream_, r, (const uint8_t*)nbr0_, g0_, rtab_, rgeo_,
@@ -1242,19 +1243,17 @@ public:
                 // UAAMG_FORM_NT_P plain): 33.6 vs 33.0 solves/s at 256^3 in three paired runs
                 const bool pnt = rows_nt(UAAMG_FORM_NT_P) && fr_;
                 forms_used_ |= pnt ? UAAMG_FORM_NT_P : 0;
-                auto kern = rows_win_ ? (fr_ ? (pnt ? k_rows_pmv<2, PMV_NW, PMV_RW, true, true, false, true, T>
-                                                    : k_rows_pmv<2, PMV_NW, PMV_RW, true, false, false, true, T>)
-                                             : k_rows_pmv<2, PMV_NW, PMV_RW, false, false, false, true, T>)
-                                      : (fr_ ? k_rows_pmv<2, PMV_NW, PMV_RW, true, false, false, false, T>
-                                             : k_rows_pmv<2, PMV_NW, PMV_RW, false, false, false, false, T>);
-                if constexpr (ROWS_CPL == 4)
-                    if (rows_cpl_ == 4 && rows_win_)
-                        kern = fr_ ? (pnt ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, false, true> : k_rows_pmv<4, PMV_NW, PMV_RW, true, false, false, true>)
-                                   : k_rows_pmv<4, PMV_NW, PMV_RW, false, false, false, true>;
-                    else if (rows_cpl_ == 4)
-                        kern = fr_ ? (pnt ? (rows_full() ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, true> : k_rows_pmv<4, PMV_NW, PMV_RW, true, true>)
-                                          : k_rows_pmv<4, PMV_NW, PMV_RW, true>)
-                                   : k_rows_pmv<4, PMV_NW, PMV_RW, false>;
+                auto kern = rows_win_ ? (fr_ ? (pnt ? k_rows_pmv<2, PMV_NW, PMV_RW, true, true, false, true>
+                                                    : k_rows_pmv<2, PMV_NW, PMV_RW, true, false, false, true>)
+                                             : k_rows_pmv<2, PMV_NW, PMV_RW, false, false, false, true>)
+                                      : (fr_ ? k_rows_pmv<2, PMV_NW, PMV_RW, true> : k_rows_pmv<2, PMV_NW, PMV_RW, false>);
+                if (rows_cpl_ == 4 && rows_win_)
+                    kern = fr_ ? (pnt ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, false, true> : k_rows_pmv<4, PMV_NW, PMV_RW, true, false, false, true>)
+                               : k_rows_pmv<4, PMV_NW, PMV_RW, false, false, false, true>;
+                else if (rows_cpl_ == 4)
+                    kern = fr_ ? (pnt ? (rows_full() ? k_rows_pmv<4, PMV_NW, PMV_RW, true, true, true> : k_rows_pmv<4, PMV_NW, PMV_RW, true, true>)
+                                      : k_rows_pmv<4, PMV_NW, PMV_RW, true>)
+                               : k_rows_pmv<4, PMV_NW, PMV_RW, false>;
                 tlaunch(timer_, UAAMG_K_MATVEC, kern, dim3(pmv_blocks_), dim3(PMV_NW * 64), stream_, (const T*)z_,
                         (const T*)pold, (T*)pnew, (T*)Ap_, (const uint8_t*)nbr0_, g0_, ptab_, pgeo_,
                         partials_m_, ctrl_, (const double*)partials_, (int)rows_blocks_);

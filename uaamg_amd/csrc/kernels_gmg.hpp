@@ -445,7 +445,7 @@ __global__ __launch_bounds__(GMG_TAIL_THREADS) void k_gmg_tail(GmgTailArgs A_, V
         gmg_tail_sync(wave);
     };
     auto prolong_from = [&](const auto& L, int l, bool wave) {   // level l + 1 -> l
-        const Geo g = A.g[l], cg = A.g[l + 1];
+        const Geo cg = A.g[l + 1];
         const CT* XC = Xa + A.off[l + 1];
         const uint8_t* FC = Fa + A.off[l + 1];
         constexpr int NP = (int)(sizeof(L.e) / sizeof(int));
@@ -460,7 +460,6 @@ __global__ __launch_bounds__(GMG_TAIL_THREADS) void k_gmg_tail(GmgTailArgs A_, V
             if (L.F[k] & GF_FLUID) L.X[k] = L.X[k] + XC[cid];
             if (L.in1[v] && (L.F[k + 1] & GF_FLUID)) L.X[k + 1] = L.X[k + 1] + XC[cid];
         }
-        (void)g;
         gmg_tail_sync(wave);
     };
     auto pairs = [&](int l) { return A.g[l].ny * ((A.g[l].nx + 1) >> 1); };

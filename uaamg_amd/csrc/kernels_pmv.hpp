@@ -1,5 +1,5 @@
 // kernels_pmv.hpp -- level-0 search direction and operator in one pass (3D,
-// FP32 vectors: F = float; FP64: k_t2_pmv).
+// FP32 vectors; FP64: k_t2_pmv).
 //
 // One pass replaces the p update of iteration k-1 and the operator of
 // iteration k (pcg_3d.cpp:116-122 and 94-96):
@@ -40,9 +40,9 @@ struct PmvTab {
     int any_dirichlet;
 };
 
-template <int CPL, int NW, typename F>
+template <int CPL, int NW>
 struct PmvLDS {
-    F ex[2][NW][2][CPL][64];   // [step parity][wave][first / last row][cell][lane]
+    float ex[2][NW][2][CPL][64];   // [step parity][wave][first / last row][cell][lane]
 };
 
 // With FZ the pass also does the finish of the z sums (finish_zsums,
@@ -51,15 +51,15 @@ struct PmvLDS {
 // and beta; workgroup 0 stores them.  rsold and the first-iteration flag are
 // read here and only written by the next kernel (the level-0 down kernel),
 // so no workgroup can see a value of this launch.
-template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false, bool WIN = false, typename F>
-__device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __restrict__ pold,
-                                           F* __restrict__ pnew, F* __restrict__ Ap,
+template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false, bool WIN = false>
+__device__ __forceinline__ void d_rows_pmv(const float* __restrict__ z, const float* __restrict__ pold,
+                                           float* __restrict__ pnew, float* __restrict__ Ap,
                                            const uint8_t* __restrict__ nbr, const Geo& g, const PmvTab& K,
                                            const RowGeo& rg, double* partials, Ctrl* ctrl, int tile,
                                            const double* zp = nullptr, int nzp = 0) {
-    using RV = typename RowVec<CPL, F>::V;
+    using RV = typename RowVec<CPL>::V;
     if (ctrl->done) return;
-    __shared__ PmvLDS<CPL, NW, F> L;
+    __shared__ PmvLDS<CPL, NW> L;
     __shared__ double sd[64];
     __shared__ double s_zs[3];
     double acc[1] = {0.0};
@@ -73,9 +73,9 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
     const int dir = (th.kc & 1) ? -1 : 1;
     const int lane = th.lane, w = th.w;
 
-    F PN[4][RW][CPL];        // p_new of the last four planes
+    float PN[4][RW][CPL];        // p_new of the last four planes
     uint8_t NB[4][RW][CPL];
-    F pfz[2][RW][CPL], pfp[2][RW][CPL];
+    float pfz[2][RW][CPL], pfp[2][RW][CPL];
     uint8_t pfn[2][RW][CPL];
     auto issue = [&](int slot, int P) {
         const int po = th.plane(g, P);
@@ -112,7 +112,7 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
     // A = FP32: the p update is one FMA with the FP64 scalars rounded once: it
     // differs from k_pupdate's FP64 form by the rounding of the scalars, far
     // below the FP32 storage of the vectors
-    using A = RowCG<CPL, WIN, F>;
+    using A = RowCG<CPL, WIN>;
     A mean, beta;
     if constexpr (FZ) {
         const double sz = s_zs[0], srz = s_zs[1], sr = s_zs[2];
@@ -136,7 +136,7 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
 #pragma unroll
             for (int t = 0; t < RW; t++)
 #pragma unroll
-                for (int q = 0; q < CPL; q++) { PN[s][t][q] = F(0); NB[s][t][q] = 0; }
+                for (int q = 0; q < CPL; q++) { PN[s][t][q] = 0.0f; NB[s][t][q] = 0; }
 
         // step: plane P enters (slot S); the operator on plane P-1
         auto step = [&](auto Sc, int P) {
@@ -151,7 +151,7 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
                     const uint8_t nb = pin ? pfn[PB][t][q] : (uint8_t)0;
                     NB[S][t][q] = nb;
                     PN[S][t][q] = (nb & NB_FLUID)
-                        ? (F)rfma(beta, (A)pfp[PB][t][q], (A)pfz[PB][t][q] - mean) : F(0);
+                        ? (float)rfma(beta, (A)pfp[PB][t][q], (A)pfz[PB][t][q] - mean) : 0.0f;
                 }
             // the last plane to enter is last + 1 (upwards) or m0 - 1 (downwards);
             // beyond it the loads repeat that cached plane (no memory traffic), so
@@ -190,16 +190,16 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
                 }
                 sfor<RW>([&](auto tc) {
                     constexpr int t = decltype(tc)::value;
-                    const F el = lane_from_left(PN[S1][t][CPL - 1]);
-                    const F er = lane_from_right(PN[S1][t][0]);
-                    F out[CPL];
+                    const float el = lane_from_left(PN[S1][t][CPL - 1]);
+                    const float er = lane_from_right(PN[S1][t][0]);
+                    float out[CPL];
                     A pap = A(0);   // the row's p.Ap, accumulated in FP64
                     sfor<CPL>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
-                        const F vc = PN[S1][t][q];
-                        const F vl = (q > 0) ? PN[S1][t][q > 0 ? q - 1 : 0] : el;
-                        const F vr = (q < CPL - 1) ? PN[S1][t][q < CPL - 1 ? q + 1 : 0] : er;
-                        F vb, vt;
+                        const float vc = PN[S1][t][q];
+                        const float vl = (q > 0) ? PN[S1][t][q > 0 ? q - 1 : 0] : el;
+                        const float vr = (q < CPL - 1) ? PN[S1][t][q < CPL - 1 ? q + 1 : 0] : er;
+                        float vb, vt;
                         if constexpr (t > 0) vb = PN[S1][t - 1][q]; else vb = L.ex[RB][w > 0 ? w - 1 : 0][1][q][lane];
                         if constexpr (t < RW - 1) vt = PN[S1][t + 1][q]; else vt = L.ex[RB][w < NW - 1 ? w + 1 : NW - 1][0][q][lane];
                         const uint8_t nb = NB[S1][t][q];
@@ -207,8 +207,8 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
                         const double sum = K.idx2 * ((double)vl + (double)vr) + K.idy2 * ((double)vb + (double)vt)
                                          + K.idz2 * ((double)PN[S2][t][q] + (double)PN[S][t][q]);
                         const bool fl = nb & NB_FLUID;
-                        const F o = fl ? (F)(d * (double)vc - sum) : F(0);
-                        pap = rfma((A)(th.okw[q] ? vc : F(0)), (A)o, pap);
+                        const float o = fl ? (float)(d * (double)vc - sum) : 0.0f;
+                        pap = rfma((A)(th.okw[q] ? vc : 0.0f), (A)o, pap);
                         out[q] = o;
                     });
                     if (th.tile_row[t]) acc[0] += (double)pap;
@@ -243,13 +243,13 @@ __device__ __forceinline__ void d_rows_pmv(const F* __restrict__ z, const F* __r
     block_store<1>(acc, partials);
 }
 
-template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false, bool WIN = false, typename F = float>
-__global__ __launch_bounds__(NW * 64) void k_rows_pmv(const F* __restrict__ z, const F* __restrict__ pold,
-                                                      F* __restrict__ pnew, F* __restrict__ Ap,
+template <int CPL, int NW, int RW, bool FZ = false, bool NT = false, bool FULL = false, bool WIN = false>
+__global__ __launch_bounds__(NW * 64) void k_rows_pmv(const float* __restrict__ z, const float* __restrict__ pold,
+                                                      float* __restrict__ pnew, float* __restrict__ Ap,
                                                       const uint8_t* __restrict__ nbr, Geo g, PmvTab K,
                                                       RowGeo rg, double* partials, Ctrl* ctrl,
                                                       const double* zp, int nzp) {
-    d_rows_pmv<CPL, NW, RW, FZ, NT, FULL, WIN, F>(z, pold, pnew, Ap, nbr, g, K, rg, partials, ctrl, row_tile_of_block(rg, blockIdx.x),
+    d_rows_pmv<CPL, NW, RW, FZ, NT, FULL, WIN>(z, pold, pnew, Ap, nbr, g, K, rg, partials, ctrl, row_tile_of_block(rg, blockIdx.x),
                                 zp, nzp);
 }
 

@@ -1,5 +1,5 @@
-// kernels_rows.hpp -- level-0 V(1,1) kernels in 3D for FP32 vectors (F =
-// float; FP64 vectors: kernels_rows64.hpp).
+// kernels_rows.hpp -- level-0 V(1,1) kernels in 3D for FP32 vectors
+// (FP64 vectors: kernels_rows64.hpp).
 //
 // The same preconditioner as the reference's level-0 smooth /
 // restrictResidual / prolongateAdd (uaamg_preconditioner_3d.cpp:123-181).
@@ -46,15 +46,13 @@ namespace uaamg {
 // Level-0 stencil constants of the FP32 path: 1/d and d per neighbour pattern
 // (nb >> 1 = +x,-x,+y,-y,+z,-z present; 1/d = 0 where d < 1e-30).  Dirichlet
 // walls add their excess per cell.
-template <typename F>
-struct RowTabOf {
-    F rinv[64];
-    F d[64];
-    F idx2, idy2, idz2;
-    F ex[6];
+struct RowTab {
+    float rinv[64];
+    float d[64];
+    float idx2, idy2, idz2;
+    float ex[6];
     int any_dirichlet;
 };
-using RowTab = RowTabOf<float>;
 
 struct RowGeo {
     int nty;       // tiles in y
@@ -77,8 +75,8 @@ __device__ __forceinline__ double rfma(double a, double b, double c) { return fm
 // lane) do it all in FP64, as the flat passes that such grids have with the
 // fused passes switched off (512 x 256 x 256 35.0 -> 36.8 ms a solve for it,
 // 300^3 51.6 -> 57.4; on march kernels and flat passes 57 and 80).
-template <int CPL, bool WIN, typename F>
-using RowCG = std::conditional_t<WIN && CPL == 4, double, F>;
+template <int CPL, bool WIN>
+using RowCG = std::conditional_t<WIN && CPL == 4, double, float>;
 
 // Whole-wave shifts by one lane with DPP (wave_shr:1 = 0x138, wave_shl:1 =
 // 0x130; all rows and banks enabled, lanes with no source keep old = 0):
@@ -108,14 +106,14 @@ __device__ __forceinline__ int row_tile_of_block(const RowGeo& rg, int b) {
 
 // 1/d of the RW x CPL cells of a lane's plane (0 on non-fluid cells and
 // where d < 1e-30): without Dirichlet walls the table value; with them d =
-// the table's d plus each touching wall's excess, divided in F.  Every
+// the table's d plus each touching wall's excess, divided.  Every
 // table read is issued before the first is used (one LDS round trip per
 // plane, not one per cell) and the Dirichlet test is one uniform branch.
-template <int RW, int CPL, typename F>
-__device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], F (&ri)[RW][CPL], const F* srinv,
-                                                const F* sd, const RowTabOf<F>& T, const Geo& g, int i0,
+template <int RW, int CPL>
+__device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], float (&ri)[RW][CPL], const float* srinv,
+                                                const float* sd, const RowTab& T, const Geo& g, int i0,
                                                 const int (&jrow)[RW], int k) {
-    F v[RW][CPL];
+    float v[RW][CPL];
     if (!T.any_dirichlet) {
 #pragma unroll
         for (int t = 0; t < RW; t++)
@@ -124,7 +122,7 @@ __device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], F 
 #pragma unroll
         for (int t = 0; t < RW; t++)
 #pragma unroll
-            for (int q = 0; q < CPL; q++) ri[t][q] = (nb[t][q] & NB_FLUID) ? v[t][q] : F(0);
+            for (int q = 0; q < CPL; q++) ri[t][q] = (nb[t][q] & NB_FLUID) ? v[t][q] : 0.0f;
     } else {
 #pragma unroll
         for (int t = 0; t < RW; t++)
@@ -134,7 +132,7 @@ __device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], F 
         for (int t = 0; t < RW; t++)
 #pragma unroll
             for (int q = 0; q < CPL; q++) {
-                F d = v[t][q];
+                float d = v[t][q];
                 const int i = i0 + q, j = jrow[t];
                 if (i == 1) d += T.ex[0];
                 if (i == g.nx) d += T.ex[1];
@@ -142,7 +140,7 @@ __device__ __forceinline__ void rows_rinv_plane(const uint8_t (&nb)[RW][CPL], F 
                 if (j == g.ny) d += T.ex[3];
                 if (k == 1) d += T.ex[4];
                 if (k == g.nz) d += T.ex[5];
-                ri[t][q] = (nb[t][q] & NB_FLUID) ? (d >= F(1e-30) ? F(1) / d : F(0)) : F(0);
+                ri[t][q] = (nb[t][q] & NB_FLUID) ? (d >= 1e-30f ? 1.0f / d : 0.0f) : 0.0f;
             }
     }
 }
@@ -180,12 +178,12 @@ __device__ __forceinline__ void row_load(const F* __restrict__ r, const uint8_t*
     }
 }
 
-template <int CPL, int NW, int RW, typename F = float>
+template <int CPL, int NW, int RW>
 struct RowLDS {
-    F tab[2][64];
+    float tab[2][64];
     // rows shared between waves: [buffer][kind 0: S1 output, 1: S2 output]
     // [wave][0: first row, 1: last row][colour cell q/2][lane]
-    F ex[2][2][NW][2][CPL / 2][64];
+    float ex[2][2][NW][2][CPL / 2][64];
 };
 
 template <int V> using IC = std::integral_constant<int, V>;
@@ -193,10 +191,10 @@ template <int V> using IC = std::integral_constant<int, V>;
 // Sum over the 6 neighbours of cell (T, Q) of plane slot s: in-plane values
 // from X[s] (other waves' rows from the LDS exchange eb/kind), z-neighbours
 // from slots sp and sm; edge = the neighbour across the lane boundary.
-template <int CPL, int NW, int RW, int T, int Q, int s, int sp, int sm, typename F>
-__device__ __forceinline__ F row_nsum(const F (&X)[4][RW][CPL], F edge, const RowLDS<CPL, NW, RW, F>& L,
-                                      int eb, int kind, int w, int lane, const RowTabOf<F>& K) {
-    F xl, xr, xu, xd;
+template <int CPL, int NW, int RW, int T, int Q, int s, int sp, int sm>
+__device__ __forceinline__ float row_nsum(const float (&X)[4][RW][CPL], float edge, const RowLDS<CPL, NW, RW>& L,
+                                      int eb, int kind, int w, int lane, const RowTab& K) {
+    float xl, xr, xu, xd;
     if constexpr (Q > 0) xl = X[s][T][Q - 1]; else xl = edge;
     if constexpr (Q < CPL - 1) xr = X[s][T][Q + 1]; else xr = edge;
     if constexpr (T > 0) xu = X[s][T - 1][Q]; else xu = L.ex[eb][kind][w > 0 ? w - 1 : 0][1][Q / 2][lane];
@@ -289,10 +287,9 @@ struct FinUpd {
     Ctrl* ctrl = nullptr;
 };
 
-template <typename F>
-struct RUpdOf {
-    const F* Ap = nullptr;
-    F* rnew = nullptr;
+struct RUpd {
+    const float* Ap = nullptr;
+    float* rnew = nullptr;
     double* partials = nullptr;      // r.r partials (this kernel's)
     const double* pap = nullptr;     // p.Ap partials of the operator pass
     int npap = 0;
@@ -300,19 +297,19 @@ struct RUpdOf {
     int xslot = 0;                   // ctrl->xa slot of this iteration's x pass (its p buffer)
 };
 
-template <int CPL, int NW, int RW, typename VC, bool FR = false, bool NT = false, bool FULL = false, bool WIN = false, typename F>
-__device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
-                                             const RowTabOf<F>& K, const RowGeo& rg, VC* __restrict__ bc, const Geo& cg,
-                                             const int* skip, int tile, const RUpdOf<F>& u = RUpdOf<F>{}) {
-    using RV = typename RowVec<CPL, F>::V;
+template <int CPL, int NW, int RW, typename VC, bool FR = false, bool NT = false, bool FULL = false, bool WIN = false>
+__device__ __forceinline__ void d_rows_down0(const float* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
+                                             const RowTab& K, const RowGeo& rg, VC* __restrict__ bc, const Geo& cg,
+                                             const int* skip, int tile, const RUpd& u = RUpd{}) {
+    using RV = typename RowVec<CPL>::V;
     static_assert(CPL % 2 == 0 && RW % 2 == 0, "pairs of cells and rows");
     if (skip && *skip) {
         // a stopped solve: no x update for this iteration
         if constexpr (FR) { if (blockIdx.x == 0 && threadIdx.x == 0) u.ctrl->xa[u.xslot] = 0.0; }
         return;
     }
-    __shared__ RowLDS<CPL, NW, RW, F> L;
-    using A = RowCG<CPL, WIN, F>;
+    __shared__ RowLDS<CPL, NW, RW> L;
+    using A = RowCG<CPL, WIN>;
     A alpha = A(0);
     if constexpr (FR) {
         __shared__ double s_pap;
@@ -346,24 +343,24 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
     th.init(g, rg, tile);
     const int lane = th.lane, w = th.w;
     for (int e = threadIdx.x; e < 64; e += NW * 64) { L.tab[0][e] = K.rinv[e]; L.tab[1][e] = K.d[e]; }
-    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = F(0);
+    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = 0.0f;
     __syncthreads();
 
-    F X[4][RW][CPL], Rq[2][RW][CPL], Iq[4][RW][CPL];
-    F pfr[2][RW][CPL];
-    F pfa[FR ? 2 : 1][RW][CPL];
+    float X[4][RW][CPL], Rq[2][RW][CPL], Iq[4][RW][CPL];
+    float pfr[2][RW][CPL];
+    float pfa[FR ? 2 : 1][RW][CPL];
     uint8_t pfn[2][RW][CPL];
-    F acc[RW / 2][CPL / 2];
+    float acc[RW / 2][CPL / 2];
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
         for (int t = 0; t < RW; t++)
 #pragma unroll
-            for (int q = 0; q < CPL; q++) { X[s][t][q] = F(0); Rq[s & 1][t][q] = F(0); Iq[s][t][q] = F(0); }
+            for (int q = 0; q < CPL; q++) { X[s][t][q] = 0.0f; Rq[s & 1][t][q] = 0.0f; Iq[s][t][q] = 0.0f; }
 #pragma unroll
     for (int a = 0; a < RW / 2; a++)
 #pragma unroll
-        for (int c = 0; c < CPL / 2; c++) acc[a][c] = F(0);
+        for (int c = 0; c < CPL / 2; c++) acc[a][c] = 0.0f;
 
     auto issue = [&](int slot, int P) {
         // unconditional loads from clamped addresses: straight-line code lets
@@ -402,9 +399,9 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     const bool fl = pfn[PB][t][q] & NB_FLUID;
-                    const F rn = fl ? (F)rfma(-alpha, (A)pfa[PB][t][q], (A)pfr[PB][t][q]) : F(0);
+                    const float rn = fl ? (float)rfma(-alpha, (A)pfa[PB][t][q], (A)pfr[PB][t][q]) : 0.0f;
                     pfr[PB][t][q] = rn;
-                    rs = rfma((A)(th.okw[q] ? rn : F(0)), (A)rn, rs);
+                    rs = rfma((A)(th.okw[q] ? rn : 0.0f), (A)rn, rs);
                 });
                 if (pin && th.tile_row[t]) rr[0] += (double)rs;
                 if (pin && th.tile_row[t]) {
@@ -422,21 +419,21 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
                 }
             });
         }
-        F riP[RW][CPL];
-        rows_rinv_plane<RW, CPL, F>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
+        float riP[RW][CPL];
+        rows_rinv_plane<RW, CPL>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
         sfor<RW>([&](auto tc) {
             constexpr int t = decltype(tc)::value;
             sfor<CPL>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
                 const uint8_t nb = pfn[PB][t][q];
-                const F rv = (nb & NB_FLUID) ? pfr[PB][t][q] : F(0);
-                const F ri = riP[t][q];
+                const float rv = (nb & NB_FLUID) ? pfr[PB][t][q] : 0.0f;
+                const float ri = riP[t][q];
                 Rq[S & 1][t][q] = rv;
                 Iq[S][t][q] = ri;
                 // isolated fluid cells (ri == 0, no fluid neighbour: their x is
                 // never read) carry r, their residual; non-fluid cells carry 0
-                if constexpr (((q + t + S) & 1) == 1) X[S][t][q] = (ri != F(0)) ? rv * ri : rv;
-                else X[S][t][q] = (ri != F(0)) ? F(0) : rv;
+                if constexpr (((q + t + S) & 1) == 1) X[S][t][q] = (ri != 0.0f) ? rv * ri : rv;
+                else X[S][t][q] = (ri != 0.0f) ? 0.0f : rv;
             });
         });
         issue(PB, min(P + 2, th.last + 2));   // past last + 2 (never used): the cached plane last + 2 again, no memory traffic
@@ -450,15 +447,15 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
                 constexpr bool q0 = ((t + S1) & 1) == 0;   // cell 0 of this row is even
-                const F edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
+                const float edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     if constexpr (((q + t + S1) & 1) == 0) {
-                        const F s = row_nsum<CPL, NW, RW, t, q, S1, S, S2, F>(X, edge, L, ER, 0, w, lane, K);
+                        const float s = row_nsum<CPL, NW, RW, t, q, S1, S, S2>(X, edge, L, ER, 0, w, lane, K);
                         // (r + s) / d on cells with 1/d != 0; isolated and non-fluid
                         // cells keep X.  Written as a blend so it stays branch-free.
-                        const F ri = Iq[S1][t][q];
-                        X[S1][t][q] = (Rq[S1 & 1][t][q] + s) * ri + ((ri != F(0)) ? F(0) : X[S1][t][q]);
+                        const float ri = Iq[S1][t][q];
+                        X[S1][t][q] = (Rq[S1 & 1][t][q] + s) * ri + ((ri != 0.0f) ? 0.0f : X[S1][t][q]);
                     }
                 });
             });
@@ -476,21 +473,21 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
 #pragma unroll
                 for (int a = 0; a < RW / 2; a++)
 #pragma unroll
-                    for (int c = 0; c < CPL / 2; c++) acc[a][c] = F(0);
+                    for (int c = 0; c < CPL / 2; c++) acc[a][c] = 0.0f;
             }
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
                 constexpr bool q0 = ((t + S2) & 1) == 1;   // cell 0 of this row is odd
-                const F edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
+                const float edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     if constexpr (((q + t + S2) & 1) == 1) {
-                        const F s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3, F>(X, edge, L, ER, 1, w, lane, K);
-                        const bool iso = Iq[S2][t][q] == F(0);
-                        acc[t / 2][q / 2] += (iso ? F(0) : s) + (iso ? X[S2][t][q] : F(0));
+                        const float s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3>(X, edge, L, ER, 1, w, lane, K);
+                        const bool iso = Iq[S2][t][q] == 0.0f;
+                        acc[t / 2][q / 2] += (iso ? 0.0f : s) + (iso ? X[S2][t][q] : 0.0f);
                     } else {
                         // even cells: residual 0 after the even update, r on isolated cells
-                        acc[t / 2][q / 2] += (Iq[S2][t][q] != F(0)) ? F(0) : X[S2][t][q];
+                        acc[t / 2][q / 2] += (Iq[S2][t][q] != 0.0f) ? 0.0f : X[S2][t][q];
                     }
                 });
             });
@@ -523,51 +520,51 @@ __device__ __forceinline__ void d_rows_down0(const F* __restrict__ r, const uint
     if constexpr (FR) block_store<1>(rr, u.partials);
 }
 
-template <int CPL, int NW, int RW, typename VC, bool WIN = false, typename F = float>
-__global__ __launch_bounds__(NW * 64) void k_rows_down0(const F* __restrict__ r, const uint8_t* __restrict__ nbr,
-                                                        Geo g, RowTabOf<F> K, RowGeo rg, VC* __restrict__ bc, Geo cg,
+template <int CPL, int NW, int RW, typename VC, bool WIN = false>
+__global__ __launch_bounds__(NW * 64) void k_rows_down0(const float* __restrict__ r, const uint8_t* __restrict__ nbr,
+                                                        Geo g, RowTab K, RowGeo rg, VC* __restrict__ bc, Geo cg,
                                                         const int* skip) {
-    d_rows_down0<CPL, NW, RW, VC, false, false, false, WIN, F>(r, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x));
+    d_rows_down0<CPL, NW, RW, VC, false, false, false, WIN>(r, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x));
 }
 
 // down0 with the fused residual update (r_old -> r_new, r.r partials) and
 // the operator's finish (alpha from the p.Ap partials)
-template <int CPL, int NW, int RW, typename VC, bool NT = false, bool FULL = false, bool WIN = false, typename F = float>
-__global__ __launch_bounds__(NW * 64) void k_rows_down0r(const F* __restrict__ rold, const uint8_t* __restrict__ nbr,
-                                                         Geo g, RowTabOf<F> K, RowGeo rg, VC* __restrict__ bc, Geo cg,
-                                                         const int* skip, const F* __restrict__ Ap,
-                                                         F* __restrict__ rnew, double* partials,
+template <int CPL, int NW, int RW, typename VC, bool NT = false, bool FULL = false, bool WIN = false>
+__global__ __launch_bounds__(NW * 64) void k_rows_down0r(const float* __restrict__ rold, const uint8_t* __restrict__ nbr,
+                                                         Geo g, RowTab K, RowGeo rg, VC* __restrict__ bc, Geo cg,
+                                                         const int* skip, const float* __restrict__ Ap,
+                                                         float* __restrict__ rnew, double* partials,
                                                          const double* pap, int npap, Ctrl* ctrl, int xslot) {
-    RUpdOf<F> u;
+    RUpd u;
     u.Ap = Ap; u.rnew = rnew; u.partials = partials; u.pap = pap; u.npap = npap; u.ctrl = ctrl; u.xslot = xslot;
-    d_rows_down0<CPL, NW, RW, VC, true, NT, FULL, WIN, F>(rold, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x), u);
+    d_rows_down0<CPL, NW, RW, VC, true, NT, FULL, WIN>(rold, nbr, g, K, rg, bc, cg, skip, row_tile_of_block(rg, blockIdx.x), u);
 }
 
 // ------------------------------------------------------------------ up
 // r, coarse x -> z (prolongation + reverse sweep), with sum z, sum r z, sum r
 // over fluid cells reduced per workgroup into partials.
-template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false, bool WIN = false, typename F>
-__device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
-                                           const RowTabOf<F>& K, const RowGeo& rg, const VCX* __restrict__ xc, const Geo& cg,
-                                           F* __restrict__ z, const int* skip, double* partials, int tile) {
+template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false, bool WIN = false>
+__device__ __forceinline__ void d_rows_up0(const float* __restrict__ r, const uint8_t* __restrict__ nbr, const Geo& g,
+                                           const RowTab& K, const RowGeo& rg, const VCX* __restrict__ xc, const Geo& cg,
+                                           float* __restrict__ z, const int* skip, double* partials, int tile) {
     static_assert(CPL % 2 == 0 && RW % 2 == 0, "pairs of cells and rows");
-    using RV = typename RowVec<CPL, F>::V;
+    using RV = typename RowVec<CPL, float>::V;
     if (skip && *skip) return;
-    __shared__ RowLDS<CPL, NW, RW, F> L;
+    __shared__ RowLDS<CPL, NW, RW> L;
     const bool active = tile < rg.ntiles;   // idle workgroups still store zero partials
     RowThread<CPL, NW, RW, 2, FULL, WIN> th;
     th.init(g, rg, active ? tile : 0);
     const int lane = th.lane, w = th.w;
     for (int e = threadIdx.x; e < 64; e += NW * 64) { L.tab[0][e] = K.rinv[e]; L.tab[1][e] = K.d[e]; }
-    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = F(0);
+    for (int e = threadIdx.x; e < 2 * 2 * NW * 2 * (CPL / 2) * 64; e += NW * 64) (&L.ex[0][0][0][0][0][0])[e] = 0.0f;
     __syncthreads();
     double red[3] = {0.0, 0.0, 0.0};
 
     if (active) {
-        F X[4][RW][CPL], Rq[4][RW][CPL], Iq[4][RW][CPL];
-        F pfr[2][RW][CPL];
+        float X[4][RW][CPL], Rq[4][RW][CPL], Iq[4][RW][CPL];
+        float pfr[2][RW][CPL];
         uint8_t pfn[2][RW][CPL];
-        F pfx[2][RW / 2][CPL / 2];
+        float pfx[2][RW / 2][CPL / 2];
         bool pcin[2];
         int coff[RW / 2][CPL / 2];
         bool cok[RW / 2][CPL / 2];
@@ -584,7 +581,7 @@ __device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_
 #pragma unroll
             for (int t = 0; t < RW; t++)
 #pragma unroll
-                for (int q = 0; q < CPL; q++) { X[s][t][q] = F(0); Rq[s][t][q] = F(0); Iq[s][t][q] = F(0); }
+                for (int q = 0; q < CPL; q++) { X[s][t][q] = 0.0f; Rq[s][t][q] = 0.0f; Iq[s][t][q] = 0.0f; }
 
         auto issue = [&](int slot, int P) {
             const int po = th.plane(g, P);
@@ -598,7 +595,7 @@ __device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_
 #pragma unroll
             for (int a = 0; a < RW / 2; a++)
 #pragma unroll
-                for (int c = 0; c < CPL / 2; c++) pfx[slot][a][c] = (F)xc[coff[a][c] + cpo];
+                for (int c = 0; c < CPL / 2; c++) pfx[slot][a][c] = (float)xc[coff[a][c] + cpo];
         };
         issue(1, th.m0 - 2);
         issue(0, th.m0 - 1);
@@ -610,17 +607,17 @@ __device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_
             // S1: plane P: x' = x0 + 2 x_coarse (x0 = r/d on odd cells; the
             // even x0 is replaced by the reverse sweep, except on isolated cells
             // where it is 0)
-            F riP[RW][CPL];
-            rows_rinv_plane<RW, CPL, F>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
+            float riP[RW][CPL];
+            rows_rinv_plane<RW, CPL>(pfn[PB], riP, L.tab[0], L.tab[1], K, g, th.i0, th.jrow, P);
             sfor<RW>([&](auto tc) {
                 constexpr int t = decltype(tc)::value;
                 sfor<CPL>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
                     const uint8_t nb = pfn[PB][t][q];
                     const bool fl = nb & NB_FLUID;
-                    const F rv = fl ? pfr[PB][t][q] : F(0);
-                    const F ri = riP[t][q];
-                    const F w2 = (fl && pcin[PB] && cok[t / 2][q / 2]) ? F(2) * pfx[PB][t / 2][q / 2] : F(0);
+                    const float rv = fl ? pfr[PB][t][q] : 0.0f;
+                    const float ri = riP[t][q];
+                    const float w2 = (fl && pcin[PB] && cok[t / 2][q / 2]) ? 2.0f * pfx[PB][t / 2][q / 2] : 0.0f;
                     Rq[S][t][q] = rv;
                     Iq[S][t][q] = ri;
                     if constexpr (((q + t + S) & 1) == 1) X[S][t][q] = rv * ri + w2;
@@ -638,13 +635,13 @@ __device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_
                 sfor<RW>([&](auto tc) {
                     constexpr int t = decltype(tc)::value;
                     constexpr bool q0 = ((t + S1) & 1) == 0;
-                    const F edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
+                    const float edge = q0 ? lane_from_left(X[S1][t][CPL - 1]) : lane_from_right(X[S1][t][0]);
                     sfor<CPL>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
                         if constexpr (((q + t + S1) & 1) == 0) {
-                            const F s = row_nsum<CPL, NW, RW, t, q, S1, S, S2, F>(X, edge, L, ER, 0, w, lane, K);
-                            const F ri = Iq[S1][t][q];
-                            X[S1][t][q] = (Rq[S1][t][q] + s) * ri + ((ri != F(0)) ? F(0) : X[S1][t][q]);
+                            const float s = row_nsum<CPL, NW, RW, t, q, S1, S, S2>(X, edge, L, ER, 0, w, lane, K);
+                            const float ri = Iq[S1][t][q];
+                            X[S1][t][q] = (Rq[S1][t][q] + s) * ri + ((ri != 0.0f) ? 0.0f : X[S1][t][q]);
                         }
                     });
                 });
@@ -660,23 +657,23 @@ __device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_
                 sfor<RW>([&](auto tc) {
                     constexpr int t = decltype(tc)::value;
                     constexpr bool q0 = ((t + S2) & 1) == 1;
-                    const F edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
+                    const float edge = q0 ? lane_from_left(X[S2][t][CPL - 1]) : lane_from_right(X[S2][t][0]);
                     sfor<CPL>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
                         if constexpr (((q + t + S2) & 1) == 1) {
-                            const F s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3, F>(X, edge, L, ER, 1, w, lane, K);
-                            const F ri = Iq[S2][t][q];
-                            X[S2][t][q] = (Rq[S2][t][q] + s) * ri + ((ri != F(0)) ? F(0) : X[S2][t][q]);
+                            const float s = row_nsum<CPL, NW, RW, t, q, S2, S1, S3>(X, edge, L, ER, 1, w, lane, K);
+                            const float ri = Iq[S2][t][q];
+                            X[S2][t][q] = (Rq[S2][t][q] + s) * ri + ((ri != 0.0f) ? 0.0f : X[S2][t][q]);
                         }
                     });
                     if (th.tile_row[t]) {
                         // the row's CPL cells summed (FP32: one FMA each), the
                         // row sums accumulated in FP64
-                        using A = RowCG<CPL, WIN, F>;
+                        using A = RowCG<CPL, WIN>;
                         A s0 = A(0), s1 = A(0), s2 = A(0);
                         sfor<CPL>([&](auto qc) {
                             constexpr int q = decltype(qc)::value;
-                            const A zv = (A)(th.okw[q] ? X[S2][t][q] : F(0)), rv = (A)(th.okw[q] ? Rq[S2][t][q] : F(0));
+                            const A zv = (A)(th.okw[q] ? X[S2][t][q] : 0.0f), rv = (A)(th.okw[q] ? Rq[S2][t][q] : 0.0f);
                             s0 += zv;
                             s1 = rfma(rv, zv, s1);
                             s2 += rv;
@@ -713,11 +710,11 @@ __device__ __forceinline__ void d_rows_up0(const F* __restrict__ r, const uint8_
     block_store<3>(red, partials);
 }
 
-template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false, bool WIN = false, typename F = float>
-__global__ __launch_bounds__(NW * 64) void k_rows_up0(const F* __restrict__ r, const uint8_t* __restrict__ nbr,
-                                                      Geo g, RowTabOf<F> K, RowGeo rg, const VCX* __restrict__ xc, Geo cg,
-                                                      F* __restrict__ z, const int* skip, double* partials) {
-    d_rows_up0<CPL, NW, RW, VCX, NT, FULL, WIN, F>(r, nbr, g, K, rg, xc, cg, z, skip, partials, row_tile_of_block(rg, blockIdx.x));
+template <int CPL, int NW, int RW, typename VCX, bool NT = false, bool FULL = false, bool WIN = false>
+__global__ __launch_bounds__(NW * 64) void k_rows_up0(const float* __restrict__ r, const uint8_t* __restrict__ nbr,
+                                                      Geo g, RowTab K, RowGeo rg, const VCX* __restrict__ xc, Geo cg,
+                                                      float* __restrict__ z, const int* skip, double* partials) {
+    d_rows_up0<CPL, NW, RW, VCX, NT, FULL, WIN>(r, nbr, g, K, rg, xc, cg, z, skip, partials, row_tile_of_block(rg, blockIdx.x));
 }
 
 // ================================================================== record levels
