@@ -110,13 +110,15 @@ enum { UAAMG_HIERARCHY_REFERENCE = 0, UAAMG_HIERARCHY_KEEP_FLUID = 1 };
 
 /* kernel forms (uaamg_opts.forms, uaamg_stats.forms_used) */
 enum {
-    UAAMG_FORM_ROWS = 1 << 0,        /* level-0 row kernels (3D, FP32 vectors, nx <= 256) */
+    UAAMG_FORM_ROWS = 1 << 0,        /* level-0 row kernels (3D) */
     UAAMG_FORM_ROWS_COARSE = 1 << 1, /* record row kernels on levels with 64 < nx <= 128 */
     UAAMG_FORM_TAIL = 1 << 2,        /* small coarse levels in one LDS-resident workgroup */
     UAAMG_FORM_PMV = 1 << 3,         /* p update fused into the operator pass; with the fused
                                         V-cycle also r update in the level-0 down kernel and
-                                        x update on a second stream (2D: the finishes of the
-                                        dot products in the launches that use them) */
+                                        x update on a second stream (2D, and 3D with FP64
+                                        vectors: the finishes of the dot products in the
+                                        launches that use them).  Needs more memory, see
+                                        uaamg_bytes_required */
     UAAMG_FORM_XMASK = 1 << 4,       /* x update reads the mask (default: it does not need to) */
     UAAMG_FORM_NT_X = 1 << 5,        /* nontemporal loads/stores in the x update */
     UAAMG_FORM_NT_P = 1 << 6,        /* nontemporal loads of z, p_old in the operator pass */
@@ -140,8 +142,8 @@ typedef struct {
     double alg_bytes;          /* canonical algorithmic HBM bytes of this solve */
     int    kernel_set;         /* level-0 CG kernels used: 0 separate passes; 1 p update fused into the
                                   operator; 2 in addition r update in the level-0 down kernel and the
-                                  x update on a second stream, beside the coarse levels (2D: both in
-                                  one launch that also forms alpha) */
+                                  x update on a second stream, beside the coarse levels (2D, and 3D
+                                  with FP64 vectors: both in one launch that also forms alpha) */
     int    forms_used;         /* UAAMG_FORM_* bits of the kernel forms that ran */
 } uaamg_stats;
 
@@ -262,7 +264,11 @@ int uaamg_project(uaamg_ctx* ctx, double* u, double* v, double* w, double* p, do
                   int max_iter, double tol, uaamg_stats* st);
 
 /* Device memory (bytes) a context would hold for grid g under opts o; 0 when
- * uaamg_set_grid would reject the pair (invalid grid or options). */
+ * uaamg_set_grid would reject the pair (invalid grid or options).  Most of it
+ * is level-0 vectors: five of them; seven for 3D grids with FP32 vectors and
+ * six for the others under UAAMG_FORM_PMV | UAAMG_FORM_ROWS (2D: _PMV alone; GMG
+ * and AMG always six).  A grid that does not fit with the default forms may
+ * fit without UAAMG_FORM_PMV. */
 size_t uaamg_bytes_required(const uaamg_grid* g, const uaamg_opts* o);
 
 /* ---- batches: many independent solves in one set of launches ----

@@ -698,7 +698,7 @@ public:
     // nx <= 128 with 2 cells a lane, <= 256 with 4; FP64: 2 cells, nx <= 128,
     // which is the same bytes and registers per lane as FP32 with 4), wider
     // rows in windows.  Against the march kernels and flat CG passes that ran
-    // here before: 512 x 256 x 256 FP32 solve (3 windows) 57.7 -> 37.5 ms; FP64:
+    // here before: 512 x 256 x 256 FP32 solve (3 windows) 59.7 -> 37.8 ms; FP64:
     // kernels_rows64.hpp.
     static constexpr int ROWS_NW = 10, ROWS_RW = 2;
     int rows_cpl_ = 0;          // cells per lane (0: row kernels not used)
@@ -778,8 +778,11 @@ public:
         rg.nty = (ny + TY - 1) / TY;
         auto tiles = [&](int k) { return (long)rg.nty * nwx * ((nz + k - 1) / k); };
         // fewest plane steps in sequence on a CU: rounds of 256 workgroups
-        // (one per CU: ten waves of about 145 VGPRs) times the planes of a
-        // chunk, its 4 halo planes and about 2 steps' time to start
+        // (one per CU: FP32 ten waves of about 145 VGPRs, FP64 eight of 160 to
+        // 190) times the planes of a chunk, its 4 halo planes and about 2
+        // steps' time to start.  FP64, us an iteration with this choice and
+        // with the best of 4, 8, 12, 16, 24 and 32 planes: 96^3 115 / 114, 128^3
+        // 164 / 163, 160^3 255 / 264, 256 x 128 x 128 250 / 259, 256^3 832 / 832.
         int KC = 4;
         long best = 0;
         for (int k = 4; k <= 64; k += 4) {
@@ -788,8 +791,9 @@ public:
             if (tiles(k) <= (long)rg.nty * nwx) break;
         }
         // 2 planes (6 steps for 8) where the chip holds those tiles too: 64^3
-        // FP32 1.77 -> 1.64 ms per solve, 160 x 100 x 60 4.02 -> 3.59, 128 x 64
-        // x 64 FP64 2.26 -> 2.14; in two rounds slower (96^3 2.36 -> 2.79)
+        // FP32 1.77 -> 1.64 ms per solve, 160 x 100 x 60 4.02 -> 3.59; FP64 128 x
+        // 64 x 64 95 -> 91 us an iteration; in two rounds slower (96^3 FP32 2.36
+        // -> 2.79 ms)
         if (alone && KC == 4 && tiles(2) <= 256) KC = 2;
         if (kc_force > 0) KC = std::max(4, kc_force / 4 * 4);
         rg.KC = KC;
@@ -1463,8 +1467,7 @@ private:
     // 12 us of barrier packets per iteration and as many host calls, the update
     // itself 3 to 11 (FP32, per solve: 48 x 40 x 36 1.29 -> 1.13 ms, 64^3 1.63 ->
     // 1.44, 128^3 2.77 -> 2.65, 160^3 4.48 -> 4.42, but 200^3 8.13 -> 8.32 and
-    // 256^3 11.6 -> 12.0; FP64 128 x 64 x 64 2.11 -> 1.96, 256 x 128 x 128 6.03 ->
-    // 5.93).
+    // 256^3 11.6 -> 12.0).  FP64 vectors update x in k_t2_update.
     static constexpr long kInlineCells = 6L << 20;
     bool xinline() const { return N4_ <= kInlineCells; }
     void launch_x(hipStream_t s, unsigned threads, long blocks) {
