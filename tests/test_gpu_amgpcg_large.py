@@ -10,6 +10,7 @@ import pytest
 import oracle_bind as ob
 import uaamg_amd as U
 from test_gpu_amgpcg import _rhs
+from test_zz_no_alloc import _noalloc
 
 pytestmark = pytest.mark.gpu
 
@@ -24,3 +25,14 @@ def test_fixed_count(gpu, N):
         assert it == ito == 5
         bar = 1e-9 if prec == U.FP64 else 6e-8 * 4 * N * N / (2 * np.pi ** 2)
         assert np.abs(x - xo).max() <= bar * np.abs(xo).max()
+
+
+def test_folded_without_allocation(gpu):
+    """The folded sums lie in the room of the fixed array too (FP32, N = 1040)."""
+    b = _rhs(1040)
+    print("[amgpcg large] noalloc N=1040", flush=True)
+    for k in (3, 6):
+        x, it = gpu.amgpcg(1040, b, k, 1e-300, U.FP32)
+        y, iy = _noalloc(gpu, 1040, b, k, 1e-300, U.FP32, None)
+        assert it == iy == k
+        np.testing.assert_array_equal(x, y)
